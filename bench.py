@@ -100,8 +100,8 @@ def load_traffic(variant, name, grid, table="families"):
 
 
 def kernel_key(name):
-    """Kernel name without its variant tag: 'k_cols_c16<float> [GRAD]' ->
-    'k_cols_c16<float>', the key under which counter traffic is kept (all
+    """Kernel name without its variant tag: 'k_cols_reg<float> [GRAD]' ->
+    'k_cols_reg<float>', the key under which counter traffic is kept (all
     instances of a kernel template at one set of precisions)."""
     return name.split(" [")[0]
 

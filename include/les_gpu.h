@@ -116,7 +116,7 @@ int les_set_timing(int on);
  * whose profiling.txt has the five phases only): *count receives the number
  * of kernels timed since the last les_timers reset; for 0 <= i < *count,
  * name receives the kernel's name (template precisions and variant, e.g.
- * "k_cols_c16<float> [GRAD]"; memset and copy groups are named after the
+ * "k_cols_reg<float> [GRAD]"; memset and copy groups are named after the
  * runtime call), v[0] its summed ms, v[1] launches, v[2] algorithmic bytes,
  * v[3] its family.  i < 0 with name and v NULL only sets *count. */
 int les_kernel_stat(int i, int* count, char* name, int name_cap, double* v);

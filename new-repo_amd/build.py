@@ -6,6 +6,7 @@ Outputs stay in-tree so they travel with the source tree.
 """
 from __future__ import annotations
 
+import concurrent.futures
 import os
 import pathlib
 import shutil
@@ -27,7 +28,9 @@ HIP_FLAGS = [
     "-Wno-unused-value", "-Wno-unused-result",
 ]
 
-SOURCES = ["les_gpu.hip"]
+# (source, defines): the kernels with one instance per transform length are
+# compiled in parts, side by side
+SOURCES = [("les_gpu.hip", {})] + [("fft_cols.hip", {"LES_T": t, "LES_PART": p}) for t in ("double", "float") for p in range(4)]
 
 
 def _run(cmd, cwd=None):
@@ -53,16 +56,17 @@ def flang() -> str | None:
 
 
 def build_lib() -> pathlib.Path:
-    objs = []
     bdir = PKG / "_build"
     bdir.mkdir(exist_ok=True)
-    for s in SOURCES:
-        src = CSRC / s
-        if not src.exists():
-            continue
-        obj = bdir / (src.stem + ".o")
-        _run([hipcc(), *HIP_FLAGS, "-c", str(src), "-o", str(obj)])
-        objs.append(str(obj))
+
+    def compile_one(job):
+        src, defines = job
+        obj = bdir / ("_".join([pathlib.Path(src).stem, *map(str, defines.values())]) + ".o")
+        _run([hipcc(), *HIP_FLAGS, *[f"-D{k}={v}" for k, v in defines.items()], "-c", str(CSRC / src), "-o", str(obj)])
+        return str(obj)
+
+    with concurrent.futures.ThreadPoolExecutor(min(8, os.cpu_count() or 1)) as pool:
+        objs = list(pool.map(compile_one, SOURCES))
     tmp = LIB.with_suffix(".so.tmp")
     _run([hipcc(), "--offload-arch=gfx950", "-shared", "-fPIC", "-o", str(tmp), *objs])
     tmp.replace(LIB)

@@ -251,8 +251,8 @@ k_rows_c2r(RowC2RArgs<T, TO> a, FftPlan pl, const Cplx<T>* __restrict__ tw) {
 enum { COP_GRAD = 0, COP_DIV = 1, COP_FILT2 = 2, COP_FILT1 = 3, COP_COPY = 4, COP_PGRAD = 5 };
 
 template <typename T>
-struct ColArgs {
-  // per job (blockIdx.y of the register-resident kernel; job 0 elsewhere):
+struct ColArgs {  // k_cols_reg, cols_reg.h
+  // per job (blockIdx.y):
   // the same op on up to LES_COL_JOBS independent input/output sets
   const Cplx<T>* in[LES_COL_JOBS][2];
   Cplx<T>* out[LES_COL_JOBS][3];
@@ -260,199 +260,9 @@ struct ColArgs {
   const T* kky;
   const T* g0;
   const T* g1;
-  int lhx, ny;
+  int lhx;
   int k0, nplanes;
-  int ls;        // LDS line stride (at least ny, chosen so the tile transposes hit distinct banks)
-  int ncb;       // column blocks per plane
-  int nin, nout;
-  int op;
-  int fwd, inv;  // apply forward y transform to inputs / inverse to outputs
-  int ntiles;    // ncb * nplanes
 };
-
-template <typename T>
-__device__ __forceinline__ Cplx<T> col_op(const ColArgs<T>& a, int o, int kx, int j, Cplx<T> x0, Cplx<T> x1) {
-  const long q = (long)j * a.lhx + kx;
-  const bool nyq = (kx == a.lhx - 1) || (j == a.ny / 2);
-  switch (a.op) {
-    case COP_GRAD: {
-      Cplx<T> v = nyq ? Cplx<T>{(T)0, (T)0} : x0;
-      if (o == 0) return c_ik(a.kkx[q], v);
-      if (o == 1) return c_ik(a.kky[q], v);
-      return v;
-    }
-    case COP_DIV: {
-      Cplx<T> v0 = nyq ? Cplx<T>{(T)0, (T)0} : x0;
-      Cplx<T> v1 = nyq ? Cplx<T>{(T)0, (T)0} : x1;
-      return c_add(c_ik(a.kkx[q], v0), c_ik(a.kky[q], v1));
-    }
-    case COP_FILT2:
-      return c_scale(x0, o == 0 ? a.g0[q] : a.g1[q]);
-    case COP_FILT1:
-      return c_scale(x0, a.g0[q]);
-    case COP_PGRAD:
-      if (o == 0) return c_ik(a.kkx[q], x0);
-      if (o == 1) return c_ik(a.kky[q], x0);
-      return x0;
-    default:
-      return x0;
-  }
-}
-
-template <typename T, int CB, typename FFT>
-__device__ __forceinline__ void cols_body(const ColArgs<T>& a, unsigned char* smem, FFT&& fft) {
-  const int ny = a.ny, LS = a.ls;
-  Cplx<T>* X0 = reinterpret_cast<Cplx<T>*>(smem);
-  Cplx<T>* X1 = X0 + CB * LS;
-  Cplx<T>* Y = X0 + (a.nin > 1 ? 2 : 1) * CB * LS;
-  const int tile = xcd_tile(blockIdx.x, gridDim.x);
-  const int k = a.k0 + tile / a.ncb;
-  const int c0 = (tile % a.ncb) * CB;
-  int nc = a.lhx - c0;
-  if (nc > CB) nc = CB;
-  const long pbase = (long)k * ny * a.lhx + c0;
-  for (int t = 0; t < a.nin; ++t) {
-    const Cplx<T>* __restrict__ src = a.in[0][t] + pbase;
-    Cplx<T>* X = t == 0 ? X0 : X1;
-    for (int idx = threadIdx.x; idx < CB * ny; idx += blockDim.x) {
-      const int j = idx / CB, c = idx % CB;
-      if (c < nc) X[c * LS + j] = src[(long)j * a.lhx + c];
-    }
-  }
-  __syncthreads();
-  const int lane = threadIdx.x & (LES_WAVE - 1), wave = threadIdx.x / LES_WAVE, nw = blockDim.x / LES_WAVE;
-  if (a.fwd) {
-    for (int c = wave; c < nc; c += nw) {
-      fft(X0 + c * LS, false);
-      if (a.nin > 1) fft(X1 + c * LS, false);
-    }
-  }
-  for (int o = 0; o < a.nout; ++o) {
-    for (int c = wave; c < nc; c += nw) {
-      const Cplx<T>* x0 = X0 + c * LS;
-      const Cplx<T>* x1 = (a.nin > 1 ? X1 : X0) + c * LS;
-      Cplx<T>* y = Y + c * LS;
-      for (int j = lane; j < ny; j += LES_WAVE) y[j] = col_op(a, o, c0 + c, j, x0[j], x1[j]);
-      wave_sync();
-      if (a.inv) fft(y, true);
-    }
-    __syncthreads();
-    Cplx<T>* __restrict__ dst = a.out[0][o] + pbase;
-    for (int idx = threadIdx.x; idx < CB * ny; idx += blockDim.x) {
-      const int j = idx / CB, c = idx % CB;
-      if (c < nc) dst[(long)j * a.lhx + c] = Y[c * LS + j];
-    }
-    __syncthreads();
-  }
-}
-
-// Persistent, software-pipelined version for ny = 256 (tiles of CB columns,
-// E = CB * 256 / LES_BLOCK elements per thread and input): the block walks a
-// contiguous run of tiles of its XCD (stride = blocks of that XCD, so the
-// concurrently running blocks of one XCD take adjacent tiles) and loads the
-// next tile into registers while it transforms the current one.
-template <typename T, int CB, typename FFT>
-__device__ __forceinline__ void cols_body_pipe(const ColArgs<T>& a, unsigned char* smem, FFT&& fft) {
-  constexpr int NY = 256, E = CB * NY / LES_BLOCK;
-  static_assert(E * LES_BLOCK == CB * NY, "tile must split evenly over the block");
-  const int LS = a.ls;
-  Cplx<T>* X0 = reinterpret_cast<Cplx<T>*>(smem);
-  Cplx<T>* X1 = X0 + CB * LS;
-  Cplx<T>* Y = X0 + (a.nin > 1 ? 2 : 1) * CB * LS;
-  const int x = blockIdx.x % LES_NXCD, m = blockIdx.x / LES_NXCD, nb = gridDim.x / LES_NXCD;
-  const int q = a.ntiles / LES_NXCD, r = a.ntiles % LES_NXCD;
-  const int tbeg = x * q + (x < r ? x : r), tend = tbeg + q + (x < r ? 1 : 0);
-  int t = tbeg + m;
-  if (t >= tend) return;
-  const int lane = threadIdx.x & (LES_WAVE - 1), wave = threadIdx.x / LES_WAVE, nw = blockDim.x / LES_WAVE;
-  Cplx<T> pre[2][E];
-  auto fetch = [&](int tt) {
-    const int k = a.k0 + tt / a.ncb, c0 = (tt % a.ncb) * CB;
-    int nc = a.lhx - c0;
-    if (nc > CB) nc = CB;
-    const long pb = (long)k * NY * a.lhx + c0;
-#pragma unroll
-    for (int in = 0; in < 2; ++in) {
-      if (in < a.nin) {
-#pragma unroll
-        for (int e = 0; e < E; ++e) {
-          const int idx = threadIdx.x + e * LES_BLOCK, j = idx / CB, c = idx % CB;
-          pre[in][e] = c < nc ? a.in[0][in][pb + (long)j * a.lhx + c] : Cplx<T>{(T)0, (T)0};
-        }
-      }
-    }
-  };
-  fetch(t);
-  while (true) {
-    const int k = a.k0 + t / a.ncb, c0 = (t % a.ncb) * CB;
-    int nc = a.lhx - c0;
-    if (nc > CB) nc = CB;
-    const long pbase = (long)k * NY * a.lhx + c0;
-#pragma unroll
-    for (int in = 0; in < 2; ++in) {
-      if (in < a.nin) {
-        Cplx<T>* X = in == 0 ? X0 : X1;
-#pragma unroll
-        for (int e = 0; e < E; ++e) {
-          const int idx = threadIdx.x + e * LES_BLOCK, j = idx / CB, c = idx % CB;
-          X[c * LS + j] = pre[in][e];
-        }
-      }
-    }
-    block_sync_lds();
-    const int tn = t + nb;
-    if (tn < tend) fetch(tn);  // in flight during this tile's transforms
-    if (a.fwd) {
-      for (int c = wave; c < nc; c += nw) {
-        fft(X0 + c * LS, false);
-        if (a.nin > 1) fft(X1 + c * LS, false);
-      }
-    }
-    for (int o = 0; o < a.nout; ++o) {
-      for (int c = wave; c < nc; c += nw) {
-        const Cplx<T>* x0 = X0 + c * LS;
-        const Cplx<T>* x1 = (a.nin > 1 ? X1 : X0) + c * LS;
-        Cplx<T>* y = Y + c * LS;
-        for (int j = lane; j < NY; j += LES_WAVE) y[j] = col_op(a, o, c0 + c, j, x0[j], x1[j]);
-        wave_sync();
-        if (a.inv) fft(y, true);
-      }
-      block_sync_lds();
-      Cplx<T>* __restrict__ dst = a.out[0][o] + pbase;
-#pragma unroll
-      for (int e = 0; e < E; ++e) {
-        const int idx = threadIdx.x + e * LES_BLOCK, j = idx / CB, c = idx % CB;
-        if (c < nc) dst[(long)j * a.lhx + c] = Y[c * LS + j];
-      }
-      block_sync_lds();
-    }
-    if (tn >= tend) break;
-    t = tn;
-  }
-}
-
-// A tile of CB adjacent kx columns of one plane: loaded row by row (CB
-// contiguous complex values per row), transposed into LDS so every column is
-// a contiguous line, transformed along y by one wavefront per column,
-// combined by the spectral op and transformed back, then stored row by row.
-// Length 256 runs on register twiddles and the pipelined persistent body.
-template <typename T, int CB>
-__global__ void __launch_bounds__(LES_BLOCK) k_cols(ColArgs<T> a, FftPlan pl, const Cplx<T>* __restrict__ tw) {
-  extern __shared__ __align__(16) unsigned char smem_raw[];
-  const int lane = threadIdx.x & (LES_WAVE - 1);
-  cols_body<T, CB>(a, smem_raw, [&](Cplx<T>* p, bool inv) { wave_fft(p, pl, tw, inv, lane); });
-}
-
-// ny = 256: a kernel of its own, so its register budget is not set by the
-// runtime-plan path (whose radix-2 stages need twice the butterflies).
-template <typename T, int CB>
-__global__ void __launch_bounds__(LES_BLOCK) k_cols_256(ColArgs<T> a, FftPlan pl, const Cplx<T>* __restrict__ tw) {
-  extern __shared__ __align__(16) unsigned char smem_raw[];
-  const int lane = threadIdx.x & (LES_WAVE - 1);
-  TwReg<T, 256> tr;
-  tw_load(tr, tw + pl.twf, lane);
-  cols_body_pipe<T, CB>(a, smem_raw, [&](Cplx<T>* p, bool inv) { wave_fft_t(p, tr, inv, lane); });
-}
 
 // ------------------------------------------------------------------ columns, ny = 256, in registers
 // The 256-point column transform as two register-resident halves.  The four
@@ -528,117 +338,6 @@ __device__ __forceinline__ void c16_pair_b(Cplx<T>* X, const Cplx<T>* __restrict
     bfly(x, 4, sgn);
 #pragma unroll
     for (int r2 = 0; r2 < 4; ++r2) X[r + 4 * r2] = x[r2];
-  }
-}
-
-// Whole transform of thread (c, a)'s 16 values through the exchange buffer
-// (ex: this block's buffer; the caller's barrier protects earlier readers).
-template <typename T>
-__device__ __forceinline__ void c16_fft(Cplx<T>* X, const Cplx<T>* __restrict__ twf, bool inverse, Cplx<T>* ex, int c,
-                                        int a) {
-  c16_pair_a(X, twf, inverse);
-  Cplx<T>* col = ex + c * LES_C16_LS;
-#pragma unroll
-  for (int cc = 0; cc < 16; ++cc) lds_st(col + 17 * a + cc, X[cc]);
-  __syncthreads();
-#pragma unroll
-  for (int t = 0; t < 16; ++t) X[t] = lds_ld(col + a + 17 * t);
-  __syncthreads();
-  c16_pair_b(X, twf, a, inverse);
-}
-
-// col_op with the operation fixed at compile time (same arithmetic).
-template <typename T, int OP>
-__device__ __forceinline__ Cplx<T> c16_op(const ColArgs<T>& a, int o, int kx, int j, Cplx<T> x0, Cplx<T> x1) {
-  const long q = (long)j * a.lhx + kx;
-  const bool nyq = (kx == a.lhx - 1) || (j == a.ny / 2);
-  const Cplx<T> zero = {(T)0, (T)0};
-  if constexpr (OP == COP_GRAD) {
-    const Cplx<T> v = nyq ? zero : x0;
-    if (o == 0) return c_ik(a.kkx[q], v);
-    if (o == 1) return c_ik(a.kky[q], v);
-    return v;
-  } else if constexpr (OP == COP_DIV) {
-    const Cplx<T> v0 = nyq ? zero : x0;
-    const Cplx<T> v1 = nyq ? zero : x1;
-    return c_add(c_ik(a.kkx[q], v0), c_ik(a.kky[q], v1));
-  } else if constexpr (OP == COP_FILT2) {
-    return c_scale(x0, o == 0 ? a.g0[q] : a.g1[q]);
-  } else if constexpr (OP == COP_FILT1) {
-    return c_scale(x0, a.g0[q]);
-  } else if constexpr (OP == COP_PGRAD) {
-    if (o == 0) return c_ik(a.kkx[q], x0);
-    if (o == 1) return c_ik(a.kky[q], x0);
-    return x0;
-  } else {
-    return x0;
-  }
-}
-
-template <typename T, int NIN, int OP, int NOUT>
-__global__ void __launch_bounds__(LES_BLOCK) k_cols_c16(ColArgs<T> a, const Cplx<T>* __restrict__ twf) {
-  extern __shared__ __align__(16) unsigned char smem_raw[];
-  Cplx<T>* ex = reinterpret_cast<Cplx<T>*>(smem_raw);
-  const int c = threadIdx.x & 15, ar = threadIdx.x >> 4;  // column in the tile, row class
-  const int job = blockIdx.y;
-  const int tile = xcd_tile(blockIdx.x, gridDim.x);
-  const int k = a.k0 + tile / a.ncb;
-  const int c0 = (tile % a.ncb) * 16;
-  const bool valid = c0 + c < a.lhx;
-  const int kx = valid ? c0 + c : a.lhx - 1;
-  const long base = (long)k * 256 * a.lhx + kx;
-  Cplx<T> X0[16], X1[16];
-#pragma unroll
-  for (int t = 0; t < 16; ++t) X0[t] = valid ? a.in[job][0][base + (long)(ar + 16 * t) * a.lhx] : Cplx<T>{(T)0, (T)0};
-  if constexpr (NIN == 2 && OP == COP_DIV && NOUT == 1) {
-    // divergence: i kx X0 is formed before the second input is loaded (the
-    // transforms' barriers keep its loads after), so only one input line
-    // and the partial sum are live at a time; the same operations in the
-    // same order as c16_op's COP_DIV
-    if (a.fwd) c16_fft(X0, twf, false, ex, c, ar);
-    const Cplx<T> zero = {(T)0, (T)0};
-#pragma unroll
-    for (int t = 0; t < 16; ++t) {
-      const int j = ar + 16 * t;
-      const bool nyq = (kx == a.lhx - 1) || (j == a.ny / 2);
-      X0[t] = c_ik(a.kkx[(long)j * a.lhx + kx], nyq ? zero : X0[t]);
-    }
-#pragma unroll
-    for (int t = 0; t < 16; ++t) X1[t] = valid ? a.in[job][1][base + (long)(ar + 16 * t) * a.lhx] : zero;
-    if (a.fwd) c16_fft(X1, twf, false, ex, c, ar);
-#pragma unroll
-    for (int t = 0; t < 16; ++t) {
-      const int j = ar + 16 * t;
-      const bool nyq = (kx == a.lhx - 1) || (j == a.ny / 2);
-      X0[t] = c_add(X0[t], c_ik(a.kky[(long)j * a.lhx + kx], nyq ? zero : X1[t]));
-    }
-    if (a.inv) c16_fft(X0, twf, true, ex, c, ar);
-    if (valid) {
-      Cplx<T>* __restrict__ dst = a.out[job][0] + base;
-#pragma unroll
-      for (int t = 0; t < 16; ++t) dst[(long)(ar + 16 * t) * a.lhx] = X0[t];
-    }
-    return;
-  }
-  if constexpr (NIN > 1) {
-#pragma unroll
-    for (int t = 0; t < 16; ++t) X1[t] = valid ? a.in[job][1][base + (long)(ar + 16 * t) * a.lhx] : Cplx<T>{(T)0, (T)0};
-  }
-  if (a.fwd) {
-    c16_fft(X0, twf, false, ex, c, ar);
-    if constexpr (NIN > 1) c16_fft(X1, twf, false, ex, c, ar);
-  }
-#pragma unroll
-  for (int o = 0; o < NOUT; ++o) {
-    Cplx<T> Y[16];
-#pragma unroll
-    for (int t = 0; t < 16; ++t) Y[t] = c16_op<T, OP>(a, o, kx, ar + 16 * t, X0[t], NIN > 1 ? X1[t] : X0[t]);
-    if (a.inv) c16_fft(Y, twf, true, ex, c, ar);
-    if (valid) {
-      Cplx<T>* __restrict__ dst = a.out[job][o] + base;
-#pragma unroll
-      for (int t = 0; t < 16; ++t) dst[(long)(ar + 16 * t) * a.lhx] = Y[t];
-    }
   }
 }
 

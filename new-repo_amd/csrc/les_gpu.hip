@@ -20,6 +20,7 @@
 
 #include "les_state.h"
 #include "les_ops.h"
+#include "fft_launch.h"
 
 Les* g_les = nullptr;
 static char g_err[512] = "";
@@ -214,16 +215,6 @@ static void rows_c2r(Les& L, const Cplx<T>* const* src, TO* const* dst, int nf, 
          "k_rows_c2r", sizeof(T), sizeof(TO));
 }
 
-// Column tiles: LES_COL_TILE_BYTES contiguous bytes per row for
-// single-input ops, half that for two-input ops (three LDS tiles instead of
-// two), at least 4 columns.  With the XCD-aware tile order (xcd_tile) the
-// narrow rows are not over-fetched; 32-byte rows (4 FP32 / 4 FP64 columns)
-// measured fastest at 256^2 because the small tiles leave room for more
-// blocks per CU.
-#ifndef LES_COL_TILE_BYTES
-#define LES_COL_TILE_BYTES 32
-#endif
-
 // LDS line stride (in line elements of eb bytes, at least n) for a tile of
 // `lines` lines filled and drained row by row (consecutive lanes take
 // consecutive lines, then the next row).  One LDS cycle serves 128 bytes:
@@ -236,70 +227,9 @@ static int lds_stride(int n, int lines, int eb) {
   while (st % g != r % g) ++st;
   return st;
 }
-template <typename T>
-static int col_tile(int nin) {
-  int cb = (nin > 1 ? LES_COL_TILE_BYTES / 2 : LES_COL_TILE_BYTES) / (int)sizeof(Cplx<T>);
-  return cb < 4 ? 4 : cb;
-}
-
-// ny = 256 runs the persistent pipelined kernel body: a grid of (resident
-// blocks per CU) x (CUs), a multiple of the 8 XCDs; other lengths one block
-// per tile.
-// ny = 256: register-resident transform (k_cols_c16); LES_COL16=0 selects
-// the LDS-engine kernel (k_cols_256) instead.
-#ifndef LES_COL16
-#define LES_COL16 1
-#endif
-template <typename T, int CB>
-static void launch_cols(Les& L, const ColArgs<T>& a, int npl, int njobs) {
-  const size_t sh = (size_t)(a.nin + 1) * CB * a.ls * sizeof(Cplx<T>);
-  if (!(L.ny == 256 && LES_COL16) && njobs > 1) {
-    // the LDS-engine kernels take one job per launch
-    for (int j = 0; j < njobs; ++j) {
-      ColArgs<T> b = a;
-      for (int t = 0; t < 2; ++t) b.in[0][t] = a.in[j][t];
-      for (int o = 0; o < 3; ++o) b.out[0][o] = a.out[j][o];
-      launch_cols<T, CB>(L, b, npl, 1);
-    }
-    return;
-  }
-  if (L.ny == 256 && LES_COL16) {
-    ColArgs<T> b = a;
-    b.ncb = (L.lhx + 15) / 16;
-    b.ntiles = b.ncb * npl;
-    const size_t sh16 = (size_t)16 * LES_C16_LS * sizeof(Cplx<T>);
-    const dim3 g((unsigned)b.ntiles, (unsigned)njobs);
-    const Cplx<T>* tw = twpool<T>(L) + L.py.twf;
-#define LES_C16(NIN, OP, NOUT) \
-  hipLaunchKernelGGL((k_cols_c16<T, NIN, OP, NOUT>), g, dim3(LES_BLOCK), sh16, L.stream, b, tw)
-    if (a.op == COP_GRAD && a.nout == 3) LES_C16(1, COP_GRAD, 3);
-    else if (a.op == COP_GRAD) LES_C16(1, COP_GRAD, 2);
-    else if (a.op == COP_DIV) LES_C16(2, COP_DIV, 1);
-    else if (a.op == COP_FILT2) LES_C16(1, COP_FILT2, 2);
-    else if (a.op == COP_FILT1) LES_C16(1, COP_FILT1, 1);
-    else if (a.op == COP_PGRAD) LES_C16(1, COP_PGRAD, 3);
-    else LES_C16(1, COP_COPY, 1);
-#undef LES_C16
-  } else if (L.ny == 256) {
-    static int occ[2] = {0, 0};  // per input count
-    int& o = occ[a.nin > 1];
-    if (o == 0) {
-      if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&o, k_cols_256<T, CB>, LES_BLOCK, sh) != hipSuccess || o < 1) o = 1;
-    }
-    long g = (long)o * L.ncu;
-    long need = ((long)a.ntiles + LES_NXCD - 1) / LES_NXCD * LES_NXCD;
-    if (g > need) g = need;
-    const unsigned grid = (unsigned)((g + LES_NXCD - 1) / LES_NXCD * LES_NXCD);
-    hipLaunchKernelGGL((k_cols_256<T, CB>), dim3(grid), dim3(LES_BLOCK), sh, L.stream, a, L.py, twpool<T>(L));
-  } else {
-    hipLaunchKernelGGL((k_cols<T, CB>), dim3((unsigned)a.ntiles), dim3(LES_BLOCK), sh, L.stream, a, L.py, twpool<T>(L));
-  }
-}
-
 // The same column op on njobs (at most LES_COL_JOBS) independent sets of
-// inputs and outputs, one launch on the register-resident path: the sets'
-// tiles share the grid, so the partly filled last round of blocks is paid
-// once instead of once per set.
+// inputs and outputs in one launch: the sets' tiles share the grid, so the
+// partly filled last round of blocks is paid once instead of once per set.
 template <typename T>
 static void cols_jobs(Les& L, int op, int njobs, const Cplx<T>* const* in0, const Cplx<T>* const* in1,
                       Cplx<T>* const* o0, Cplx<T>* const* o1, Cplx<T>* const* o2, int nout, int fwd, int inv, int k0,
@@ -314,20 +244,11 @@ static void cols_jobs(Les& L, int op, int njobs, const Cplx<T>* const* in0, cons
   a.kkx = sizeof(T) == 8 ? (const T*)L.kkx64 : (const T*)L.kkx32;
   a.kky = sizeof(T) == 8 ? (const T*)L.kky64 : (const T*)L.kky32;
   a.g0 = g0; a.g1 = g1;
-  a.lhx = L.lhx; a.ny = L.ny; a.k0 = k0; a.nplanes = npl;
-  a.nin = in1 ? 2 : 1;
-  a.nout = nout; a.op = op; a.fwd = fwd; a.inv = inv;
-  const int cb = col_tile<T>(a.nin);
-  a.ls = lds_stride(L.ny, cb, (int)sizeof(Cplx<T>));
-  a.ncb = (L.lhx + cb - 1) / cb;
-  a.ntiles = a.ncb * npl;
+  a.lhx = L.lhx; a.k0 = k0; a.nplanes = npl;
   kt_begin(L, KT_COLS);
-  if (cb == 4) launch_cols<T, 4>(L, a, npl, njobs);
-  else if (cb == 8) launch_cols<T, 8>(L, a, npl, njobs);
-  else launch_cols<T, 16>(L, a, npl, njobs);
+  cols_reg<T>(false, L.ny, op, nout, fwd, inv, a, njobs, twpool<T>(L) + L.py.twf, L.stream);
   static const char* const opn[] = {"GRAD", "DIV", "FILT2", "FILT1", "COPY", "PGRAD"};
-  kt_end(L, KT_COLS, (double)njobs * npl * L.ns * sizeof(Cplx<T>) * (a.nin + nout),
-         (L.ny == 256 && LES_COL16) ? "k_cols_c16" : L.ny == 256 ? "k_cols_256" : "k_cols", sizeof(T), 0, opn[op]);
+  kt_end(L, KT_COLS, (double)njobs * npl * L.ns * sizeof(Cplx<T>) * ((in1 ? 2 : 1) + nout), "k_cols_reg", sizeof(T), 0, opn[op]);
 }
 
 template <typename T>
@@ -391,7 +312,7 @@ static void grad_filt(Les& L, int fid, int dx_id, int dy_id) {
 // or one per field where the mixed mode forms the Nyquist sums), one column
 // launch of three jobs, one inverse launch of the six derivatives and, in
 // FP64, one of the three filtered fields.  The FP64 filtered spectra
-// overwrite the inputs: k_cols_c16 reads its whole tile before its first
+// overwrite the inputs: k_cols_reg reads its whole tile before its first
 // store and every block owns its tile.
 // Measured at 256^3 (MI355X): FP64 0.055 ms per step faster than three
 // grad_filt chains; in FP32 0.025 ms slower, its six-field inverse launch
@@ -1016,16 +937,7 @@ static int les_step_t(Les& L) {
 }
 
 // ------------------------------------------------------------------ set-up
-template <typename T>
-static void c16_attrs(int big) {
-  const void* k[] = {(const void*)k_cols_c16<T, 1, COP_GRAD, 3>, (const void*)k_cols_c16<T, 1, COP_GRAD, 2>,
-                     (const void*)k_cols_c16<T, 2, COP_DIV, 1>,  (const void*)k_cols_c16<T, 1, COP_FILT2, 2>,
-                     (const void*)k_cols_c16<T, 1, COP_FILT1, 1>, (const void*)k_cols_c16<T, 1, COP_PGRAD, 3>,
-                     (const void*)k_cols_c16<T, 1, COP_COPY, 1>};
-  for (const void* f : k) hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, big);
-}
-
-static int setup_kernel_attrs() {
+static int setup_kernel_attrs(const Les& L) {
   const int big = 160 * 1024;
   hipFuncSetAttribute((const void*)k_rows_r2c<double, double>, hipFuncAttributeMaxDynamicSharedMemorySize, big);
   hipFuncSetAttribute((const void*)k_rows_r2c<double, float>, hipFuncAttributeMaxDynamicSharedMemorySize, big);
@@ -1033,18 +945,13 @@ static int setup_kernel_attrs() {
   hipFuncSetAttribute((const void*)k_rows_c2r<double, double>, hipFuncAttributeMaxDynamicSharedMemorySize, big);
   hipFuncSetAttribute((const void*)k_rows_c2r<float, float>, hipFuncAttributeMaxDynamicSharedMemorySize, big);
   hipFuncSetAttribute((const void*)k_rows_c2r<float, double>, hipFuncAttributeMaxDynamicSharedMemorySize, big);
-  hipFuncSetAttribute((const void*)k_cols_256<double, 4>, hipFuncAttributeMaxDynamicSharedMemorySize, big);
-  c16_attrs<double>(big);
-  c16_attrs<float>(big);
+  if (!cols_reg<double>(true, L.ny, 0, 0, 0, 0, ColArgs<double>(), 0, nullptr, 0) ||
+      !cols_reg<float>(true, L.ny, 0, 0, 0, 0, ColArgs<float>(), 0, nullptr, 0))
+    return 10;
   hipFuncSetAttribute((const void*)k_colres_c16<float, true>, hipFuncAttributeMaxDynamicSharedMemorySize, big);
   hipFuncSetAttribute((const void*)k_colres_c16<float, false>, hipFuncAttributeMaxDynamicSharedMemorySize, big);
   hipFuncSetAttribute((const void*)k_colres_c16<double, true>, hipFuncAttributeMaxDynamicSharedMemorySize, big);
   hipFuncSetAttribute((const void*)k_colres_c16<double, false>, hipFuncAttributeMaxDynamicSharedMemorySize, big);
-  hipFuncSetAttribute((const void*)k_cols_256<float, 4>, hipFuncAttributeMaxDynamicSharedMemorySize, big);
-  hipFuncSetAttribute((const void*)k_cols<double, 4>, hipFuncAttributeMaxDynamicSharedMemorySize, big);
-  hipFuncSetAttribute((const void*)k_cols<double, 8>, hipFuncAttributeMaxDynamicSharedMemorySize, big);
-  hipFuncSetAttribute((const void*)k_cols<float, 8>, hipFuncAttributeMaxDynamicSharedMemorySize, big);
-  hipFuncSetAttribute((const void*)k_cols<float, 16>, hipFuncAttributeMaxDynamicSharedMemorySize, big);
   hipFuncSetAttribute((const void*)k_rows_resample<double, double, double>, hipFuncAttributeMaxDynamicSharedMemorySize, big);
   hipFuncSetAttribute((const void*)k_rows_resample<float, double, float>, hipFuncAttributeMaxDynamicSharedMemorySize, big);
   hipFuncSetAttribute((const void*)k_rows_resample<float, float, float>, hipFuncAttributeMaxDynamicSharedMemorySize, big);
@@ -1301,7 +1208,7 @@ int les_init(const les_params* p) {
   L->dg_out = (double*)dalloc(*L, sizeof(double) * 4);
   if (L->alloc_failed) { les_finalize(); les_set_error("out of memory (workspaces)"); return 3; }
   for (int i = 0; i < 64; ++i) if (!L->wk_real[i]) { les_finalize(); les_set_error("out of memory"); return 3; }
-  setup_kernel_attrs();
+  if (setup_kernel_attrs(*L)) { les_set_error("no column kernels for ny = %d", ny); les_finalize(); return 10; }
   if (hipDeviceSynchronize() != hipSuccess) { les_set_error("init sync failed"); les_finalize(); return 5; }
   return 0;
 }

@@ -82,8 +82,8 @@ def rocprof_key(name: str) -> str:
     """rocprofv3's kernel name -> the key of the library's per-kernel
     statistics: the kernel name with its floating-point template arguments
     (at most two), without other template arguments or the parameter list:
-    'void k_cols_c16<float, 1, 2, 2>(ColArgs<float>, ...)' ->
-    'k_cols_c16<float>', 'k_proj(ProjArgs)' -> 'k_proj'."""
+    'void k_cols_reg<float, 256, 2, 2, true, true>(ColArgs<float>, ...)' ->
+    'k_cols_reg<float>', 'k_proj(ProjArgs)' -> 'k_proj'."""
     n = name.strip()
     if n.startswith("void "):
         n = n[5:]
@@ -116,7 +116,7 @@ def rocprof_key(name: str) -> str:
 
 # kernel-name patterns of the benchmark's kernel families
 FAMILY_KERNELS = {"rows_r2c": r"\bk_rows_r2c<", "rows_c2r": r"\bk_rows_c2r(_div<|_proj\(|<)",
-                  "cols": r"\bk_cols(_256|_c16)?<", "rows_resample": r"\bk_rows_resample<",
+                  "cols": r"\bk_cols_reg<", "rows_resample": r"\bk_rows_resample<",
                   "cols_resample": r"\bk_(cols_resample|colres_c16)<", "tridiag": r"\bk_tridiag",
                   "lagrangian": r"\bk_lagr<"}
 
