@@ -264,83 +264,6 @@ struct ColArgs {  // k_cols_reg, cols_reg.h
   int k0, nplanes;
 };
 
-// ------------------------------------------------------------------ columns, ny = 256, in registers
-// The 256-point column transform as two register-resident halves.  The four
-// radix-4 Stockham stages (engine above) fall into 16 closed groups twice:
-// stages 0-1 map inputs a + 16 t (t < 16) of thread a to its outputs 16 a + c
-// (c < 16), and stages 2-3 map inputs k + 16 t of thread k to outputs
-// k + 16 t.  So a thread loads its column's rows a + 16 t straight from
-// global memory, runs stages 0-1 in registers, trades through LDS (16 x 16
-// transpose per column, row e at 17 (e >> 4) + (e & 15): conflict-free), runs
-// stages 2-3 in registers and holds spectral rows a + 16 t, which is again
-// the input layout of stages 0-1, so the spectral op and the inverse
-// transform continue in registers and the result is stored from them.  The
-// butterflies, twiddles and their order are those of the Stockham stages.
-// Block: 16 columns (128-byte row segments) x 16 row classes; one LDS
-// exchange per transform instead of one per stage plus two tile transposes.
-#define LES_C16_LS 273  // column stride in the exchange buffer (= 1 mod 16)
-static_assert(cp_OFF(256, 1) == 3 && cp_OFF(256, 2) == 15 && cp_OFF(256, 3) == 63, "256-point twiddle layout");
-
-// Twiddles are read from the plan's table (4 KB at most, cache-resident)
-// where they are used: stages 0-1 read the same entries in every thread,
-// stages 2-3 the thread's own.
-template <typename T>
-__device__ __forceinline__ Cplx<T> tw16(const Cplx<T>* __restrict__ twf, int idx, bool inverse) {
-  Cplx<T> w = twf[idx];
-  if (inverse) w.y = -w.y;
-  return w;
-}
-
-// stages 0-1: X[t] = z[a + 16 t] -> X[c] = z'[16 a + c]
-template <typename T>
-__device__ __forceinline__ void c16_pair_a(Cplx<T>* X, const Cplx<T>* __restrict__ twf, bool inverse) {
-  const int sgn = inverse ? 1 : -1;
-  Cplx<T> Y[4][4];
-#pragma unroll
-  for (int m = 0; m < 4; ++m) {
-    Cplx<T> x[4] = {X[m], X[m + 4], X[m + 8], X[m + 12]};
-#pragma unroll
-    for (int r = 1; r < 4; ++r) x[r] = c_mul(x[r], tw16(twf, r - 1, inverse));
-    bfly(x, 4, sgn);
-#pragma unroll
-    for (int r = 0; r < 4; ++r) Y[m][r] = x[r];
-  }
-#pragma unroll
-  for (int b = 0; b < 4; ++b) {
-    Cplx<T> x[4] = {Y[0][b], Y[1][b], Y[2][b], Y[3][b]};
-#pragma unroll
-    for (int r = 1; r < 4; ++r) x[r] = c_mul(x[r], tw16(twf, 3 + (r - 1) * 4 + b, inverse));
-    bfly(x, 4, sgn);
-#pragma unroll
-    for (int r = 0; r < 4; ++r) X[b + 4 * r] = x[r];
-  }
-}
-
-// stages 2-3: X[t] = z'[k + 16 t] -> X[t] = Z[k + 16 t]
-template <typename T>
-__device__ __forceinline__ void c16_pair_b(Cplx<T>* X, const Cplx<T>* __restrict__ twf, int k, bool inverse) {
-  const int sgn = inverse ? 1 : -1;
-  Cplx<T> V[4][4];
-#pragma unroll
-  for (int q = 0; q < 4; ++q) {
-    Cplx<T> x[4] = {X[q], X[q + 4], X[q + 8], X[q + 12]};
-#pragma unroll
-    for (int r = 1; r < 4; ++r) x[r] = c_mul(x[r], tw16(twf, 15 + (r - 1) * 16 + k, inverse));
-    bfly(x, 4, sgn);
-#pragma unroll
-    for (int r = 0; r < 4; ++r) V[q][r] = x[r];
-  }
-#pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    Cplx<T> x[4] = {V[0][r], V[1][r], V[2][r], V[3][r]};
-#pragma unroll
-    for (int rp = 1; rp < 4; ++rp) x[rp] = c_mul(x[rp], tw16(twf, 63 + (rp - 1) * 64 + k + 16 * r, inverse));
-    bfly(x, 4, sgn);
-#pragma unroll
-    for (int r2 = 0; r2 < 4; ++r2) X[r + 4 * r2] = x[r2];
-  }
-}
-
 // ------------------------------------------------------------------ 3/2 resampling
 // Padding keeps modes |k| < n/2 (Nyquist dropped) of a length-n1 line in a
 // length-n2 spectrum; truncation is the mirror image
@@ -509,261 +432,13 @@ k_rows_resample(RowResArgs<T, TI, TO> a, FftPlan p1, FftPlan p2, const Cplx<T>* 
   });
 }
 
-// Column resampling: column pairs (i, i+1) of a real (W, h1) plane -> (W, h2).
-// A tile of CP pairs is loaded row by row (2 CP contiguous reals), held as
-// CP complex lines in LDS, resampled by one wavefront per line, stored row by
-// row.
+// Column resampling: column pairs (i, i+1) of a real (W, h1) plane -> (W, h2)
+// as complex lines (k_colres_reg, colres_reg.h).
 template <typename T>
 struct ColResArgs {
   const T* src[LES_MAX_FIELDS];
   T* dst[LES_MAX_FIELDS];
-  int W, h1, h2;
+  int W;  // real columns
   int k0, nplanes;
-  long src_plane, dst_plane;
-  int ls;   // LDS line stride (at least max(h1, h2))
-  int ncp;  // column-pair tiles per plane
+  long src_plane, dst_plane;  // plane strides (elements)
 };
-
-template <typename T, int CP, typename RES>
-__device__ __forceinline__ void cols_resample_body(const ColResArgs<T>& a, unsigned char* smem, RES&& res) {
-  const int h1 = a.h1, h2 = a.h2, LS = a.ls;
-  Cplx<T>* buf = reinterpret_cast<Cplx<T>*>(smem);
-  const int f = blockIdx.y;
-  const int tile = xcd_tile(blockIdx.x, gridDim.x);
-  const int k = a.k0 + tile / a.ncp;
-  const int p0 = (tile % a.ncp) * CP;  // first column pair
-  int nl = a.W / 2 - p0;
-  if (nl > CP) nl = CP;
-  const T* __restrict__ src = a.src[f] + (long)k * a.src_plane + 2 * p0;
-  for (int idx = threadIdx.x; idx < 2 * CP * h1; idx += blockDim.x) {
-    const int j = idx / (2 * CP), r = idx % (2 * CP);
-    const int l = r >> 1;
-    if (l < nl) {
-      const T v = src[(long)j * a.W + r];
-      if (r & 1) buf[l * LS + j].y = v;
-      else buf[l * LS + j].x = v;
-    }
-  }
-  __syncthreads();
-  const int wave = threadIdx.x / LES_WAVE, nw = blockDim.x / LES_WAVE;
-  for (int l = wave; l < nl; l += nw) res(buf + l * LS);
-  __syncthreads();
-  T* __restrict__ dst = a.dst[f] + (long)k * a.dst_plane + 2 * p0;
-  for (int idx = threadIdx.x; idx < 2 * CP * h2; idx += blockDim.x) {
-    const int j = idx / (2 * CP), r = idx % (2 * CP);
-    const int l = r >> 1;
-    if (l < nl) {
-      const Cplx<T> z = buf[l * LS + j];
-      dst[(long)j * a.W + r] = (r & 1) ? z.y : z.x;
-    }
-  }
-}
-
-// ------------------------------------------------------------------ column resampling 256 <-> 384, in registers
-// The 384-point transform (stages radix 4, 4, 4, 2, 3) splits like the
-// 256-point one: stages 0-1 map inputs a + 24 t (t < 16) of thread a (a < 24)
-// to outputs 16 a + c, stages 2-4 stay in the residue class k mod 16 (thread
-// k < 16 holds k + 16 t, t < 24).  A block resamples 16 complex lines (32
-// real columns, 128-byte row segments) with 384 threads (line l = tid % 16,
-// row class r = tid / 16): the 256-point halves use row classes 0..15, the
-// 384-point first half all 24.  Between the transforms the spectrum is
-// re-laid through LDS with the padding / truncation of wave_remap.
-#define LES_C24_LS 417  // line stride in the exchange buffer (>= c16_pad(383) + 1, = 1 mod 16)
-// exchange-buffer row e of a line: one pad slot after every 16 rows
-__device__ __forceinline__ int c16_pad(int e) { return e + (e >> 4); }
-static_assert(cp_OFF(384, 1) == 3 && cp_OFF(384, 2) == 15 && cp_OFF(384, 3) == 63 && cp_OFF(384, 4) == 127,
-              "384-point twiddle layout");
-
-// stages 2-4 of the 384-point transform: X[t] = z''[k + 16 t] -> X[t] = Z[k + 16 t]
-template <typename T>
-__device__ __forceinline__ void c24_pair_b(Cplx<T>* X, const Cplx<T>* __restrict__ twf, int k, bool inverse) {
-  const int sgn = inverse ? 1 : -1;
-  Cplx<T> V[24];
-#pragma unroll
-  for (int q = 0; q < 6; ++q) {  // stage 2 (radix 4, span 16): butterfly 16 q + k
-    Cplx<T> x[4] = {X[q], X[q + 6], X[q + 12], X[q + 18]};
-#pragma unroll
-    for (int r = 1; r < 4; ++r) x[r] = c_mul(x[r], tw16(twf, 15 + (r - 1) * 16 + k, inverse));
-    bfly(x, 4, sgn);
-#pragma unroll
-    for (int r = 0; r < 4; ++r) V[4 * q + r] = x[r];
-  }
-#pragma unroll
-  for (int u = 0; u < 12; ++u) {  // stage 3 (radix 2, span 64): butterfly 16 u + k
-    Cplx<T> x[4] = {V[u], c_mul(V[u + 12], tw16(twf, 63 + 16 * (u % 4) + k, inverse)), V[u], V[u]};
-    bfly(x, 2, sgn);
-    X[8 * (u / 4) + (u % 4)] = x[0];
-    X[8 * (u / 4) + (u % 4) + 4] = x[1];
-  }
-#pragma unroll
-  for (int v = 0; v < 8; ++v) {  // stage 4 (radix 3, span 128): butterfly k + 16 v
-    Cplx<T> x[4] = {X[v], X[v + 8], X[v + 16], X[v]};
-#pragma unroll
-    for (int r = 1; r < 3; ++r) x[r] = c_mul(x[r], tw16(twf, 127 + (r - 1) * 128 + k + 16 * v, inverse));
-    bfly(x, 3, sgn);
-    V[v] = x[0];
-    V[v + 8] = x[1];
-    V[v + 16] = x[2];
-  }
-#pragma unroll
-  for (int t = 0; t < 24; ++t) X[t] = V[t];
-}
-
-// PAD: 256 -> 384 rows (forward 256, pad, inverse 384); else 384 -> 256.
-// FP32: held to 96 VGPRs (5 waves per SIMD instead of 4; two VGPRs spill
-// in the padding direction).
-template <typename T, bool PAD>
-__global__ void __launch_bounds__(384) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? 5 : 1)))
-k_colres_c16(ColResArgs<T> a, const Cplx<T>* __restrict__ tw256,
-                                                    const Cplx<T>* __restrict__ tw384) {
-  extern __shared__ __align__(16) unsigned char smem_raw[];
-  Cplx<T>* ex = reinterpret_cast<Cplx<T>*>(smem_raw);
-  const int l = threadIdx.x & 15, rc = threadIdx.x >> 4;  // line, row class (0..23)
-  const int f = blockIdx.y;
-  const int tile = xcd_tile(blockIdx.x, gridDim.x);
-  const int k = a.k0 + tile / a.ncp;
-  const int p0 = (tile % a.ncp) * 16;  // first line (column pair)
-  const bool valid = p0 + l < a.W / 2;
-  const long col = 2L * (valid ? p0 + l : 0);
-  const Cplx<T>* __restrict__ src = reinterpret_cast<const Cplx<T>*>(a.src[f] + (long)k * a.src_plane + col);
-  Cplx<T>* __restrict__ dst = reinterpret_cast<Cplx<T>*>(a.dst[f] + (long)k * a.dst_plane + col);
-  const long rs = a.W / 2;  // row stride in complex elements
-  Cplx<T>* line = ex + l * LES_C24_LS;
-  const Cplx<T> zero = {(T)0, (T)0};
-  Cplx<T> X[24];
-  if constexpr (PAD) {
-    // forward 256: rows rc + 16 t
-    if (rc < 16) {
-#pragma unroll
-      for (int t = 0; t < 16; ++t) X[t] = valid ? src[(long)(rc + 16 * t) * rs] : zero;
-      c16_pair_a(X, tw256, false);
-#pragma unroll
-      for (int c = 0; c < 16; ++c) lds_st(line + c16_pad(16 * rc + c), X[c]);
-    }
-    __syncthreads();
-    if (rc < 16) {
-#pragma unroll
-      for (int t = 0; t < 16; ++t) X[t] = lds_ld(line + c16_pad(rc + 16 * t));
-    }
-    __syncthreads();
-    if (rc < 16) {
-      c16_pair_b(X, tw256, rc, false);
-      // spectrum rows m = rc + 16 t of 256 -> rows of 384: m < 128 kept, 128
-      // (Nyquist) dropped, m > 128 -> m + 128; rows 128..256 zero
-#pragma unroll
-      for (int t = 0; t < 16; ++t) {
-        const int m = rc + 16 * t;
-        if (m != 128) {
-          const int e = m < 128 ? m : m + 128;
-          lds_st(line + c16_pad(e), X[t]);
-        }
-      }
-#pragma unroll
-      for (int t = 0; t < 8; ++t) lds_st(line + c16_pad(128 + rc + 16 * t), zero);
-      if (rc == 0) lds_st(line + c16_pad(256), zero);
-    }
-    __syncthreads();
-    // inverse 384, first half: rows rc + 24 t
-#pragma unroll
-    for (int t = 0; t < 16; ++t) X[t] = lds_ld(line + c16_pad(rc + 24 * t));
-    __syncthreads();
-    c16_pair_a(X, tw384, true);
-#pragma unroll
-    for (int c = 0; c < 16; ++c) lds_st(line + c16_pad(16 * rc + c), X[c]);
-    __syncthreads();
-    if (rc < 16) {
-#pragma unroll
-      for (int t = 0; t < 24; ++t) X[t] = lds_ld(line + c16_pad(rc + 16 * t));
-      c24_pair_b(X, tw384, rc, true);
-      if (valid) {
-#pragma unroll
-        for (int t = 0; t < 24; ++t) dst[(long)(rc + 16 * t) * rs] = X[t];
-      }
-    }
-  } else {
-    // forward 384, first half: rows rc + 24 t
-#pragma unroll
-    for (int t = 0; t < 16; ++t) X[t] = valid ? src[(long)(rc + 24 * t) * rs] : zero;
-    c16_pair_a(X, tw384, false);
-#pragma unroll
-    for (int c = 0; c < 16; ++c) lds_st(line + c16_pad(16 * rc + c), X[c]);
-    __syncthreads();
-    if (rc < 16) {
-#pragma unroll
-      for (int t = 0; t < 24; ++t) X[t] = lds_ld(line + c16_pad(rc + 16 * t));
-    }
-    __syncthreads();
-    if (rc < 16) {
-      c24_pair_b(X, tw384, rc, false);
-      // spectrum rows m = rc + 16 t of 384 -> rows of 256: m < 128 kept,
-      // m > 256 -> m - 128, the rest dropped; row 128 zero
-#pragma unroll
-      for (int t = 0; t < 24; ++t) {
-        const int m = rc + 16 * t;
-        if (m < 128) lds_st(line + c16_pad(m), X[t]);
-        else if (m > 256) lds_st(line + c16_pad(m - 128), X[t]);
-      }
-      if (rc == 0) lds_st(line + c16_pad(128), zero);
-    }
-    __syncthreads();
-    // inverse 256
-    if (rc < 16) {
-#pragma unroll
-      for (int t = 0; t < 16; ++t) X[t] = lds_ld(line + c16_pad(rc + 16 * t));
-    }
-    __syncthreads();
-    if (rc < 16) {
-      c16_pair_a(X, tw256, true);
-#pragma unroll
-      for (int c = 0; c < 16; ++c) lds_st(line + c16_pad(16 * rc + c), X[c]);
-    }
-    __syncthreads();
-    if (rc < 16) {
-#pragma unroll
-      for (int t = 0; t < 16; ++t) X[t] = lds_ld(line + c16_pad(rc + 16 * t));
-      c16_pair_b(X, tw256, rc, true);
-      if (valid) {
-#pragma unroll
-        for (int t = 0; t < 16; ++t) dst[(long)(rc + 16 * t) * rs] = X[t];
-      }
-    }
-  }
-}
-
-template <typename T, int CP>
-__global__ void __launch_bounds__(LES_BLOCK) k_cols_resample(ColResArgs<T> a, FftPlan p1, FftPlan p2,
-                                                             const Cplx<T>* __restrict__ tw) {
-  extern __shared__ __align__(16) unsigned char smem_raw[];
-  const int lane = threadIdx.x & (LES_WAVE - 1);
-  if constexpr (sizeof(T) == 4) {
-    if (p1.n == 256 && p2.n == 384) {
-      TwReg<T, 256> ta;
-      TwReg<T, 384> tb;
-      tw_load(ta, tw + p1.twf, lane);
-      tw_load(tb, tw + p2.twf, lane);
-      cols_resample_body<T, CP>(a, smem_raw, [&](Cplx<T>* q) {
-        wave_fft_t(q, ta, false, lane);
-        wave_remap(q, 256, 384, lane);
-        wave_fft_t(q, tb, true, lane);
-      });
-      return;
-    }
-    if (p1.n == 384 && p2.n == 256) {
-      TwReg<T, 384> ta;
-      TwReg<T, 256> tb;
-      tw_load(ta, tw + p1.twf, lane);
-      tw_load(tb, tw + p2.twf, lane);
-      cols_resample_body<T, CP>(a, smem_raw, [&](Cplx<T>* q) {
-        wave_fft_t(q, ta, false, lane);
-        wave_remap(q, 384, 256, lane);
-        wave_fft_t(q, tb, true, lane);
-      });
-      return;
-    }
-  }
-  cols_resample_body<T, CP>(a, smem_raw, [&](Cplx<T>* q) {
-    wave_fft(q, p1, tw, false, lane);
-    wave_remap(q, a.h1, a.h2, lane);
-    wave_fft(q, p2, tw, true, lane);
-  });
-}

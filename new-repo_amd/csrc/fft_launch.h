@@ -11,11 +11,23 @@
 template <typename T, int PART>
 bool cols_reg_part(bool attr, int ny, int op, int nout, bool fwd, bool inv, const ColArgs<T>& a, int njobs,
                    const Cplx<T>* tw, hipStream_t s);
+// Column resampling n <-> 3 n / 2 of nf fields; twn, twb: the forward tables
+// of n and 3 n / 2.
+template <typename T, int PART>
+bool colres_reg_part(bool attr, int n, bool pad, const ColResArgs<T>& a, int nf, const Cplx<T>* twn, const Cplx<T>* twb,
+                     hipStream_t s);
 
 template <typename T, int PART = 0>
 static bool cols_reg(bool attr, int ny, int op, int nout, bool fwd, bool inv, const ColArgs<T>& a, int njobs,
                      const Cplx<T>* tw, hipStream_t s) {
   if (cols_reg_part<T, PART>(attr, ny, op, nout, fwd, inv, a, njobs, tw, s)) return true;
   if constexpr (PART + 1 < LES_LENGTH_PARTS) return cols_reg<T, PART + 1>(attr, ny, op, nout, fwd, inv, a, njobs, tw, s);
+  return false;
+}
+template <typename T, int PART = 0>
+static bool colres_reg(bool attr, int n, bool pad, const ColResArgs<T>& a, int nf, const Cplx<T>* twn, const Cplx<T>* twb,
+                       hipStream_t s) {
+  if (colres_reg_part<T, PART>(attr, n, pad, a, nf, twn, twb, s)) return true;
+  if constexpr (PART + 1 < LES_LENGTH_PARTS) return colres_reg<T, PART + 1>(attr, n, pad, a, nf, twn, twb, s);
   return false;
 }

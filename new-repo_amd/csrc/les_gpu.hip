@@ -215,18 +215,6 @@ static void rows_c2r(Les& L, const Cplx<T>* const* src, TO* const* dst, int nf, 
          "k_rows_c2r", sizeof(T), sizeof(TO));
 }
 
-// LDS line stride (in line elements of eb bytes, at least n) for a tile of
-// `lines` lines filled and drained row by row (consecutive lanes take
-// consecutive lines, then the next row).  One LDS cycle serves 128 bytes:
-// g = 128 / eb lanes spread over r = g / lines rows.  A stride of r (mod g)
-// puts line c, row j at bank slot c r + j, all distinct.
-static int lds_stride(int n, int lines, int eb) {
-  const int g = 128 / eb;
-  const int r = lines >= g ? 1 : g / lines;
-  int st = n;
-  while (st % g != r % g) ++st;
-  return st;
-}
 // The same column op on njobs (at most LES_COL_JOBS) independent sets of
 // inputs and outputs in one launch: the sets' tiles share the grid, so the
 // partly filled last round of blocks is paid once instead of once per set.
@@ -948,18 +936,13 @@ static int setup_kernel_attrs(const Les& L) {
   if (!cols_reg<double>(true, L.ny, 0, 0, 0, 0, ColArgs<double>(), 0, nullptr, 0) ||
       !cols_reg<float>(true, L.ny, 0, 0, 0, 0, ColArgs<float>(), 0, nullptr, 0))
     return 10;
-  hipFuncSetAttribute((const void*)k_colres_c16<float, true>, hipFuncAttributeMaxDynamicSharedMemorySize, big);
-  hipFuncSetAttribute((const void*)k_colres_c16<float, false>, hipFuncAttributeMaxDynamicSharedMemorySize, big);
-  hipFuncSetAttribute((const void*)k_colres_c16<double, true>, hipFuncAttributeMaxDynamicSharedMemorySize, big);
-  hipFuncSetAttribute((const void*)k_colres_c16<double, false>, hipFuncAttributeMaxDynamicSharedMemorySize, big);
   hipFuncSetAttribute((const void*)k_rows_resample<double, double, double>, hipFuncAttributeMaxDynamicSharedMemorySize, big);
   hipFuncSetAttribute((const void*)k_rows_resample<float, double, float>, hipFuncAttributeMaxDynamicSharedMemorySize, big);
   hipFuncSetAttribute((const void*)k_rows_resample<float, float, float>, hipFuncAttributeMaxDynamicSharedMemorySize, big);
   hipFuncSetAttribute((const void*)k_rows_resample<float, double, double>, hipFuncAttributeMaxDynamicSharedMemorySize, big);
-  hipFuncSetAttribute((const void*)k_cols_resample<double, LES_COLRES_TILE_BYTES / 16>,
-                      hipFuncAttributeMaxDynamicSharedMemorySize, big);
-  hipFuncSetAttribute((const void*)k_cols_resample<float, LES_COLRES_TILE_BYTES / 8>,
-                      hipFuncAttributeMaxDynamicSharedMemorySize, big);
+  if (!colres_reg<double>(true, L.ny, true, ColResArgs<double>(), 0, nullptr, nullptr, 0) ||
+      !colres_reg<float>(true, L.ny, true, ColResArgs<float>(), 0, nullptr, nullptr, 0))
+    return 10;
   return 0;
 }
 

@@ -74,49 +74,10 @@ __global__ void k_set_planes(SetPlaneArgs s) {
 }
 
 // compute_dealias_convec (src/compute_convective_padd.f90:115-262)
-// Column-pair tiles of LES_COLRES_TILE_BYTES contiguous bytes per row.
-#ifndef LES_COLRES_TILE_BYTES
-#define LES_COLRES_TILE_BYTES 64
-#endif
-// 256 <-> 384: register-resident kernel (k_colres_c16); LES_COLRES16=0
-// selects the LDS-engine kernel (k_cols_resample) instead, LES_COLRES16_FP64=0
-// for the FP64 path only.
-#ifndef LES_COLRES16
-#define LES_COLRES16 1
-#endif
-#ifndef LES_COLRES16_FP64
-#define LES_COLRES16_FP64 1
-#endif
-// the kernel launch_cols_resample runs for the column lengths h1 -> h2
-static const char* colres_name(int h1, int h2) {
-  return (LES_COLRES16 && ((h1 == 256 && h2 == 384) || (h1 == 384 && h2 == 256))) ? "k_colres_c16" : "k_cols_resample";
-}
-
+// (the y resampling: k_colres_reg, colres_reg.h)
 template <typename T>
-static void launch_cols_resample(Les& L, ColResArgs<T>& a, int nf, const FftPlan& p1, const FftPlan& p2) {
-  if constexpr (LES_COLRES16 && (sizeof(T) == 4 || LES_COLRES16_FP64)) {
-   if ((a.h1 == 256 && a.h2 == 384) || (a.h1 == 384 && a.h2 == 256)) {
-    // register-resident 256 <-> 384 (k_colres_c16)
-    a.ncp = (a.W / 2 + 15) / 16;
-    a.ls = LES_C24_LS;
-    const size_t sh = (size_t)16 * LES_C24_LS * sizeof(Cplx<T>);
-    const Cplx<T>* t256 = twpool<T>(L) + (p1.n == 256 ? p1.twf : p2.twf);
-    const Cplx<T>* t384 = twpool<T>(L) + (p1.n == 384 ? p1.twf : p2.twf);
-    const dim3 g((unsigned)(a.ncp * a.nplanes), nf);
-    if (a.h1 == 256)
-      hipLaunchKernelGGL((k_colres_c16<T, true>), g, dim3(384), sh, L.stream, a, t256, t384);
-    else
-      hipLaunchKernelGGL((k_colres_c16<T, false>), g, dim3(384), sh, L.stream, a, t256, t384);
-    return;
-   }
-  }
-  constexpr int CP = LES_COLRES_TILE_BYTES / 2 / (int)sizeof(T);
-  const int nm = a.h1 > a.h2 ? a.h1 : a.h2;
-  a.ls = lds_stride(nm, CP, (int)sizeof(Cplx<T>));
-  a.ncp = (a.W / 2 + CP - 1) / CP;
-  const size_t sh = (size_t)CP * a.ls * sizeof(Cplx<T>);
-  hipLaunchKernelGGL((k_cols_resample<T, CP>), dim3((unsigned)(a.ncp * a.nplanes), nf), dim3(LES_BLOCK), sh, L.stream, a,
-                     p1, p2, twpool<T>(L));
+static void launch_cols_resample(Les& L, const ColResArgs<T>& a, int nf, bool pad) {
+  colres_reg<T>(false, L.ny, pad, a, nf, twpool<T>(L) + L.py.twf, twpool<T>(L) + L.py2.twf, L.stream);
 }
 
 // Real multiplier g on the 2D spectrum of planes 1..nlev of nf real fields:
@@ -238,11 +199,11 @@ static void convection(Les& L, double* cx, double* cy, double* cz) {
   {
     ColResArgs<T> a;
     for (int f = 0; f < 6; ++f) { a.src[f] = (const T*)L.wk_hyb[f]; a.dst[f] = (T*)L.wk_big[f]; }
-    a.W = nx2; a.h1 = ny; a.h2 = ny2; a.k0 = 1; a.nplanes = nz + 1;
+    a.W = nx2; a.k0 = 1; a.nplanes = nz + 1;
     a.src_plane = (long)nx2 * ny; a.dst_plane = L.nbp;
     kt_begin(L, KT_COLS_RES);
-    launch_cols_resample<T>(L, a, 6, L.py, L.py2);
-    kt_end(L, KT_COLS_RES, 6.0 * a.nplanes * nx2 * (double)(ny + ny2) * sizeof(T), colres_name(ny, ny2), sizeof(T), 0, "pad");
+    launch_cols_resample<T>(L, a, 6, true);
+    kt_end(L, KT_COLS_RES, 6.0 * a.nplanes * nx2 * (double)(ny + ny2) * sizeof(T), "k_colres_reg", sizeof(T), 0, "pad");
   }
   // products
   {
@@ -260,11 +221,11 @@ static void convection(Les& L, double* cx, double* cy, double* cz) {
   {
     ColResArgs<T> a;
     for (int f = 0; f < 3; ++f) { a.src[f] = (const T*)L.wk_prod[f]; a.dst[f] = (T*)L.wk_hyb3[f]; }
-    a.W = nx2; a.h1 = ny2; a.h2 = ny; a.k0 = 1; a.nplanes = nz;
+    a.W = nx2; a.k0 = 1; a.nplanes = nz;
     a.src_plane = L.nbp; a.dst_plane = (long)nx2 * ny;
     kt_begin(L, KT_COLS_RES);
-    launch_cols_resample<T>(L, a, 3, L.py2, L.py);
-    kt_end(L, KT_COLS_RES, 3.0 * a.nplanes * nx2 * (double)(ny + ny2) * sizeof(T), colres_name(ny2, ny), sizeof(T), 0, "truncate");
+    launch_cols_resample<T>(L, a, 3, false);
+    kt_end(L, KT_COLS_RES, 3.0 * a.nplanes * nx2 * (double)(ny + ny2) * sizeof(T), "k_colres_reg", sizeof(T), 0, "truncate");
   }
   // truncate in x, straight into rhs
   {

@@ -117,7 +117,7 @@ def rocprof_key(name: str) -> str:
 # kernel-name patterns of the benchmark's kernel families
 FAMILY_KERNELS = {"rows_r2c": r"\bk_rows_r2c<", "rows_c2r": r"\bk_rows_c2r(_div<|_proj\(|<)",
                   "cols": r"\bk_cols_reg<", "rows_resample": r"\bk_rows_resample<",
-                  "cols_resample": r"\bk_(cols_resample|colres_c16)<", "tridiag": r"\bk_tridiag",
+                  "cols_resample": r"\bk_colres_reg<", "tridiag": r"\bk_tridiag",
                   "lagrangian": r"\bk_lagr<"}
 
 
