@@ -9,7 +9,7 @@
  *   0 ok, 1 invalid option/model, 3 out of memory, 4 double initialisation,
  *   5 HIP runtime error, 9 NaN found / singular solve, 10 bad shape or id.
  * Calls come from one host thread; every entry point runs its kernels on the
- * library's HIP stream (les_step also uses a second one inside a step, joined
+ * default (null) HIP stream (les_step also uses side streams inside a step, joined
  * before it returns, see les_set_overlap); host buffers are synchronised only
  * by download/status calls.  Not reentrant,
  * like the reference's module state.

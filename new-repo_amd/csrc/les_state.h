@@ -25,7 +25,7 @@ struct Les {
   int jt_total;
   int jt;                // steps since les_init (the reference's local count)
   int F_coeff_init;
-  hipStream_t stream;
+  hipStream_t stream;    // the stream calls run on: the default (null) one, except while a step issues work to a side stream
   hipStream_t stream2;   // second stream of the step: the SGS stage beside the convection
   hipEvent_t ev_fork, ev_join;
   hipStream_t stream3;   // learned mode: the surrogate's chain beside the band's plain update
