@@ -30,7 +30,9 @@ HIP_FLAGS = [
 
 # (source, defines): the kernels with one instance per transform length are
 # compiled in parts, side by side
-SOURCES = [("les_gpu.hip", {})] + [("fft_cols.hip", {"LES_T": t, "LES_PART": p}) for t in ("double", "float") for p in range(4)]
+SOURCES = [("les_gpu.hip", {})] + [(f, {"LES_T": t, "LES_FP32": int(t == "float"), "LES_PART": p})
+                                   for p in range(4) for t in ("double", "float")
+                                   for f in ("fft_rows.hip", "fft_cols.hip")]
 
 
 def _run(cmd, cwd=None):

@@ -21,7 +21,7 @@
 // LOAD_AB2_SCALE_DIV: the AB2 predictor u + dt (t1 r + t2 r_f) of each
 // value (the arithmetic of k_ab2, src/LES_engine.f90:253-283), then
 // LOAD_SCALE_DIV: the pressure right-hand side straight from u, rhs, rhs_f.
-// LOAD_PCLEAN (the PCL instance only): the TKE budget's cleaned pressure
+// LOAD_PCLEAN: the TKE budget's cleaned pressure
 // p - (u u + v v + W W) / 2, W = (w(k) + w(k+1)) / 2, from p (src) and u, v, w
 // (ab_r), 0 on the planes 0 and nz+1.
 enum { LOAD_SCALE = 0, LOAD_SCALE_DIV = 1, LOAD_AB2_SCALE_DIV = 2, LOAD_PCLEAN = 3 };
@@ -56,11 +56,11 @@ __host__ __device__ constexpr int row_line(int n) {
   return row_layout<T>(n) == LES_LAY_PAD ? lds_line_cap(n) : n;
 }
 
-// One wavefront per row pair: load, transform and unpack without any
-// block-level barrier.  LDS: one line of a.ls points per wavefront.
-template <bool NYQ = false, bool PCL = false, typename TI, typename T, typename FFT>
-__device__ __forceinline__ void rows_r2c_body(const RowR2CArgs<TI, T>& a, Cplx<T>* z, int lane, long job, FFT&& fft,
-                                              double* part = nullptr) {
+// One wavefront per row pair, the line in LDS (a.ls points per wavefront): load
+// with the Nyquist sums, transform and unpack without any block-level barrier.
+template <typename TI, typename T, typename FFT>
+__device__ __forceinline__ void rows_r2c_nyq_body(const RowR2CArgs<TI, T>& a, Cplx<T>* z, int lane, long job, FFT&& fft,
+                                                  double* part) {
   const int nx = a.nx, lhx = a.lhx;
   const int npairs = a.ny / 2;
   const int f = blockIdx.y;
@@ -68,55 +68,21 @@ __device__ __forceinline__ void rows_r2c_body(const RowR2CArgs<TI, T>& a, Cplx<T
   const TI* __restrict__ src = a.src[f] + ((long)k * a.ny + 2 * jp) * nx;
   double s0 = 0.0, s1 = 0.0;
   for (int n = lane; n < nx; n += LES_WAVE) {
-    if constexpr (NYQ) {
-      // alternating row sums and the pair's column partial (-1)^j f, in FP64
-      const double r0 = src[n], r1 = src[n + nx];
-      s0 += (n & 1) ? -r0 : r0;
-      s1 += (n & 1) ? -r1 : r1;
-      part[n] = r0 - r1;
-    }
-    T v0 = (T)src[n], v1 = (T)src[n + nx];
-    if (a.mode == LOAD_AB2_SCALE_DIV) {
-      const long o = ((long)k * a.ny + 2 * jp) * nx + n;
-      const TI* __restrict__ r = a.ab_r[f];
-      const TI* __restrict__ rf = a.ab_f[f];
-      v0 = v0 + a.ab_dt * (a.ab_t1 * (T)r[o] + a.ab_t2 * (T)rf[o]);
-      v1 = v1 + a.ab_dt * (a.ab_t1 * (T)r[o + nx] + a.ab_t2 * (T)rf[o + nx]);
-    }
-    if constexpr (PCL) {
-      if (k == 0 || k == a.pc_nz + 1) {
-        v0 = (T)0;
-        v1 = (T)0;
-      } else {
-        const long o = ((long)k * a.ny + 2 * jp) * nx + n, pl = (long)a.ny * nx;
-        const TI* __restrict__ u = a.ab_r[0];
-        const TI* __restrict__ v = a.ab_r[1];
-        const TI* __restrict__ w = a.ab_r[2];
-        const T h0 = (T)0.5 * ((T)w[o] + (T)w[o + pl]);
-        const T h1 = (T)0.5 * ((T)w[o + nx] + (T)w[o + nx + pl]);
-        v0 = v0 - (T)0.5 * (((T)u[o] * (T)u[o] + (T)v[o] * (T)v[o]) + h0 * h0);
-        v1 = v1 - (T)0.5 * (((T)u[o + nx] * (T)u[o + nx] + (T)v[o + nx] * (T)v[o + nx]) + h1 * h1);
-      }
-    }
-    if (a.mode == LOAD_SCALE_DIV || a.mode == LOAD_AB2_SCALE_DIV) {
-      v0 = a.scale * (v0 / a.div);
-      v1 = a.scale * (v1 / a.div);
-    } else {
-      v0 = a.scale * v0;
-      v1 = a.scale * v1;
-    }
-    z[n] = {v0, v1};
+    // alternating row sums and the pair's column partial (-1)^j f, in FP64
+    const double r0 = src[n], r1 = src[n + nx];
+    s0 += (n & 1) ? -r0 : r0;
+    s1 += (n & 1) ? -r1 : r1;
+    part[n] = r0 - r1;
+    z[n] = {a.scale * (T)r0, a.scale * (T)r1};
   }
-  if constexpr (NYQ) {
-    for (int o = LES_WAVE / 2; o > 0; o >>= 1) {
-      s0 += __shfl_xor(s0, o, LES_WAVE);
-      s1 += __shfl_xor(s1, o, LES_WAVE);
-    }
-    if (lane == 0) {
-      double* A = a.nyq_a + (long)k * a.ny + 2 * jp;
-      A[0] = s0 / (double)nx;
-      A[1] = s1 / (double)nx;
-    }
+  for (int o = LES_WAVE / 2; o > 0; o >>= 1) {
+    s0 += __shfl_xor(s0, o, LES_WAVE);
+    s1 += __shfl_xor(s1, o, LES_WAVE);
+  }
+  if (lane == 0) {
+    double* A = a.nyq_a + (long)k * a.ny + 2 * jp;
+    A[0] = s0 / (double)nx;
+    A[1] = s1 / (double)nx;
   }
   wave_sync();
   fft(z, false);
@@ -130,25 +96,7 @@ __device__ __forceinline__ void rows_r2c_body(const RowR2CArgs<TI, T>& a, Cplx<T
   }
 }
 
-// FP32: held to 64 VGPRs (8 waves per SIMD instead of 7; two VGPRs spill).
-template <typename TI, typename T, bool PCL = false>
-__global__ void __launch_bounds__(LES_BLOCK) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? 8 : 1)))
-k_rows_r2c(RowR2CArgs<TI, T> a, FftPlan pl, const Cplx<T>* __restrict__ tw) {
-  extern __shared__ __align__(16) unsigned char smem_raw[];
-  const int lane = threadIdx.x & (LES_WAVE - 1), wave = threadIdx.x / LES_WAVE;
-  Cplx<T>* z = reinterpret_cast<Cplx<T>*>(smem_raw) + wave * a.ls;
-  const long job = (long)blockIdx.x * (blockDim.x / LES_WAVE) + wave;
-  if (job >= (long)a.nplanes * (a.ny / 2)) return;
-  if (pl.n == 256) {
-    TwReg<T, 256> tr;
-    tw_load(tr, tw + pl.twf, lane);
-    rows_r2c_body<false, PCL>(a, z, lane, job, [&](Cplx<T>* p, bool inv) { wave_fft_t<T, 256, row_layout<T>(256)>(p, tr, inv, lane); });
-  } else {
-    rows_r2c_body<false, PCL>(a, z, lane, job, [&](Cplx<T>* p, bool inv) { wave_fft(p, pl, tw, inv, lane); });
-  }
-}
-
-// k_rows_r2c with the first pass of the mixed mode's FP64 Nyquist removal
+// k_rows_r2c_reg with the first pass of the mixed mode's FP64 Nyquist removal
 // folded into the load (the sums k_nyq_reduce forms, from the values this
 // kernel reads anyway): A_j = sum_i (-1)^i f_ij / nx of both rows (the same
 // lane-strided sums and butterfly as k_nyq_reduce), and per block of 4 row
@@ -172,10 +120,10 @@ k_rows_r2c_nyq(RowR2CArgs<double, T> a, FftPlan pl, const Cplx<T>* __restrict__ 
   if (pl.n == 256) {
     TwReg<T, 256> tr;
     tw_load(tr, tw + pl.twf, lane);
-    rows_r2c_body<true>(a, z, lane, job, [&](Cplx<T>* p, bool inv) { wave_fft_t<T, 256, row_layout<T>(256)>(p, tr, inv, lane); },
+    rows_r2c_nyq_body(a, z, lane, job, [&](Cplx<T>* p, bool inv) { wave_fft_t<T, 256, row_layout<T>(256)>(p, tr, inv, lane); },
                         part + wave * a.nx);
   } else {
-    rows_r2c_body<true>(a, z, lane, job, [&](Cplx<T>* p, bool inv) { wave_fft(p, pl, tw, inv, lane); }, part + wave * a.nx);
+    rows_r2c_nyq_body(a, z, lane, job, [&](Cplx<T>* p, bool inv) { wave_fft(p, pl, tw, inv, lane); }, part + wave * a.nx);
   }
   __syncthreads();
   const int nx = a.nx;
@@ -191,60 +139,7 @@ struct RowC2RArgs {
   TO* dst[LES_MAX_FIELDS];
   int nx, ny, lhx;
   int k0, nplanes;
-  int ls;  // LDS line stride per wavefront (row_line<T>(nx))
 };
-
-// Load the half spectra of rows (2jp, 2jp+1) of plane k as one complex line
-// and run the inverse transform: z then holds row 2jp in .x, row 2jp+1 in .y.
-template <typename T, typename TO, typename FFT>
-__device__ __forceinline__ void rows_c2r_line(const RowC2RArgs<T, TO>& a, Cplx<T>* z, int lane, int k, int jp, FFT&& fft) {
-  const int nx = a.nx, lhx = a.lhx, h = nx / 2;
-  const int f = blockIdx.y;
-  const Cplx<T>* __restrict__ src = a.src[f] + ((long)k * a.ny + 2 * jp) * lhx;
-  for (int kk = lane; kk < lhx; kk += LES_WAVE) {
-    Cplx<T> A = src[kk], B = src[kk + lhx];
-    if (kk == 0 || kk == h) {
-      A.y = (T)0;
-      B.y = (T)0;
-    }
-    z[kk] = {A.x - B.y, A.y + B.x};
-    if (kk != 0 && kk != h) z[nx - kk] = {A.x + B.y, B.x - A.y};
-  }
-  wave_sync();
-  fft(z, true);
-}
-
-template <typename T, typename TO, typename FFT>
-__device__ __forceinline__ void rows_c2r_body(const RowC2RArgs<T, TO>& a, Cplx<T>* z, int lane, long job, FFT&& fft) {
-  const int nx = a.nx;
-  const int npairs = a.ny / 2;
-  const int k = a.k0 + (int)(job / npairs), jp = (int)(job % npairs);
-  rows_c2r_line(a, z, lane, k, jp, fft);
-  TO* __restrict__ dst = a.dst[blockIdx.y] + ((long)k * a.ny + 2 * jp) * nx;
-  for (int n = lane; n < nx; n += LES_WAVE) {
-    const Cplx<T> v = z[n];
-    dst[n] = (TO)v.x;
-    dst[n + nx] = (TO)v.y;
-  }
-}
-
-// FP32: held to 64 VGPRs, as the r2c kernel.
-template <typename T, typename TO>
-__global__ void __launch_bounds__(LES_BLOCK) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? 8 : 1)))
-k_rows_c2r(RowC2RArgs<T, TO> a, FftPlan pl, const Cplx<T>* __restrict__ tw) {
-  extern __shared__ __align__(16) unsigned char smem_raw[];
-  const int lane = threadIdx.x & (LES_WAVE - 1), wave = threadIdx.x / LES_WAVE;
-  Cplx<T>* z = reinterpret_cast<Cplx<T>*>(smem_raw) + wave * a.ls;
-  const long job = (long)blockIdx.x * (blockDim.x / LES_WAVE) + wave;
-  if (job >= (long)a.nplanes * (a.ny / 2)) return;
-  if (pl.n == 256) {
-    TwReg<T, 256> tr;
-    tw_load(tr, tw + pl.twf, lane);
-    rows_c2r_body(a, z, lane, job, [&](Cplx<T>* p, bool inv) { wave_fft_t<T, 256, row_layout<T>(256)>(p, tr, inv, lane); });
-  } else {
-    rows_c2r_body(a, z, lane, job, [&](Cplx<T>* p, bool inv) { wave_fft(p, pl, tw, inv, lane); });
-  }
-}
 
 // ------------------------------------------------------------------ columns
 // Spectral-space operations applied between the forward and inverse y passes.
@@ -294,143 +189,17 @@ __device__ __forceinline__ T conv_src(const ConvSrc<TI>& s, int which, int k, lo
   }
 }
 
-// Row resampling: real rows of length n1 -> real rows of length n2, one
-// wavefront per row pair (transform, pad or truncate in place, transform
-// back).  src_mode 0: plain real array (nx = n1) src[f]; src_mode 1:
-// convection sources (field = blockIdx.y) computed from ConvSrc.
+// Row resampling (k_rows_resample_reg, rows_reg.h): padding computes the
+// convection sources (field = blockIdx.y) from ConvSrc, truncation reads src.
 template <typename T, typename TI, typename TO>
 struct RowResArgs {
   const T* src[LES_MAX_FIELDS];
   TO* dst[LES_MAX_FIELDS];
   ConvSrc<TI> cs;
   T cconv;
-  int src_mode;
-  int n1, n2, ny;
+  int ny;
   int k0, nplanes;
-  long src_plane, dst_plane;  // plane strides (elements)
-  int ls;                     // LDS line stride per wavefront (res_line<T>(n1, n2))
 };
-
-// The FP32 256 <-> 384 pair runs on register twiddles with the padded
-// placement; other lengths on the generic transform (XOR placement).
-template <typename T>
-__host__ __device__ constexpr bool res_fixed(int n1, int n2) {
-  return sizeof(T) == 4 && ((n1 == 256 && n2 == 384) || (n1 == 384 && n2 == 256));
-}
-template <typename T>
-__host__ __device__ constexpr int res_line(int n1, int n2) {
-  return res_fixed<T>(n1, n2) ? lds_line_cap(n1 > n2 ? n1 : n2) : (n1 > n2 ? n1 : n2);
-}
-
-template <typename T, typename TI, typename TO, typename RES>
-__device__ __forceinline__ void rows_resample_body(const RowResArgs<T, TI, TO>& a, Cplx<T>* z, int lane, long job,
-                                                   RES&& res) {
-  const int n1 = a.n1, n2 = a.n2;
-  const int npairs = a.ny / 2;
-  const int f = blockIdx.y;
-  const int k = a.k0 + (int)(job / npairs), jp = (int)(job % npairs);
-  const long np = (long)n1 * a.ny;
-  if (a.src_mode == 1) {
-    for (int n = lane; n < n1; n += LES_WAVE) {
-      const long q = (long)(2 * jp) * n1 + n;
-      z[n] = {conv_src<T, TI>(a.cs, f, k, q, np, a.cconv), conv_src<T, TI>(a.cs, f, k, q + n1, np, a.cconv)};
-    }
-  } else {
-    const T* __restrict__ src = a.src[f] + (long)k * a.src_plane + (long)(2 * jp) * n1;
-    for (int n = lane; n < n1; n += LES_WAVE) z[n] = {src[n], src[n + n1]};
-  }
-  wave_sync();
-  res(z);
-  TO* __restrict__ dst = a.dst[f] + (long)k * a.dst_plane + (long)(2 * jp) * n2;
-  for (int n = lane; n < n2; n += LES_WAVE) {
-    const Cplx<T> v = z[n];
-    dst[n] = (TO)v.x;
-    dst[n + n2] = (TO)v.y;
-  }
-}
-
-// The FP32 256 <-> 384 pair runs on register twiddles (37 per lane); FP32
-// instances are held to 80 VGPRs (6 waves per SIMD, no spills).
-template <typename T, typename TI, typename TO>
-__global__ void __launch_bounds__(LES_BLOCK) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? 6 : 1)))
-k_rows_resample(RowResArgs<T, TI, TO> a, FftPlan p1, FftPlan p2, const Cplx<T>* __restrict__ tw) {
-  extern __shared__ __align__(16) unsigned char smem_raw[];
-  const int lane = threadIdx.x & (LES_WAVE - 1), wave = threadIdx.x / LES_WAVE;
-  Cplx<T>* z = reinterpret_cast<Cplx<T>*>(smem_raw) + wave * a.ls;
-  const long job = (long)blockIdx.x * (blockDim.x / LES_WAVE) + wave;
-  if (job >= (long)a.nplanes * (a.ny / 2)) return;
-  if constexpr (sizeof(T) == 4) {
-    // each transform's twiddles are loaded where it starts, so the two sets
-    // are never live together (fewer VGPRs, more waves per SIMD)
-    if (res_fixed<T>(p1.n, p2.n) && p1.n == 256) {
-      rows_resample_body(a, z, lane, job, [&](Cplx<T>* q) {
-        {
-          TwReg<T, 256> ta;
-          tw_load(ta, tw + p1.twf, lane);
-          wave_fft_t<T, 256, LES_LAY_PAD>(q, ta, false, lane);
-        }
-        wave_remap(q, 256, 384, lane);
-        TwReg<T, 384> tb;
-        tw_load(tb, tw + p2.twf, lane);
-        wave_fft_t<T, 384, LES_LAY_PAD>(q, tb, true, lane);
-      });
-      return;
-    }
-    if (res_fixed<T>(p1.n, p2.n) && p1.n == 384) {
-      rows_resample_body(a, z, lane, job, [&](Cplx<T>* q) {
-        {
-          TwReg<T, 384> ta;
-          tw_load(ta, tw + p1.twf, lane);
-          wave_fft_t<T, 384, LES_LAY_PAD>(q, ta, false, lane);
-        }
-        wave_remap(q, 384, 256, lane);
-        TwReg<T, 256> tb;
-        tw_load(tb, tw + p2.twf, lane);
-        wave_fft_t<T, 256, LES_LAY_PAD>(q, tb, true, lane);
-      });
-      return;
-    }
-  }
-#ifndef LES_RES64_FIXED
-#define LES_RES64_FIXED 1
-#endif
-  if constexpr (sizeof(T) == 8 && LES_RES64_FIXED) {
-    // FP64 256 <-> 384: register twiddles with the XOR placement (line of n2)
-    if ((p1.n == 256 && p2.n == 384) || (p1.n == 384 && p2.n == 256)) {
-      if (p1.n == 256) {
-        rows_resample_body(a, z, lane, job, [&](Cplx<T>* q) {
-          {
-            TwReg<T, 256> ta;
-            tw_load(ta, tw + p1.twf, lane);
-            wave_fft_t<T, 256, LES_LAY_XOR>(q, ta, false, lane);
-          }
-          wave_remap(q, 256, 384, lane);
-          TwReg<T, 384> tb;
-          tw_load(tb, tw + p2.twf, lane);
-          wave_fft_t<T, 384, LES_LAY_XOR>(q, tb, true, lane);
-        });
-      } else {
-        rows_resample_body(a, z, lane, job, [&](Cplx<T>* q) {
-          {
-            TwReg<T, 384> ta;
-            tw_load(ta, tw + p1.twf, lane);
-            wave_fft_t<T, 384, LES_LAY_XOR>(q, ta, false, lane);
-          }
-          wave_remap(q, 384, 256, lane);
-          TwReg<T, 256> tb;
-          tw_load(tb, tw + p2.twf, lane);
-          wave_fft_t<T, 256, LES_LAY_XOR>(q, tb, true, lane);
-        });
-      }
-      return;
-    }
-  }
-  rows_resample_body(a, z, lane, job, [&](Cplx<T>* q) {
-    wave_fft(q, p1, tw, false, lane);
-    wave_remap(q, a.n1, a.n2, lane);
-    wave_fft(q, p2, tw, true, lane);
-  });
-}
 
 // Column resampling: column pairs (i, i+1) of a real (W, h1) plane -> (W, h2)
 // as complex lines (k_colres_reg, colres_reg.h).

@@ -1,7 +1,8 @@
 // Launchers of the kernels that have one instance per transform length,
-// compiled in parts (fft_cols.hip, once per precision and part).
+// compiled in parts (fft_cols.hip and fft_rows.hip, once per precision and part).
 #pragma once
 #include "fft_kernels.h"
+#include "les_epi.h"
 
 #define LES_LENGTH_PARTS 4
 
@@ -30,4 +31,64 @@ static bool colres_reg(bool attr, int n, bool pad, const ColResArgs<T>& a, int n
   if (colres_reg_part<T, PART>(attr, n, pad, a, nf, twn, twb, s)) return true;
   if constexpr (PART + 1 < LES_LENGTH_PARTS) return colres_reg<T, PART + 1>(attr, n, pad, a, nf, twn, twb, s);
   return false;
+}
+
+// Row transforms of length n (nf fields; tw: the forward table of n), the
+// resampling n <-> 3 n / 2 (twn, twb).  attr and the result as above.
+template <typename TI, typename T, int PART>
+bool rows_r2c_part(bool attr, int n, const RowR2CArgs<TI, T>& a, int nf, const Cplx<T>* tw, hipStream_t s);
+template <typename T, typename TO, int PART>
+bool rows_c2r_part(bool attr, int n, const RowC2RArgs<T, TO>& a, int nf, const Cplx<T>* tw, hipStream_t s);
+template <typename T, int PART>
+bool rows_div_part(bool attr, int n, const RowC2RArgs<T, T>& a, const DivEpi3<T>& ep, int nf, const Cplx<T>* tw, hipStream_t s);
+template <typename T, int PART>
+bool rows_proj_part(bool attr, int n, const RowC2RArgs<T, T>& a, const ProjEpi3& ep, int nf, const Cplx<T>* tw, hipStream_t s);
+template <typename T, int PART>
+bool rows_pad_part(bool attr, int n, const RowResArgs<T, T, T>& a, int nf, const Cplx<T>* twn, const Cplx<T>* twb, hipStream_t s);
+template <typename T, int PART>
+bool rows_trunc_part(bool attr, int n, const RowResArgs<T, T, double>& a, int nf, const Cplx<T>* twn, const Cplx<T>* twb,
+                     hipStream_t s);
+
+// the part that has length n, over all parts
+#define LES_EACH_PART(CALL) CALL(0) || CALL(1) || CALL(2) || CALL(3)
+static_assert(LES_LENGTH_PARTS == 4, "LES_EACH_PART lists the parts");
+template <typename TI, typename T>
+static bool rows_r2c_reg(bool attr, int n, const RowR2CArgs<TI, T>& a, int nf, const Cplx<T>* tw, hipStream_t s) {
+#define C(P) (rows_r2c_part<TI, T, P>(attr, n, a, nf, tw, s))
+  return LES_EACH_PART(C);
+#undef C
+}
+template <typename T, typename TO>
+static bool rows_c2r_reg(bool attr, int n, const RowC2RArgs<T, TO>& a, int nf, const Cplx<T>* tw, hipStream_t s) {
+#define C(P) (rows_c2r_part<T, TO, P>(attr, n, a, nf, tw, s))
+  return LES_EACH_PART(C);
+#undef C
+}
+template <typename T>
+static bool rows_div_reg(bool attr, int n, const RowC2RArgs<T, T>& a, const DivEpi3<T>& ep, int nf, const Cplx<T>* tw,
+                         hipStream_t s) {
+#define C(P) (rows_div_part<T, P>(attr, n, a, ep, nf, tw, s))
+  return LES_EACH_PART(C);
+#undef C
+}
+template <typename T>
+static bool rows_proj_reg(bool attr, int n, const RowC2RArgs<T, T>& a, const ProjEpi3& ep, int nf, const Cplx<T>* tw,
+                          hipStream_t s) {
+#define C(P) (rows_proj_part<T, P>(attr, n, a, ep, nf, tw, s))
+  return LES_EACH_PART(C);
+#undef C
+}
+template <typename T>
+static bool rows_pad_reg(bool attr, int n, const RowResArgs<T, T, T>& a, int nf, const Cplx<T>* twn, const Cplx<T>* twb,
+                         hipStream_t s) {
+#define C(P) (rows_pad_part<T, P>(attr, n, a, nf, twn, twb, s))
+  return LES_EACH_PART(C);
+#undef C
+}
+template <typename T>
+static bool rows_trunc_reg(bool attr, int n, const RowResArgs<T, T, double>& a, int nf, const Cplx<T>* twn, const Cplx<T>* twb,
+                           hipStream_t s) {
+#define C(P) (rows_trunc_part<T, P>(attr, n, a, nf, twn, twb, s))
+  return LES_EACH_PART(C);
+#undef C
 }

@@ -130,9 +130,16 @@ __device__ __forceinline__ void ph_stages(Cplx<T>* X, const Cplx<T>* __restrict_
 
 // A line of N values shared by NT threads (this one is number a), through an
 // LDS line of its own.  MAXG: the most values per group (the phase split).
-template <typename T, int N, int NT, int MAXG>
+// PADX: between two phases the line has one unused slot after every G0 values
+// (G0 the first phase's radix, when even), so that neighbouring threads, which
+// write at stride G0, meet different banks; the line then holds XLEN values.
+template <typename T, int N, int NT, int MAXG, bool PADX = false>
 struct RegLine {
   static constexpr PhasePlan plan = ph_plan(N, MAXG);
+  static constexpr int PG = PADX && plan.np > 1 && plan.g[0] % 2 == 0 ? plan.g[0] : 0;
+  static constexpr int XLEN = N + (PG ? N / PG : 0);
+  static constexpr int xstep(int d) { return PG && d % (PG ? PG : 1) == 0 ? d + d / (PG ? PG : 1) : d; }
+  static __device__ __forceinline__ int xpos(int e) { return PG ? e + e / (PG ? PG : 1) : e; }
   static constexpr int NP = plan.np, LAST = plan.np - 1;
   static constexpr int VALS = ph_vals(plan, N, NT);
   template <int Q>
@@ -170,7 +177,8 @@ struct RegLine {
       phase<Q, INVERSE, GI + 1>(X + G, tw, a);
     }
   }
-  // outputs of phase Q to the line, inputs of phase Q + 1 from it
+  // outputs of phase Q to the line, inputs of phase Q + 1 from it (padded
+  // places between two phases; the ending and starting layouts in place)
   template <int Q, int GI = 0>
   static __device__ __forceinline__ void put(const Cplx<T>* X, Cplx<T>* line, int a) {
     if constexpr (GI < ng<Q>()) {
@@ -178,9 +186,9 @@ struct RegLine {
       const int i0 = a + NT * GI;
       if (NGR % NT == 0 || i0 < NGR) {
         const int k = Q == 0 ? 0 : (Q == LAST ? i0 : i0 % P0);
-        Cplx<T>* __restrict__ o = line + ((i0 - k) * G + k);
+        Cplx<T>* __restrict__ o = line + (Q == LAST ? (i0 - k) * G + k : Q == 0 ? i0 * xstep(G) : xpos((i0 - k) * G + k));
 #pragma unroll
-        for (int c = 0; c < G; ++c) lds_st(o + c * P0, X[c]);
+        for (int c = 0; c < G; ++c) lds_st(o + c * (Q == LAST ? P0 : xstep(P0)), X[c]);
       }
       put<Q, GI + 1>(X + G, line, a);
     }
@@ -192,7 +200,7 @@ struct RegLine {
       const int i0 = a + NT * GI;
       if (NGR % NT == 0 || i0 < NGR) {
 #pragma unroll
-        for (int t = 0; t < G; ++t) X[t] = lds_ld(line + i0 + t * NGR);
+        for (int t = 0; t < G; ++t) X[t] = lds_ld(line + (Q == 0 ? i0 + t * NGR : xpos(i0) + t * xstep(NGR)));
       }
       get<Q, GI + 1>(X + G, line, a);
     }

@@ -155,7 +155,6 @@ static void rows_r2c(Les& L, const TI* const* src, Cplx<T>* const* dst, int nf, 
   for (int f = 0; f < nf; ++f) { a.src[f] = src[f]; a.dst[f] = dst[f]; }
   a.nx = L.nx; a.ny = ny_override ? ny_override : L.ny; a.lhx = L.lhx; a.k0 = k0; a.nplanes = npl;
   a.mode = mode; a.scale = scale; a.div = div;
-  a.ls = row_line<T>(L.nx);
   if (mode == LOAD_AB2_SCALE_DIV) {
     for (int f = 0; f < nf && f < 3; ++f) { a.ab_r[f] = ab[f]; a.ab_f[f] = ab[3 + f]; }
     a.ab_dt = abc[0]; a.ab_t1 = abc[1]; a.ab_t2 = abc[2];
@@ -164,17 +163,11 @@ static void rows_r2c(Les& L, const TI* const* src, Cplx<T>* const* dst, int nf, 
     for (int f = 0; f < 3; ++f) a.ab_r[f] = ab[f];
     a.pc_nz = L.nz;
   }
-  long jobs = (long)npl * (a.ny / 2);
-  dim3 grid((unsigned)((jobs + kWavesPerBlock - 1) / kWavesPerBlock), nf);
-  size_t sh = (size_t)kWavesPerBlock * a.ls * sizeof(Cplx<T>);
   kt_begin(L, KT_ROWS_R2C);
-  if (mode == LOAD_PCLEAN)
-    hipLaunchKernelGGL((k_rows_r2c<TI, T, true>), grid, dim3(LES_BLOCK), sh, L.stream, a, L.px, twpool<T>(L));
-  else
-    hipLaunchKernelGGL((k_rows_r2c<TI, T>), grid, dim3(LES_BLOCK), sh, L.stream, a, L.px, twpool<T>(L));
+  rows_r2c_reg<TI, T>(false, L.nx, a, nf, twpool<T>(L) + L.px.twf, L.stream);
   const double in_fields = mode == LOAD_AB2_SCALE_DIV ? 3.0 : mode == LOAD_PCLEAN ? 4.0 : 1.0;
   kt_end(L, KT_ROWS_R2C, (double)nf * npl * a.ny * (in_fields * L.nx * sizeof(TI) + (double)L.lhx * sizeof(Cplx<T>)),
-         "k_rows_r2c", sizeof(TI), sizeof(T),
+         "k_rows_r2c_reg", sizeof(TI), sizeof(T),
          mode == LOAD_AB2_SCALE_DIV ? "AB2 predictor" : mode == LOAD_PCLEAN ? "cleaned pressure" : nullptr);
 }
 
@@ -205,14 +198,10 @@ static void rows_c2r(Les& L, const Cplx<T>* const* src, TO* const* dst, int nf, 
   RowC2RArgs<T, TO> a;
   for (int f = 0; f < nf; ++f) { a.src[f] = src[f]; a.dst[f] = dst[f]; }
   a.nx = L.nx; a.ny = L.ny; a.lhx = L.lhx; a.k0 = k0; a.nplanes = npl;
-  a.ls = row_line<T>(L.nx);
-  long jobs = (long)npl * (L.ny / 2);
-  dim3 grid((unsigned)((jobs + kWavesPerBlock - 1) / kWavesPerBlock), nf);
-  size_t sh = (size_t)kWavesPerBlock * a.ls * sizeof(Cplx<T>);
   kt_begin(L, KT_ROWS_C2R);
-  hipLaunchKernelGGL((k_rows_c2r<T, TO>), grid, dim3(LES_BLOCK), sh, L.stream, a, L.px, twpool<T>(L));
+  rows_c2r_reg<T, TO>(false, L.nx, a, nf, twpool<T>(L) + L.px.twf, L.stream);
   kt_end(L, KT_ROWS_C2R, (double)nf * npl * L.ny * ((double)L.lhx * sizeof(Cplx<T>) + (double)L.nx * sizeof(TO)),
-         "k_rows_c2r", sizeof(T), sizeof(TO));
+         "k_rows_c2r_reg", sizeof(T), sizeof(TO));
 }
 
 // The same column op on njobs (at most LES_COL_JOBS) independent sets of
@@ -925,25 +914,23 @@ static int les_step_t(Les& L) {
 }
 
 // ------------------------------------------------------------------ set-up
+// LDS limits of the kernels of this domain's lengths; nonzero: a length has no kernels
+template <typename T>
+static bool setup_fft_attrs(const Les& L) {
+  return cols_reg<T>(true, L.ny, 0, 0, 0, 0, ColArgs<T>(), 0, nullptr, 0) &&
+         colres_reg<T>(true, L.ny, true, ColResArgs<T>(), 0, nullptr, nullptr, 0) &&
+         rows_r2c_reg<double, T>(true, L.nx, RowR2CArgs<double, T>(), 0, nullptr, 0) &&
+         rows_c2r_reg<T, double>(true, L.nx, RowC2RArgs<T, double>(), 0, nullptr, 0) &&
+         rows_div_reg<T>(true, L.nx, RowC2RArgs<T, T>(), DivEpi3<T>(), 0, nullptr, 0) &&
+         rows_pad_reg<T>(true, L.nx, RowResArgs<T, T, T>(), 0, nullptr, nullptr, 0) &&
+         rows_trunc_reg<T>(true, L.nx, RowResArgs<T, T, double>(), 0, nullptr, nullptr, 0);
+}
 static int setup_kernel_attrs(const Les& L) {
-  const int big = 160 * 1024;
-  hipFuncSetAttribute((const void*)k_rows_r2c<double, double>, hipFuncAttributeMaxDynamicSharedMemorySize, big);
-  hipFuncSetAttribute((const void*)k_rows_r2c<double, float>, hipFuncAttributeMaxDynamicSharedMemorySize, big);
-  hipFuncSetAttribute((const void*)k_rows_r2c<float, float>, hipFuncAttributeMaxDynamicSharedMemorySize, big);
-  hipFuncSetAttribute((const void*)k_rows_c2r<double, double>, hipFuncAttributeMaxDynamicSharedMemorySize, big);
-  hipFuncSetAttribute((const void*)k_rows_c2r<float, float>, hipFuncAttributeMaxDynamicSharedMemorySize, big);
-  hipFuncSetAttribute((const void*)k_rows_c2r<float, double>, hipFuncAttributeMaxDynamicSharedMemorySize, big);
-  if (!cols_reg<double>(true, L.ny, 0, 0, 0, 0, ColArgs<double>(), 0, nullptr, 0) ||
-      !cols_reg<float>(true, L.ny, 0, 0, 0, 0, ColArgs<float>(), 0, nullptr, 0))
-    return 10;
-  hipFuncSetAttribute((const void*)k_rows_resample<double, double, double>, hipFuncAttributeMaxDynamicSharedMemorySize, big);
-  hipFuncSetAttribute((const void*)k_rows_resample<float, double, float>, hipFuncAttributeMaxDynamicSharedMemorySize, big);
-  hipFuncSetAttribute((const void*)k_rows_resample<float, float, float>, hipFuncAttributeMaxDynamicSharedMemorySize, big);
-  hipFuncSetAttribute((const void*)k_rows_resample<float, double, double>, hipFuncAttributeMaxDynamicSharedMemorySize, big);
-  if (!colres_reg<double>(true, L.ny, true, ColResArgs<double>(), 0, nullptr, nullptr, 0) ||
-      !colres_reg<float>(true, L.ny, true, ColResArgs<float>(), 0, nullptr, nullptr, 0))
-    return 10;
-  return 0;
+  const bool ok = setup_fft_attrs<double>(L) && setup_fft_attrs<float>(L) &&
+                  rows_r2c_reg<float, float>(true, L.nx, RowR2CArgs<float, float>(), 0, nullptr, 0) &&
+                  rows_c2r_reg<float, float>(true, L.nx, RowC2RArgs<float, float>(), 0, nullptr, 0) &&
+                  rows_proj_reg<double>(true, L.nx, RowC2RArgs<double, double>(), ProjEpi3(), 0, nullptr, 0);
+  return ok ? 0 : 10;
 }
 
 static void free_all(Les* L) {
@@ -1195,7 +1182,7 @@ int les_init(const les_params* p) {
   L->dg_out = (double*)dalloc(*L, sizeof(double) * 4);
   if (L->alloc_failed) { les_finalize(); les_set_error("out of memory (workspaces)"); return 3; }
   for (int i = 0; i < 64; ++i) if (!L->wk_real[i]) { les_finalize(); les_set_error("out of memory"); return 3; }
-  if (setup_kernel_attrs(*L)) { les_set_error("no column kernels for ny = %d", ny); les_finalize(); return 10; }
+  if (setup_kernel_attrs(*L)) { les_set_error("no transform kernels for %d x %d", nx, ny); les_finalize(); return 10; }
   if (hipDeviceSynchronize() != hipSuccess) { les_set_error("init sync failed"); les_finalize(); return 5; }
   return 0;
 }

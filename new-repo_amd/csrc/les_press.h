@@ -290,70 +290,6 @@ __global__ void k_proj(ProjArgs a) {
   }
 }
 
-// ---- the step's projection, fused with the pressure-gradient transforms.
-// The x and y components are projected as the store of the inverse x
-// transform of i kx phat and i ky phat (blockIdx.y 0 and 1); blockIdx.y 2
-// stores p.  The gradient then never goes through HBM: dpdx, dpdy and dpdz
-// are formed again from phat and p only when the host asks for them
-// (refresh_gradp).  The arithmetic per value is k_proj's.
-struct ProjEpiArgs {
-  double *vel, *r;          // u or v, rhsx or rhsy (null for the p component)
-  const double *rf, *lbc;   // rhs_f, lbc_u or lbc_v
-  double* p;                // p (component 2)
-  int neu;                  // top BC Neumann
-  double ubc;
-};
-struct ProjEpi3 {
-  ProjEpiArgs c[3];
-  double dt, t1, t2, dtt, dz;
-  long np;
-  int nz;
-};
-
-__device__ __forceinline__ void proj_epi_point(const ProjEpi3& e, const ProjEpiArgs& a, int k, long q, double g) {
-  const long c = (long)k * e.np + q;
-  if (a.p) {
-    a.p[c] = g;
-    return;
-  }
-  if (k < 1 || k > e.nz) return;
-  const double rc = a.r[c];
-  double us = a.vel[c];
-  us = us + e.dt * (e.t1 * rc + e.t2 * a.rf[c]);
-  const double un = us - e.dtt * g;
-  a.r[c] = rc - g;
-  a.vel[c] = un;
-  if (k == 1) a.vel[q] = un - a.lbc[q] * e.dz;
-  if (k == e.nz) a.vel[c + e.np] = a.neu ? un + a.ubc * e.dz : 2.0 * a.ubc - un;
-}
-
-__global__ void __launch_bounds__(LES_BLOCK) k_rows_c2r_proj(RowC2RArgs<double, double> a, ProjEpi3 ep, FftPlan pl,
-                                                             const Cplx<double>* __restrict__ tw) {
-  const ProjEpiArgs& e = ep.c[blockIdx.y];
-  extern __shared__ __align__(16) unsigned char smem_raw[];
-  const int lane = threadIdx.x & (LES_WAVE - 1), wave = threadIdx.x / LES_WAVE;
-  Cplx<double>* z = reinterpret_cast<Cplx<double>*>(smem_raw) + wave * a.ls;
-  const long job = (long)blockIdx.x * (blockDim.x / LES_WAVE) + wave;
-  const int npairs = a.ny / 2;
-  if (job >= (long)a.nplanes * npairs) return;
-  const int k = a.k0 + (int)(job / npairs), jp = (int)(job % npairs);
-  if (pl.n == 256) {
-    TwReg<double, 256> tr;
-    tw_load(tr, tw + pl.twf, lane);
-    rows_c2r_line(a, z, lane, k, jp, [&](Cplx<double>* p, bool inv) {
-      wave_fft_t<double, 256, row_layout<double>(256)>(p, tr, inv, lane);
-    });
-  } else {
-    rows_c2r_line(a, z, lane, k, jp, [&](Cplx<double>* p, bool inv) { wave_fft(p, pl, tw, inv, lane); });
-  }
-  const long q0 = (long)(2 * jp) * a.nx;
-  for (int n = lane; n < a.nx; n += LES_WAVE) {
-    const Cplx<double> v = z[n];
-    proj_epi_point(ep, e, k, q0 + n, v.x);
-    proj_epi_point(ep, e, k, q0 + a.nx + n, v.y);
-  }
-}
-
 // w: dpdz from p, projection, rhsz -= dpdz, the w BCs and p(nz+1) = BOGUS
 // (k_proj's arithmetic for the vertical component)
 struct ProjWArgs {
@@ -395,7 +331,6 @@ static void press_project(Les& L, double tadv1, double tadv2) {
   RowC2RArgs<double, double> ca;
   for (int f = 0; f < 3; ++f) { ca.src[f] = (const Cplx<double>*)L.pspec[f]; ca.dst[f] = nullptr; }
   ca.nx = L.nx; ca.ny = L.ny; ca.lhx = L.lhx; ca.k0 = 0; ca.nplanes = nz + 2;
-  ca.ls = row_line<double>(L.nx);
   ProjEpi3 ep;
   ep.dt = L.P.dt; ep.t1 = tadv1; ep.t2 = tadv2; ep.dtt = L.P.dt * tadv1; ep.dz = L.dz;
   ep.np = L.np; ep.nz = nz;
@@ -408,14 +343,11 @@ static void press_project(Les& L, double tadv1, double tadv2) {
     ep.c[f].ubc = f == 0 ? L.P.ubc_u : L.P.ubc_v;
   }
   ep.c[2] = ProjEpiArgs{nullptr, nullptr, nullptr, nullptr, D(L, LES_P), 0, 0.0};
-  const long jobs = (long)ca.nplanes * (L.ny / 2);
-  const size_t sh = (size_t)kWavesPerBlock * ca.ls * sizeof(Cplx<double>);
   kt_begin(L, KT_ROWS_C2R);
-  hipLaunchKernelGGL(k_rows_c2r_proj, dim3((unsigned)((jobs + kWavesPerBlock - 1) / kWavesPerBlock), 3),
-                     dim3(LES_BLOCK), sh, L.stream, ca, ep, L.px, twpool<double>(L));
+  rows_proj_reg<double>(false, L.nx, ca, ep, 3, twpool<double>(L) + L.px.twf, L.stream);
   // spectra in; p out; u, v, rhs, rhs_f in and u, v, rhs out on levels 1..nz
   kt_end(L, KT_ROWS_C2R, 3.0 * (nz + 2) * L.ny * ((double)L.lhx * 16) + 8.0 * L.np * (nz + 2) + 2.0 * 8 * L.np * nz * 5,
-         "k_rows_c2r_proj");
+         "k_rows_c2r_proj_reg");
   ProjWArgs w;
   w.w = D(L, LES_W); w.rz = D(L, LES_RHSZ); w.p = D(L, LES_P); w.fz = D(L, LES_RHSZ_F);
   w.dt = L.P.dt; w.t1 = tadv1; w.t2 = tadv2; w.dtt = L.P.dt * tadv1; w.cz = 1.0 / L.dz;

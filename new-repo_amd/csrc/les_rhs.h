@@ -182,18 +182,12 @@ static void convection(Les& L, double* cx, double* cy, double* cz) {
     a.cs.dvdx = F<T>(L, LES_DVDX); a.cs.dvdz = F<T>(L, LES_DVDZ);
     a.cs.dwdx = F<T>(L, LES_DWDX); a.cs.dwdy = F<T>(L, LES_DWDY);
     a.cconv = c;
-    a.src_mode = 1;
     for (int f = 0; f < 6; ++f) { a.src[f] = nullptr; a.dst[f] = (T*)L.wk_hyb[f]; }
-    a.n1 = nx; a.n2 = nx2; a.ny = ny; a.k0 = 1; a.nplanes = nz + 1;
-    a.src_plane = (long)nx * ny; a.dst_plane = (long)nx2 * ny;
-    a.ls = res_line<T>(nx, nx2);
-    long jobs = (long)a.nplanes * (ny / 2);
-    size_t sh = (size_t)kWavesPerBlock * a.ls * sizeof(Cplx<T>);
+    a.ny = ny; a.k0 = 1; a.nplanes = nz + 1;
     kt_begin(L, KT_ROWS_RES);
-    hipLaunchKernelGGL((k_rows_resample<T, T, T>), dim3((unsigned)((jobs + kWavesPerBlock - 1) / kWavesPerBlock), 6),
-                       dim3(LES_BLOCK), sh, L.stream, a, L.px, L.px2, twpool<T>(L));
+    rows_pad_reg<T>(false, nx, a, 6, twpool<T>(L) + L.px.twf, twpool<T>(L) + L.px2.twf, L.stream);
     kt_end(L, KT_ROWS_RES, (double)a.nplanes * L.np * (3.0 * 8 + 6.0 * sizeof(T)) + 6.0 * a.nplanes * nx2 * ny * sizeof(T),
-           "k_rows_resample", sizeof(T), sizeof(T), "pad");
+           "k_rows_resample_reg", sizeof(T), sizeof(T), "pad");
   }
   // pad in y
   {
@@ -232,17 +226,10 @@ static void convection(Les& L, double* cx, double* cy, double* cz) {
     RowResArgs<T, T, double> a;
     a.src[0] = (const T*)L.wk_hyb3[0]; a.src[1] = (const T*)L.wk_hyb3[1]; a.src[2] = (const T*)L.wk_hyb3[2];
     a.dst[0] = cx; a.dst[1] = cy; a.dst[2] = cz;
-    a.cconv = (T)0;
-    a.src_mode = 0;
-    a.n1 = nx2; a.n2 = nx; a.ny = ny; a.k0 = 1; a.nplanes = nz;
-    a.src_plane = (long)nx2 * ny; a.dst_plane = L.np;
-    a.ls = res_line<T>(nx2, nx);
-    long jobs = (long)nz * (ny / 2);
-    size_t sh = (size_t)kWavesPerBlock * a.ls * sizeof(Cplx<T>);
+    a.ny = ny; a.k0 = 1; a.nplanes = nz;
     kt_begin(L, KT_ROWS_RES);
-    hipLaunchKernelGGL((k_rows_resample<T, T, double>), dim3((unsigned)((jobs + kWavesPerBlock - 1) / kWavesPerBlock), 3),
-                       dim3(LES_BLOCK), sh, L.stream, a, L.px2, L.px, twpool<T>(L));
-    kt_end(L, KT_ROWS_RES, 3.0 * nz * ny * ((double)nx2 * sizeof(T) + (double)nx * 8), "k_rows_resample", sizeof(T),
+    rows_trunc_reg<T>(false, nx, a, 3, twpool<T>(L) + L.px.twf, twpool<T>(L) + L.px2.twf, L.stream);
+    kt_end(L, KT_ROWS_RES, 3.0 * nz * ny * ((double)nx2 * sizeof(T) + (double)nx * 8), "k_rows_resample_reg", sizeof(T),
            sizeof(T), "truncate");
   }
   SetPlaneArgs sp;
@@ -250,80 +237,6 @@ static void convection(Les& L, double* cx, double* cy, double* cz) {
   kt_begin(L, KT_POINTWISE);
   hipLaunchKernelGGL(k_set_planes, dim3(nblk(L.np)), dim3(LES_BLOCK), 0, L.stream, sp);
   kt_end(L, KT_POINTWISE, 6.0 * 8 * L.np, "k_set_planes");
-}
-
-// rhs(k) += d/dx tx + d/dy ty + d/dz tz for k = 1..nz, plus the forcing of
-// compute_RHS_adv; optionally the pressure BC layers
-// (src/compute_derivatives.f90:545-574; src/LES_engine.f90:547-562).
-template <typename T>
-struct DivEpiArgs {
-  double* rhs;
-  const T* tz;
-  int stag, save_wk;
-  double *bottom_wk, *top_wk;
-  double cz;
-  long np;
-  int nz;
-  int forcing;  // 1: x forcing, 2: y forcing
-  double pf, coriol, geo;
-  const double* vel;  // v for x, u for y (Coriolis)
-  int coriolis;
-};
-
-// rhs(k) += (horizontal divergence) + dz(tz) + forcing, applied as the store
-// of the inverse x transform of the divergence spectrum, so the divergence
-// never goes through HBM; levels 1..nz+1 (nz+1 only for top_wk).
-template <typename T>
-__device__ __forceinline__ void div_epi_point(const DivEpiArgs<T>& a, int k, long q, double dh) {
-  const long c = (long)k * a.np + q;
-  if (k <= a.nz) {
-    const double dzt = a.stag ? a.cz * ((double)a.tz[c + a.np] - (double)a.tz[c])
-                              : a.cz * ((double)a.tz[c] - (double)a.tz[c - a.np]);
-    double r = a.rhs[c] + dh + dzt;
-    if (a.forcing == 1) {
-      r = r + a.pf;
-      if (a.coriolis) r = r + a.coriol * a.vel[c] - a.coriol * a.geo;
-    } else if (a.forcing == 2) {
-      r = r + a.pf;
-      if (a.coriolis) r = r - a.coriol * a.vel[c] + a.coriol * a.geo;
-    }
-    a.rhs[c] = r;
-    if (a.save_wk && k == 1) a.bottom_wk[q] = dh + a.cz * ((double)a.tz[c] - (double)a.tz[q]);
-  } else if (a.save_wk) {
-    a.top_wk[q] = dh;
-  }
-}
-
-template <typename T>
-struct DivEpi3 {
-  DivEpiArgs<T> c[3];  // per component (blockIdx.y)
-};
-
-// FP32: held to 80 VGPRs (6 waves per SIMD instead of 5, no spills).
-template <typename T>
-__global__ void __launch_bounds__(LES_BLOCK) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? 6 : 1)))
-k_rows_c2r_div(RowC2RArgs<T, T> a, DivEpi3<T> ep, FftPlan pl, const Cplx<T>* __restrict__ tw) {
-  const DivEpiArgs<T>& e = ep.c[blockIdx.y];
-  extern __shared__ __align__(16) unsigned char smem_raw[];
-  const int lane = threadIdx.x & (LES_WAVE - 1), wave = threadIdx.x / LES_WAVE;
-  Cplx<T>* z = reinterpret_cast<Cplx<T>*>(smem_raw) + wave * a.ls;
-  const long job = (long)blockIdx.x * (blockDim.x / LES_WAVE) + wave;
-  const int npairs = a.ny / 2;
-  if (job >= (long)a.nplanes * npairs) return;
-  const int k = a.k0 + (int)(job / npairs), jp = (int)(job % npairs);
-  if (pl.n == 256) {
-    TwReg<T, 256> tr;
-    tw_load(tr, tw + pl.twf, lane);
-    rows_c2r_line(a, z, lane, k, jp, [&](Cplx<T>* p, bool inv) { wave_fft_t<T, 256, row_layout<T>(256)>(p, tr, inv, lane); });
-  } else {
-    rows_c2r_line(a, z, lane, k, jp, [&](Cplx<T>* p, bool inv) { wave_fft(p, pl, tw, inv, lane); });
-  }
-  const long q0 = (long)(2 * jp) * a.nx;
-  for (int n = lane; n < a.nx; n += LES_WAVE) {
-    const Cplx<T> v = z[n];
-    div_epi_point(e, k, q0 + n, (double)v.x);
-    div_epi_point(e, k, q0 + a.nx + n, (double)v.y);
-  }
 }
 
 template <typename T>
@@ -349,17 +262,13 @@ static void rows_c2r_div(Les& L, const Cplx<T>* const* src, const DivEpi3<T>& ep
   RowC2RArgs<T, T> ca;
   for (int f = 0; f < nf; ++f) { ca.src[f] = src[f]; ca.dst[f] = nullptr; }
   ca.nx = L.nx; ca.ny = L.ny; ca.lhx = L.lhx; ca.k0 = 1; ca.nplanes = L.nz + 1;
-  ca.ls = row_line<T>(L.nx);
-  const long jobs = (long)ca.nplanes * (L.ny / 2);
-  const size_t sh = (size_t)kWavesPerBlock * ca.ls * sizeof(Cplx<T>);
   double extra = 0.0;
   for (int f = 0; f < nf; ++f) extra += (ep.c[f].coriolis && ep.c[f].forcing) ? 8.0 : 0.0;
   kt_begin(L, KT_ROWS_C2R);
-  hipLaunchKernelGGL((k_rows_c2r_div<T>), dim3((unsigned)((jobs + kWavesPerBlock - 1) / kWavesPerBlock), nf),
-                     dim3(LES_BLOCK), sh, L.stream, ca, ep, L.px, twpool<T>(L));
+  rows_div_reg<T>(false, L.nx, ca, ep, nf, twpool<T>(L) + L.px.twf, L.stream);
   kt_end(L, KT_ROWS_C2R, (double)nf * (L.nz + 1) * L.ny * ((double)L.lhx * sizeof(Cplx<T>)) +
                              (double)L.np * L.nz * (nf * (16.0 + sizeof(T)) + extra),
-         "k_rows_c2r_div", sizeof(T));
+         "k_rows_c2r_div_reg", sizeof(T));
 }
 
 template <typename T>
