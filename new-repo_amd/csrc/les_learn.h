@@ -22,8 +22,9 @@ struct MlpState {
   int ready;
   // training buffers
   long cap;
-  short *h1, *h2, *h3, *dy, *dz;
-  float *z1, *z2, *z3, *c, *dh, *dyf, *dzf, *part, *lossp;
+  short *h1, *h2, *h3, *dy, *dz[2];
+  float *z1, *z2, *z3, *c, *dzf, *dyf, *part, *lossp;
+  float* csum;     // column sums: 256 per column, of the output layer and the three hidden ones
 };
 
 static void* dalloc(Les& L, size_t bytes);
@@ -57,57 +58,57 @@ static int mlp_train_alloc(Les& L, long n) {
   if (n <= M->cap) return 0;
   const long c = n;
   M->h1 = (short*)dalloc(L, 2 * 64 * c); M->h2 = (short*)dalloc(L, 2 * 64 * c); M->h3 = (short*)dalloc(L, 2 * 64 * c);
-  M->dy = (short*)dalloc(L, 2 * 16 * c); M->dz = (short*)dalloc(L, 2 * 64 * c);
+  M->dy = (short*)dalloc(L, 2 * 16 * c); M->dz[0] = (short*)dalloc(L, 2 * 64 * c); M->dz[1] = (short*)dalloc(L, 2 * 64 * c);
   M->z1 = (float*)dalloc(L, 4 * 64 * c); M->z2 = (float*)dalloc(L, 4 * 64 * c); M->z3 = (float*)dalloc(L, 4 * 64 * c);
-  M->c = (float*)dalloc(L, 4 * 64 * c); M->dh = (float*)dalloc(L, 4 * 64 * c);
-  M->dyf = (float*)dalloc(L, 4 * 16 * c); M->dzf = (float*)dalloc(L, 4 * 64 * c);
-  M->part = (float*)dalloc(L, 4 * (size_t)(c / MLP_KCHUNK + 2) * 64 * 64);
+  M->c = (float*)dalloc(L, 4 * 16 * c); M->dzf = (float*)dalloc(L, 4 * 64 * c);
+  M->dyf = (float*)dalloc(L, 4 * 16 * c);
+  M->part = (float*)dalloc(L, 4 * (size_t)(c / MLP_KCHUNK + 2) * MLP_NMAT);
+  M->csum = (float*)dalloc(L, 4 * (size_t)MLP_SUMS * (16 + 3 * 64));
   M->lossp = (float*)dalloc(L, 4 * (size_t)(16 * c / 256 + 2));
   M->cap = c;
   if (L.alloc_failed) { les_set_error("out of memory (MLP training)"); return 3; }
   return 0;
 }
 
-// C[M x N] = A[M x K] B[K x N]: the weight gradients (K the batch) as
-// per-wavefront K chunks summed afterwards, the activation products as
-// 16-row strips; shapes outside those (not used by training) on the
-// one-tile kernel.
-static void gemm(Les& L, const short* A, long sam, long sak, const short* B, long sbk, long sbn, float* C, int M, int N,
-                 int K) {
+// C[M x N] = A[M x K] B[K x N], K at most 64 or the batch (MLP layers only):
+// 16-row strips over every output column tile; mode and h: what is stored
+// (k_gemm_strip).
+static void gemm(Les& L, const short* A, long sam, long sak, const short* B, long sbk, long sbn, float* C, int M, int N, int K,
+                 int mode = STRIP_C, const StripOut& h = StripOut()) {
   GemmArgs g;
   g.A = A; g.sam = sam; g.sak = sak; g.B = B; g.sbk = sbk; g.sbn = sbn;
   g.C = C;
   g.M = M; g.N = N; g.K = K; g.kchunk = K;
-  const int mt = M / 16, nt = N / 16;
-  if (K > 1024 && (mt == 1 || mt == 4) && (nt == 1 || nt == 4)) {
-    g.kchunk = MLP_KCHUNK;
-    g.C = L.mlp->part;
-    const int nsplit = (K + MLP_KCHUNK - 1) / MLP_KCHUNK;
-    const dim3 grid((unsigned)((nsplit + 3) / 4));
-    if (mt == 4 && nt == 4) hipLaunchKernelGGL((k_gemm_kchunk<4, 4>), grid, dim3(256), 0, L.stream, g);
-    else if (mt == 4) hipLaunchKernelGGL((k_gemm_kchunk<4, 1>), grid, dim3(256), 0, L.stream, g);
-    else if (nt == 4) hipLaunchKernelGGL((k_gemm_kchunk<1, 4>), grid, dim3(256), 0, L.stream, g);
-    else hipLaunchKernelGGL((k_gemm_kchunk<1, 1>), grid, dim3(256), 0, L.stream, g);
-    const long n = (long)M * N;
-    hipLaunchKernelGGL(k_sum_splits, dim3(nblk(n)), dim3(LES_BLOCK), 0, L.stream, L.mlp->part, C, n, nsplit, 0);
-  } else if (K <= 1024 && (nt == 1 || nt == 4)) {
-    const dim3 grid((unsigned)((mt + 3) / 4));
-    if (nt == 4) hipLaunchKernelGGL((k_gemm_strip<4>), grid, dim3(256), 0, L.stream, g);
-    else hipLaunchKernelGGL((k_gemm_strip<1>), grid, dim3(256), 0, L.stream, g);
-  } else {
-    int kchunk = K, nsplit = 1;
-    if (K > 1024) {
-      kchunk = 512;
-      nsplit = (K + kchunk - 1) / kchunk;
-    }
-    g.kchunk = kchunk;
-    g.C = nsplit > 1 ? L.mlp->part : C;
-    hipLaunchKernelGGL(k_gemm_bf16, dim3((M / 16) * (N / 16), nsplit), dim3(64), 0, L.stream, g);
-    if (nsplit > 1) {
-      const long n = (long)M * N;
-      hipLaunchKernelGGL(k_sum_splits, dim3(nblk(n)), dim3(LES_BLOCK), 0, L.stream, L.mlp->part, C, n, nsplit, 0);
-    }
+  assert(N == 64 || (N == 16 && mode == STRIP_C));
+  const dim3 grid((unsigned)((M / 16 + 3) / 4));
+  if (mode == STRIP_HIDDEN) hipLaunchKernelGGL((k_gemm_strip<4, STRIP_HIDDEN>), grid, dim3(256), 0, L.stream, g, h);
+  else if (mode == STRIP_BACK) hipLaunchKernelGGL((k_gemm_strip<4, STRIP_BACK>), grid, dim3(256), 0, L.stream, g, h);
+  else if (N == 64) hipLaunchKernelGGL((k_gemm_strip<4, STRIP_C>), grid, dim3(256), 0, L.stream, g, h);
+  else hipLaunchKernelGGL((k_gemm_strip<1, STRIP_C>), grid, dim3(256), 0, L.stream, g, h);
+}
+
+// The weight gradients C[M x N] = A[M x K] B[K x N], K the batch, M and N 16
+// or 64: beyond 1024 rows per-wavefront K chunks into slabs of the training
+// workspace (offset off matrix values in each slab set), added to the sums sp
+// that one launch of k_sum_splits forms after the last matrix.
+static void gemm_wgrad(Les& L, const short* A, long sam, const short* B, long sbk, float* C, int M, int N, int K, SumSplits& sp,
+                       int& nm, long& off) {
+  if (K <= 1024) {
+    gemm(L, A, 1, sam, B, sbk, 1, C, M, N, K);
+    return;
   }
+  GemmArgs g;
+  g.A = A; g.sam = 1; g.sak = sam; g.B = B; g.sbk = sbk; g.sbn = 1;
+  g.M = M; g.N = N; g.K = K; g.kchunk = MLP_KCHUNK;
+  const int nsplit = (K + MLP_KCHUNK - 1) / MLP_KCHUNK;
+  g.C = L.mlp->part + off * nsplit;
+  const dim3 grid((unsigned)((nsplit + 3) / 4));
+  if (M == 64 && N == 64) hipLaunchKernelGGL((k_gemm_kchunk<4, 4>), grid, dim3(256), 0, L.stream, g);
+  else if (M == 64) hipLaunchKernelGGL((k_gemm_kchunk<4, 1>), grid, dim3(256), 0, L.stream, g);
+  else hipLaunchKernelGGL((k_gemm_kchunk<1, 4>), grid, dim3(256), 0, L.stream, g);
+  sp.part[nm] = g.C; sp.out[nm] = C; sp.n[nm] = M * N; sp.nsplit = nsplit;
+  ++nm;
+  off += (long)M * N;
 }
 
 // forward + backward over a batch of n points (n multiple of 16); fills
@@ -119,33 +120,44 @@ static int mlp_forward_backward(Les& L, const short* X, const float* Y, long n, 
   if (rc) return rc;
   const int N = (int)n;
   const float* b = M->w + MLP_NMAT;
-  const long n64 = n * 64;
   // forward
-  gemm(L, X, 16, 1, M->wb + MW1, 1, 16, M->c, N, 64, 16);
-  hipLaunchKernelGGL(k_bias_gelu, dim3(nblk(n64)), dim3(LES_BLOCK), 0, L.stream, M->c, b + MB1, M->z1, M->h1, n);
-  gemm(L, M->h1, 64, 1, M->wb + MW2, 1, 64, M->c, N, 64, 64);
-  hipLaunchKernelGGL(k_bias_gelu, dim3(nblk(n64)), dim3(LES_BLOCK), 0, L.stream, M->c, b + MB2, M->z2, M->h2, n);
-  gemm(L, M->h2, 64, 1, M->wb + MW3, 1, 64, M->c, N, 64, 64);
-  hipLaunchKernelGGL(k_bias_gelu, dim3(nblk(n64)), dim3(LES_BLOCK), 0, L.stream, M->c, b + MB3, M->z3, M->h3, n);
+  gemm(L, X, 16, 1, M->wb + MW1, 1, 16, nullptr, N, 64, 16, STRIP_HIDDEN, {b + MB1, M->z1, M->h1});
+  gemm(L, M->h1, 64, 1, M->wb + MW2, 1, 64, nullptr, N, 64, 64, STRIP_HIDDEN, {b + MB2, M->z2, M->h2});
+  gemm(L, M->h2, 64, 1, M->wb + MW3, 1, 64, nullptr, N, 64, 64, STRIP_HIDDEN, {b + MB3, M->z3, M->h3});
   gemm(L, M->h3, 64, 1, M->wb + MW4, 1, 64, M->c, N, 16, 64);
   const unsigned nb16 = nblk(n * 16);
   hipLaunchKernelGGL(k_out_grad, dim3(nb16), dim3(LES_BLOCK), 0, L.stream, M->c, b + MB4, Y, M->dy, M->dyf, M->lossp, n);
   // backward
   float* g = M->g;
-  gemm(L, M->dy, 1, 16, M->h3, 64, 1, g + MW4, 16, 64, N);
-  hipLaunchKernelGGL(k_colsum, dim3(16), dim3(LES_BLOCK), 0, L.stream, M->dyf, g + MLP_NMAT + MB4, n, 16);
-  gemm(L, M->dy, 16, 1, M->wb + MW4, 64, 1, M->dh, N, 64, 16);
+  SumSplits sp = {};
+  ColTree ct = {};
+  int nm = 0;
+  long off = 0;
+  gemm_wgrad(L, M->dy, 16, M->h3, 64, g + MW4, 16, 64, N, sp, nm, off);
+  float* cs = M->csum;
+  hipLaunchKernelGGL(k_colsum_part<16>, dim3(MLP_SUMS * 16 / 64), dim3(64), 0, L.stream, (const float*)M->dyf, cs, n);
+  ct.part[0] = cs; ct.out[0] = g + MLP_NMAT + MB4; ct.w[0] = 16;
+  cs += MLP_SUMS * 16;
+  short* dz = M->dz[0];
+  short* dn = M->dz[1];
+  gemm(L, M->dy, 16, 1, M->wb + MW4, 64, 1, nullptr, N, 64, 16, STRIP_BACK, {M->z3, M->dzf, dz});
   const short* hin[3] = {X, M->h1, M->h2};
-  const float* zs[3] = {M->z1, M->z2, M->z3};
+  const float* zs[2] = {M->z1, M->z2};
   const int mw[3] = {MW1, MW2, MW3};
   const int mb[3] = {MB1, MB2, MB3};
   const int kin[3] = {16, 64, 64};
   for (int layer = 2; layer >= 0; --layer) {
-    hipLaunchKernelGGL(k_gelu_back, dim3(nblk(n64)), dim3(LES_BLOCK), 0, L.stream, M->dh, zs[layer], M->dz, M->dzf, n);
-    hipLaunchKernelGGL(k_colsum, dim3(64), dim3(LES_BLOCK), 0, L.stream, M->dzf, g + MLP_NMAT + mb[layer], n, 64);
-    gemm(L, M->dz, 1, 64, hin[layer], kin[layer], 1, g + mw[layer], 64, kin[layer], N);
-    if (layer > 0) gemm(L, M->dz, 64, 1, M->wb + mw[layer], kin[layer], 1, M->dh, N, kin[layer], 64);
+    hipLaunchKernelGGL(k_colsum_part<64>, dim3(MLP_SUMS), dim3(64), 0, L.stream, (const float*)M->dzf, cs, n);
+    ct.part[3 - layer] = cs; ct.out[3 - layer] = g + MLP_NMAT + mb[layer]; ct.w[3 - layer] = 64;
+    cs += MLP_SUMS * 64;
+    gemm_wgrad(L, dz, 64, hin[layer], kin[layer], g + mw[layer], 64, kin[layer], N, sp, nm, off);
+    if (layer > 0) {
+      gemm(L, dz, 64, 1, M->wb + mw[layer], kin[layer], 1, nullptr, N, kin[layer], 64, STRIP_BACK, {zs[layer - 1], M->dzf, dn});
+      std::swap(dz, dn);
+    }
   }
+  if (nm > 0) hipLaunchKernelGGL(k_sum_splits, dim3(MLP_NMAT / 16), dim3(256), 0, L.stream, sp);
+  hipLaunchKernelGGL(k_colsum_tree, dim3(16 + 3 * 64), dim3(256), 0, L.stream, ct);
   if (loss) {
     std::vector<float> lp(nb16);
     LES_CHECK(hipMemcpyAsync(lp.data(), M->lossp, 4 * nb16, hipMemcpyDeviceToHost, L.stream));

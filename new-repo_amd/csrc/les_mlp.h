@@ -84,9 +84,7 @@ __device__ __forceinline__ float gelu_d(float x) {
 
 // ------------------------------------------------------------------ GEMM
 // C[M x N] (fp32) = A[M x K] * B[K x N], bf16 operands with arbitrary
-// strides (so transposes are stride swaps), one 16x16 tile per wave,
-// split-K over blockIdx.y into partial slabs C + split * M * N.
-// M, N, K are multiples of 16.  Lane layout of v_mfma_f32_16x16x16_bf16:
+// strides (so transposes are stride swaps).  M, N, K are multiples of 16.  Lane layout of v_mfma_f32_16x16x16_bf16:
 // A[m = l%16][k = 4(l/16) + j], B[k = 4(l/16) + j][n = l%16],
 // D[m = 4(l/16) + j][n = l%16], j = 0..3.
 struct GemmArgs {
@@ -97,27 +95,6 @@ struct GemmArgs {
   float* C;
   int M, N, K, kchunk;
 };
-
-__global__ void __launch_bounds__(64) k_gemm_bf16(GemmArgs g) {
-  const int l = threadIdx.x;
-  const int tn = g.N / 16;
-  const int m0 = (blockIdx.x / tn) * 16, n0 = (blockIdx.x % tn) * 16;
-  const int k0 = blockIdx.y * g.kchunk;
-  int k1 = k0 + g.kchunk;
-  if (k1 > g.K) k1 = g.K;
-  f4v acc = {0.f, 0.f, 0.f, 0.f};
-  const int r = l & 15, q = (l >> 4) * 4;
-  for (int k = k0; k < k1; k += 16) {
-    s4v a, b;
-    for (int j = 0; j < 4; ++j) {
-      a[j] = g.A[(long)(m0 + r) * g.sam + (long)(k + q + j) * g.sak];
-      b[j] = g.B[(long)(k + q + j) * g.sbk + (long)(n0 + r) * g.sbn];
-    }
-    acc = mfma16(a, b, acc);
-  }
-  float* C = g.C + (long)blockIdx.y * g.M * g.N;
-  for (int j = 0; j < 4; ++j) C[(long)(m0 + q + j) * g.N + n0 + r] = acc[j];
-}
 
 // Four consecutive-in-k bf16 operand values: one 8-byte load where they are
 // adjacent and aligned, else four 2-byte loads.
@@ -132,9 +109,17 @@ __device__ __forceinline__ s4v load4(const short* p, long stride) {
 // The training GEMMs with few columns and short K (activations times a
 // weight matrix): each wavefront computes a 16-row strip and all NT 16-wide
 // column tiles, reusing its A fragment across them; four wavefronts per
-// block.  Same lane layout as k_gemm_bf16.
-template <int NT>
-__global__ void __launch_bounds__(256) k_gemm_strip(GemmArgs g) {
+// block.  What is stored instead of C (C is then not written and read again):
+// STRIP_HIDDEN a hidden layer, Z = C + bias in fp32 and H = gelu(Z) in bf16;
+// STRIP_BACK its gradient, Zf = C gelu'(Z) in fp32 and H the same in bf16.
+enum { STRIP_C = 0, STRIP_HIDDEN = 1, STRIP_BACK = 2 };
+struct StripOut {
+  const float* in;  // bias (hidden), Z (back)
+  float* Zf;
+  short* H;
+};
+template <int NT, int MODE>
+__global__ void __launch_bounds__(256) k_gemm_strip(GemmArgs g, StripOut h) {
   const int l = threadIdx.x & 63;
   const long m0 = ((long)blockIdx.x * 4 + (threadIdx.x >> 6)) * 16;
   if (m0 >= g.M) return;
@@ -151,7 +136,20 @@ __global__ void __launch_bounds__(256) k_gemm_strip(GemmArgs g) {
 #pragma unroll
   for (int t = 0; t < NT; ++t)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) g.C[(m0 + q + j) * g.N + 16 * t + r] = acc[t][j];
+    for (int j = 0; j < 4; ++j) {
+      const long o = (m0 + q + j) * g.N + 16 * t + r;
+      if constexpr (MODE == STRIP_HIDDEN) {
+        const float z = acc[t][j] + h.in[16 * t + r];
+        h.Zf[o] = z;
+        h.H[o] = f2bf(gelu(z));
+      } else if constexpr (MODE == STRIP_BACK) {
+        const float d = acc[t][j] * gelu_d(h.in[o]);
+        h.Zf[o] = d;
+        h.H[o] = f2bf(d);
+      } else {
+        g.C[o] = acc[t][j];
+      }
+    }
 }
 
 // The weight-gradient GEMMs (M, N <= 64, K = the batch): wavefront w sums
@@ -190,21 +188,43 @@ __global__ void __launch_bounds__(256) k_gemm_kchunk(GemmArgs g) {
       for (int j = 0; j < 4; ++j) C[(long)(16 * i + q + j) * g.N + 16 * t + r] = acc[i][t][j];
 }
 
-__global__ void k_sum_splits(const float* part, float* out, long n, int nsplit, int accumulate) {
-  const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= n) return;
+// Sums of the slabs of up to four matrices, out = part[0] + part[1] + ... in
+// order, each output one running fp32 sum.  A block sums 16 outputs: its 256
+// threads stage 256 slabs of them in LDS at a time, 16 of them then add from
+// there.  (With each thread walking the slabs in memory, one load behind the
+// other in 16 blocks, the 512 slabs of a 65536-row batch took 119 us a matrix;
+// the four matrices in one launch of this take 12 us.)
+struct SumSplits {
+  const float* part[4];
+  float* out[4];
+  int n[4];  // outputs of each matrix, multiples of 16
+  int nsplit;
+};
+__global__ void __launch_bounds__(256) k_sum_splits(SumSplits a) {
+  __shared__ float buf[256 * 16];
+  int m = 0, o0 = blockIdx.x * 16;
+  while (o0 >= a.n[m]) o0 -= a.n[m++];
+  const float* __restrict__ p = a.part[m] + o0;
+  const int n = a.n[m], o = threadIdx.x & 15, w = threadIdx.x >> 4;
   float s = 0.f;
-  for (int i = 0; i < nsplit; ++i) s += part[(long)i * n + t];
-  out[t] = accumulate ? out[t] + s : s;
-}
-
-// Z = C + bias (per column), H = gelu(Z) in bf16; rows of width 64
-__global__ void k_bias_gelu(const float* C, const float* bias, float* Z, short* H, long n) {
-  const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= n * 64) return;
-  const float z = C[t] + bias[t & 63];
-  Z[t] = z;
-  H[t] = f2bf(gelu(z));
+  for (int i0 = 0; i0 < a.nsplit; i0 += 256) {
+    float v[16];
+#pragma unroll
+    for (int u = 0; u < 16; ++u) {
+      const int i = i0 + 16 * u + w;
+      v[u] = i < a.nsplit ? p[(long)i * n + o] : 0.f;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < 16; ++u) buf[(16 * u + w) * 16 + o] = v[u];
+    __syncthreads();
+    if (threadIdx.x < 16) {
+      const int c = a.nsplit - i0 < 256 ? a.nsplit - i0 : 256;
+#pragma unroll 16
+      for (int i = 0; i < c; ++i) s += buf[i * 16 + threadIdx.x];
+    }
+  }
+  if (threadIdx.x < 16) a.out[m][o0 + threadIdx.x] = s;
 }
 
 // output layer: Y = C + b4 (16 padded columns, 2 used), dY = (Y - T) / n,
@@ -235,28 +255,59 @@ __global__ void k_out_grad(const float* C, const float* b4, const float* T, shor
   if (threadIdx.x == 0) lossp[blockIdx.x] = red[0];
 }
 
-// dZ = dH * gelu'(Z)
-__global__ void k_gelu_back(const float* dH, const float* Z, short* dZ, float* dZf, long n) {
-  const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= n * 64) return;
-  const float d = dH[t] * gelu_d(Z[t]);
-  dZ[t] = f2bf(d);
-  dZf[t] = d;
+// Column sums (bias gradients) of a [n x W] fp32 matrix: 256 running sums per
+// column, sum t over the rows t, t + 256, ... in order (this kernel, part[t][c]),
+// then the 256 of a column as a tree (k_colsum_tree).  A wavefront takes whole
+// rows (a block per column read one value of every row: 89 us at 65536 x 64,
+// now 9),
+// 16 rows' loads in flight, one wavefront per block so that the 256 (W = 64)
+// spread over the CUs.
+#define MLP_SUMS 256
+template <int W>
+__global__ void __launch_bounds__(64) k_colsum_part(const float* __restrict__ X, float* part, long n) {
+  constexpr int U = 16;
+  const int t = (blockIdx.x * 64 + threadIdx.x) / W, c = threadIdx.x % W;
+  const long step = (long)MLP_SUMS * W, full = n / (U * MLP_SUMS) * (U * MLP_SUMS);
+  const float* p = X + (long)t * W + c;
+  float s = 0.f, x[U];
+  long r = t;
+  if (r < full) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) x[u] = p[u * step];
+  }
+  for (; r < full; r += (long)U * MLP_SUMS) {
+    float y[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) y[u] = x[u];
+    p += U * step;
+    if (r + (long)U * MLP_SUMS < full) {  // in flight while these rows are summed
+#pragma unroll
+      for (int u = 0; u < U; ++u) x[u] = p[u * step];
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) s += y[u];
+  }
+  for (; r < n; r += MLP_SUMS, p += step) s += *p;
+  part[t * W + c] = s;
 }
 
-// column sums of a [n x w] fp32 matrix (bias gradients)
-__global__ void k_colsum(const float* X, float* out, long n, int w) {
-  __shared__ float red[256];
-  const int c = blockIdx.x;
-  float s = 0.f;
-  for (long r = threadIdx.x; r < n; r += blockDim.x) s += X[r * w + c];
-  red[threadIdx.x] = s;
+// the tree over each column's 256 sums, one block per column of up to four matrices
+struct ColTree {
+  const float* part[4];
+  float* out[4];
+  int w[4];
+};
+__global__ void __launch_bounds__(256) k_colsum_tree(ColTree a) {
+  __shared__ float red[MLP_SUMS];
+  int m = 0, c = blockIdx.x;
+  while (c >= a.w[m]) c -= a.w[m++];
+  red[threadIdx.x] = a.part[m][threadIdx.x * a.w[m] + c];
   __syncthreads();
-  for (int k = blockDim.x / 2; k > 0; k >>= 1) {
+  for (int k = MLP_SUMS / 2; k > 0; k >>= 1) {
     if ((int)threadIdx.x < k) red[threadIdx.x] += red[threadIdx.x + k];
     __syncthreads();
   }
-  if (threadIdx.x == 0) out[c] = red[0];
+  if (threadIdx.x == 0) a.out[m][c] = red[0];
 }
 
 // Adam on the fp32 master parameters; refreshes the bf16 matrix mirror
