@@ -17,7 +17,10 @@ template <typename T, int N>
 struct ColResShape {
   static constexpr int NB = 3 * N / 2;
   static constexpr int NT = ph_threads(N, NB, col_maxg<T>());
-  static constexpr int CB0 = 128 / (int)sizeof(Cplx<T>);
+  // 128-byte segments; FP32 from 384 on 64-byte ones, where two blocks or one
+  // of 16 lines would fill the LDS of a CU (512 <-> 768, 256 levels: padding
+  // 2055 -> 1740 us, truncation 958 -> 825; 384 <-> 576 padding 448 -> 423)
+  static constexpr int CB0 = sizeof(T) == 8 || N >= 384 ? 8 : 16;
   static constexpr int CB = NT * CB0 >= 64 ? CB0 : NT * CB0 * 2 >= 64 ? 2 * CB0 : NT * CB0 * 4 >= 64 ? 4 * CB0 : 8 * CB0;
   static constexpr int LS = NB | 1;
   static constexpr int THREADS = NT * CB;
