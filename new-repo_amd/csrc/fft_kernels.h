@@ -13,8 +13,11 @@
 #include "les_common.h"
 
 #define LES_BLOCK 256
+// fields a launch takes: the dynamic models filter up to 21 at once, two results each
 #define LES_MAX_FIELDS 6
-#define LES_COL_JOBS 3
+#define LES_R2C_FIELDS 21
+#define LES_C2R_FIELDS 42
+#define LES_COL_JOBS 21
 
 // ------------------------------------------------------------------ row r2c
 // Load modes of the real input.
@@ -28,8 +31,8 @@ enum { LOAD_SCALE = 0, LOAD_SCALE_DIV = 1, LOAD_AB2_SCALE_DIV = 2, LOAD_PCLEAN =
 
 template <typename TI, typename T>
 struct RowR2CArgs {
-  const TI* src[LES_MAX_FIELDS];
-  Cplx<T>* dst[LES_MAX_FIELDS];
+  const TI* src[LES_R2C_FIELDS];
+  Cplx<T>* dst[LES_R2C_FIELDS];
   int nx, ny, lhx;
   int k0, nplanes;  // planes [k0, k0+nplanes)
   int mode;
@@ -135,8 +138,8 @@ k_rows_r2c_nyq(RowR2CArgs<double, T> a, FftPlan pl, const Cplx<T>* __restrict__ 
 // ------------------------------------------------------------------ row c2r
 template <typename T, typename TO>
 struct RowC2RArgs {
-  const Cplx<T>* src[LES_MAX_FIELDS];
-  TO* dst[LES_MAX_FIELDS];
+  const Cplx<T>* src[LES_C2R_FIELDS];
+  TO* dst[LES_C2R_FIELDS];
   int nx, ny, lhx;
   int k0, nplanes;
 };
@@ -199,6 +202,8 @@ struct RowResArgs {
   T cconv;
   int ny;
   int k0, nplanes;
+  // truncation: the planes k0 - 1 and k0 + nplanes are filled with `ghost`
+  double ghost;
 };
 
 // Column resampling: column pairs (i, i+1) of a real (W, h1) plane -> (W, h2)

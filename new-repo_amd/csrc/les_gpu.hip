@@ -287,8 +287,8 @@ static void grad_filt(Les& L, int fid, int dx_id, int dy_id) {
 // grad_velocity_filt for u, v and w together, with the arithmetic of
 // grad_filt per field: the forward transforms (one launch of three fields,
 // or one per field where the mixed mode forms the Nyquist sums), one column
-// launch of three jobs, one inverse launch of the six derivatives and, in
-// FP64, one of the three filtered fields.  The FP64 filtered spectra
+// launch of three jobs and one inverse launch of the six derivatives and, in
+// FP64, the three filtered fields.  The FP64 filtered spectra
 // overwrite the inputs: k_cols_reg reads its whole tile before its first
 // store and every block owns its tile.
 // Measured at 256^3 (MI355X): FP64 0.055 ms per step faster than three
@@ -304,8 +304,8 @@ static void grad_filt3(Les& L) {
   Cplx<T>* ox[3];
   Cplx<T>* oy[3];
   const double* src[3];
-  const Cplx<T>* cs[6];
-  T* outs[6];
+  const Cplx<T>* cs[9];
+  T* outs[9];
   for (int f = 0; f < 3; ++f) {
     in[f] = (Cplx<T>*)L.wk_spec[f];
     ox[f] = (Cplx<T>*)L.wk_spec[3 + f];
@@ -325,11 +325,12 @@ static void grad_filt3(Les& L) {
     rows_r2c<double, T>(L, src, in, 3, 0, L.nzg, c);
   }
   cols_jobs<T>(L, COP_GRAD, 3, in, nullptr, ox, oy, L.mixed ? nullptr : in, L.mixed ? 2 : 3, 1, 1, 0, L.nzg);
-  rows_c2r<T, T>(L, cs, outs, 6, 0, L.nzg);
-  if (!L.mixed) {
-    const Cplx<T>* c3[3] = {in[0], in[1], in[2]};
-    double* o3[3] = {D(L, LES_U), D(L, LES_V), D(L, LES_W)};
-    rows_c2r<T, double>(L, c3, o3, 3, 0, L.nzg);
+  if constexpr (std::is_same<T, double>::value) {
+    // the filtered fields with the derivatives in one launch
+    for (int f = 0; f < 3; ++f) { cs[6 + f] = in[f]; outs[6 + f] = D(L, fid[f]); }
+    rows_c2r<T, T>(L, cs, outs, 9, 0, L.nzg);
+  } else {
+    rows_c2r<T, T>(L, cs, outs, 6, 0, L.nzg);
   }
 }
 
@@ -401,8 +402,8 @@ static void wall_law(Les& L) {
     Cplx<T>* dst[2] = {sa, sb};
     rows_r2c<double, T>(L, src, dst, 2, 0, 1, (T)1);
     const T* g2 = sizeof(T) == 8 ? (const T*)L.g2_64 : (const T*)L.g2_32;
-    cols<T>(L, COP_FILT1, sa, nullptr, sc, nullptr, nullptr, 1, 1, 1, 0, 1, g2);
-    cols<T>(L, COP_FILT1, sb, nullptr, sd, nullptr, nullptr, 1, 1, 1, 0, 1, g2);
+    Cplx<T>* fl[2] = {sc, sd};
+    cols_jobs<T>(L, COP_FILT1, 2, dst, nullptr, fl, nullptr, nullptr, 1, 1, 1, 0, 1, g2);
     const Cplx<T>* cs[2] = {sc, sd};
     T* outs[2] = {u1, v1};
     rows_c2r<T, T>(L, cs, outs, 2, 0, 1);
@@ -1164,7 +1165,16 @@ int les_init(const les_params* p) {
   }
   // w(:,:,0) = BOGUS (src/system.f90:196-198) is set by les_set_ic.
   // ---- workspaces
-  for (int i = 0; i < LES_NSPEC; ++i) L->wk_spec[i] = dalloc(*L, 2 * tb * L->nsp);
+  // Test filters of the dynamic models: as many of the 21 fields per launch as
+  // keep the spectra (one in, two out each) within the 256 MB last-level cache.
+  // Small grids pay for launches: one update's column passes at 64^3 in FP64
+  // 87 us in 7 launches, 32 us in one; at 128^3 in FP32 141 us in 7, 121 in 3.
+  // Larger grids fill the card with 3 fields and gain nothing from more.
+  L->filt_batch = 3;
+  for (int nb : {7, 21})
+    if (3.0 * nb * 2 * tb * L->nsp <= 256.0 * (1 << 20)) L->filt_batch = nb;
+  const int nspec = 3 * L->filt_batch > LES_NSPEC ? 3 * L->filt_batch : LES_NSPEC;
+  for (int i = 0; i < nspec; ++i) L->wk_spec[i] = dalloc(*L, 2 * tb * L->nsp);
   for (int i = 0; i < 64; ++i) L->wk_real[i] = dalloc(*L, tb * L->nf);
   for (int i = 0; i < 6; ++i) L->wk_hyb[i] = dalloc(*L, tb * (size_t)L->nx2 * L->ny * L->nzg);
   for (int i = 0; i < 6; ++i) L->wk_big[i] = dalloc(*L, tb * (size_t)L->nbp * L->nzg);

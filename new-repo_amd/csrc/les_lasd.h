@@ -169,26 +169,26 @@ static void lasd_update(Les& L, int jtt, int nlev) {
   T* fl2[21];
   T* fl4[21];
   for (int f = 0; f < 21; ++f) { fl2[f] = (T*)L.wk_real[15 + f]; fl4[f] = (T*)L.wk_real[36 + f]; }
-  // three fields at a time: inputs in spectral slots 0..2, filtered outputs in 3..8
-  static_assert(LES_NSPEC >= 9, "Germano filtering needs 9 spectral workspaces");
-  for (int f0 = 0; f0 < 21; f0 += 3) {
-    const T* src[3];
-    Cplx<T>* sp[3];
-    for (int t = 0; t < 3; ++t) { src[t] = in[f0 + t]; sp[t] = (Cplx<T>*)L.wk_spec[t]; }
-    rows_r2c<T, T>(L, src, sp, 3, 1, nlev, (T)1);
-    Cplx<T>* o2[3];
-    Cplx<T>* o4[3];
-    for (int t = 0; t < 3; ++t) { o2[t] = (Cplx<T>*)L.wk_spec[3 + 2 * t]; o4[t] = (Cplx<T>*)L.wk_spec[4 + 2 * t]; }
-    cols_jobs<T>(L, COP_FILT2, 3, sp, nullptr, o2, o4, nullptr, 2, 1, 1, 1, nlev, g2, g4);
-    const Cplx<T>* cs[6];
-    T* outs[6];
-    for (int t = 0; t < 3; ++t) {
-      cs[2 * t] = (Cplx<T>*)L.wk_spec[3 + 2 * t];
-      cs[2 * t + 1] = (Cplx<T>*)L.wk_spec[4 + 2 * t];
+  // nb fields at a time: inputs in spectral slots 0.., their two results after them
+  const int nb = L.filt_batch;
+  for (int f0 = 0; f0 < 21; f0 += nb) {
+    const T* src[21];
+    Cplx<T>* sp[21];
+    Cplx<T>* o2[21];
+    Cplx<T>* o4[21];
+    const Cplx<T>* cs[42];
+    T* outs[42];
+    for (int t = 0; t < nb; ++t) {
+      src[t] = in[f0 + t];
+      sp[t] = (Cplx<T>*)L.wk_spec[t];
+      cs[2 * t] = o2[t] = (Cplx<T>*)L.wk_spec[nb + 2 * t];
+      cs[2 * t + 1] = o4[t] = (Cplx<T>*)L.wk_spec[nb + 2 * t + 1];
       outs[2 * t] = fl2[f0 + t];
       outs[2 * t + 1] = fl4[f0 + t];
     }
-    rows_c2r<T, T>(L, cs, outs, 6, 1, nlev);
+    rows_r2c<T, T>(L, src, sp, nb, 1, nlev, (T)1);
+    cols_jobs<T>(L, COP_FILT2, nb, sp, nullptr, o2, o4, nullptr, 2, 1, 1, 1, nlev, g2, g4);
+    rows_c2r<T, T>(L, cs, outs, 2 * nb, 1, nlev);
   }
   T* LM = (T*)L.wk_real[57];
   T* MM = (T*)L.wk_real[58];
@@ -355,22 +355,22 @@ static void dynsmag_update(Les& L) {
   const T* g2 = sizeof(T) == 8 ? (const T*)L.g2_64 : (const T*)L.g2_32;
   T* fl[21];
   for (int f = 0; f < 21; ++f) fl[f] = (T*)L.wk_real[15 + f];
-  for (int f0 = 0; f0 < 21; f0 += 3) {
-    const T* src[3];
-    Cplx<T>* sp[3];
-    const Cplx<T>* cs[3];
-    T* outs[3];
-    for (int t = 0; t < 3; ++t) {
+  const int nb = L.filt_batch;
+  for (int f0 = 0; f0 < 21; f0 += nb) {
+    const T* src[21];
+    Cplx<T>* sp[21];
+    Cplx<T>* fo[21];
+    const Cplx<T>* cs[21];
+    T* outs[21];
+    for (int t = 0; t < nb; ++t) {
       src[t] = in[f0 + t];
       sp[t] = (Cplx<T>*)L.wk_spec[t];
-      cs[t] = (const Cplx<T>*)L.wk_spec[3 + t];
+      cs[t] = fo[t] = (Cplx<T>*)L.wk_spec[nb + t];
       outs[t] = fl[f0 + t];
     }
-    rows_r2c<T, T>(L, src, sp, 3, 1, nlev, (T)1);
-    Cplx<T>* fo[3];
-    for (int t = 0; t < 3; ++t) fo[t] = (Cplx<T>*)L.wk_spec[3 + t];
-    cols_jobs<T>(L, COP_FILT1, 3, sp, nullptr, fo, nullptr, nullptr, 1, 1, 1, 1, nlev, g2);
-    rows_c2r<T, T>(L, cs, outs, 3, 1, nlev);
+    rows_r2c<T, T>(L, src, sp, nb, 1, nlev, (T)1);
+    cols_jobs<T>(L, COP_FILT1, nb, sp, nullptr, fo, nullptr, nullptr, 1, 1, 1, 1, nlev, g2);
+    rows_c2r<T, T>(L, cs, outs, nb, 1, nlev);
   }
   GermanoArgs<T> ga;
   for (int f = 0; f < 21; ++f) ga.fl[f] = fl[f];

@@ -15,7 +15,8 @@ struct MlpState {
   // 4-delta filtered S_ij and R_ij (fr[0..2], fr[3..11], fr[12..20]) and
   // the transforms' spectra
   float* fr[21];
-  void* fs[9];
+  void* fs[27];    // three per field of a launch (nb of the nine)
+  int nb;
   double* red;     // reduction partials
   long redn;
   int step;
@@ -42,7 +43,8 @@ static int mlp_alloc(Les& L) {
   const long npt = L.np * (L.nz + 1);
   M->X = (short*)dalloc(L, 2 * 16 * (size_t)npt);
   for (int i = 0; i < 21; ++i) M->fr[i] = (float*)dalloc(L, 4 * (size_t)L.nf);
-  for (int i = 0; i < 9; ++i) M->fs[i] = dalloc(L, 2 * 4 * (size_t)L.nsp);
+  M->nb = L.filt_batch >= 7 ? 9 : 3;  // small grids: the nine filtered fields in one launch
+  for (int i = 0; i < 3 * M->nb; ++i) M->fs[i] = dalloc(L, 2 * 4 * (size_t)L.nsp);
   M->redn = 2 * (long)nblk(npt) + 64;
   M->red = (double*)dalloc(L, 8 * (size_t)M->redn);
   L.mlp = M;
@@ -212,24 +214,25 @@ static void learned_coeffs(Les& L, void* cs, void* beta, int eb, int k0) {
   for (int i = 0; i < 9; ++i) { f2[i] = (T*)M->fr[3 + i]; f4[i] = (T*)M->fr[12 + i]; }
   const T* g2 = sizeof(T) == 8 ? (const T*)L.g2_64 : (const T*)L.g2_32;
   const T* g4 = sizeof(T) == 8 ? (const T*)L.g4_64 : (const T*)L.g4_32;
-  for (int f0 = 0; f0 < 9; f0 += 3) {
-    const T* src[3];
-    Cplx<T>* sp[3];
-    for (int t = 0; t < 3; ++t) { src[t] = in9[f0 + t]; sp[t] = (Cplx<T>*)M->fs[t]; }
-    rows_r2c<T, T>(L, src, sp, 3, k0, nlev, (T)1);
-    Cplx<T>* o2[3];
-    Cplx<T>* o4[3];
-    for (int t = 0; t < 3; ++t) { o2[t] = (Cplx<T>*)M->fs[3 + 2 * t]; o4[t] = (Cplx<T>*)M->fs[4 + 2 * t]; }
-    cols_jobs<T>(L, COP_FILT2, 3, sp, nullptr, o2, o4, nullptr, 2, 1, 1, k0, nlev, g2, g4);
-    const Cplx<T>* cs6[6];
-    T* outs[6];
-    for (int t = 0; t < 3; ++t) {
-      cs6[2 * t] = (Cplx<T>*)M->fs[3 + 2 * t];
-      cs6[2 * t + 1] = (Cplx<T>*)M->fs[4 + 2 * t];
+  const int nb = M->nb;
+  for (int f0 = 0; f0 < 9; f0 += nb) {
+    const T* src[9];
+    Cplx<T>* sp[9];
+    Cplx<T>* o2[9];
+    Cplx<T>* o4[9];
+    const Cplx<T>* cs18[18];
+    T* outs[18];
+    for (int t = 0; t < nb; ++t) {
+      src[t] = in9[f0 + t];
+      sp[t] = (Cplx<T>*)M->fs[t];
+      cs18[2 * t] = o2[t] = (Cplx<T>*)M->fs[nb + 2 * t];
+      cs18[2 * t + 1] = o4[t] = (Cplx<T>*)M->fs[nb + 2 * t + 1];
       outs[2 * t] = f2[f0 + t];
       outs[2 * t + 1] = f4[f0 + t];
     }
-    rows_c2r<T, T>(L, cs6, outs, 6, k0, nlev);
+    rows_r2c<T, T>(L, src, sp, nb, k0, nlev, (T)1);
+    cols_jobs<T>(L, COP_FILT2, nb, sp, nullptr, o2, o4, nullptr, 2, 1, 1, k0, nlev, g2, g4);
+    rows_c2r<T, T>(L, cs18, outs, 2 * nb, k0, nlev);
   }
   FeatArgs fa;
   for (int i = 0; i < 6; ++i) { fa.s[0][i] = (const float*)in9[i]; fa.s[1][i] = (const float*)f2[i]; fa.s[2][i] = (const float*)f4[i]; }

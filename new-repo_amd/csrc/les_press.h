@@ -212,8 +212,7 @@ static void press_stag_array(Les& L, double tadv1, bool ab2 = false, double tadv
   const double* lsrc[2] = {L.layer[LES_BOTTOM_WK], L.layer[LES_TOP_WK]};
   Cplx<double>* ldst[2] = {lb, lt};
   rows_r2c<double, double>(L, lsrc, ldst, 2, 0, 1, c);
-  cols<double>(L, COP_COPY, lb, nullptr, lb, nullptr, nullptr, 1, 1, 0, 0, 1);
-  cols<double>(L, COP_COPY, lt, nullptr, lt, nullptr, nullptr, 1, 1, 0, 0, 1);
+  cols_jobs<double>(L, COP_COPY, 2, ldst, nullptr, ldst, nullptr, nullptr, 1, 1, 0, 0, 1);
   // tridiagonal solve per mode
   TriArgs t;
   t.Hd = Hx; t.Hz = Hz; t.bot = lb; t.top = lt;

@@ -227,16 +227,12 @@ static void convection(Les& L, double* cx, double* cy, double* cz) {
     a.src[0] = (const T*)L.wk_hyb3[0]; a.src[1] = (const T*)L.wk_hyb3[1]; a.src[2] = (const T*)L.wk_hyb3[2];
     a.dst[0] = cx; a.dst[1] = cy; a.dst[2] = cz;
     a.ny = ny; a.k0 = 1; a.nplanes = nz;
+    a.ghost = BOGUS;  // levels 0 and nz+1 hold no value
     kt_begin(L, KT_ROWS_RES);
     rows_trunc_reg<T>(false, nx, a, 3, twpool<T>(L) + L.px.twf, twpool<T>(L) + L.px2.twf, L.stream);
     kt_end(L, KT_ROWS_RES, 3.0 * nz * ny * ((double)nx2 * sizeof(T) + (double)nx * 8), "k_rows_resample_reg", sizeof(T),
            sizeof(T), "truncate");
   }
-  SetPlaneArgs sp;
-  sp.a = cx; sp.b = cy; sp.c = cz; sp.np = L.np; sp.k0 = 0; sp.k1 = nz + 1; sp.val = BOGUS;
-  kt_begin(L, KT_POINTWISE);
-  hipLaunchKernelGGL(k_set_planes, dim3(nblk(L.np)), dim3(LES_BLOCK), 0, L.stream, sp);
-  kt_end(L, KT_POINTWISE, 6.0 * 8 * L.np, "k_set_planes");
 }
 
 template <typename T>

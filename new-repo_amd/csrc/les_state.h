@@ -6,8 +6,10 @@
 #include "../../include/les_gpu.h"
 #include "fft_kernels.h"
 
-// Number of spectral workspaces (the Germano filtering uses slots 0..8).
+// Spectral workspaces: at least LES_NSPEC, and three per field that the dynamic
+// models filter at once (Les::filt_batch, at most 21).
 #define LES_NSPEC 12
+#define LES_NSPEC_MAX 63
 
 // Kernel families timed with HIP events when timing is enabled.
 enum {
@@ -54,7 +56,8 @@ struct Les {
   double* z0;
 
   // workspaces
-  void* wk_spec[LES_NSPEC]; // spectral (lhx, ny, nzg) of flow precision
+  void* wk_spec[LES_NSPEC_MAX]; // spectral (lhx, ny, nzg) of flow precision
+  int filt_batch;         // fields of the dynamic models' test filters per launch
   void* wk_real[64];      // real (nx, ny, nzg) of flow precision
   void* wk_hyb[6];        // (nx2, ny, nzg)
   void* wk_big[6];        // (nx2, ny2, nzg)

@@ -382,6 +382,19 @@ __global__ void __launch_bounds__((RowShape<T, N, 3 * N / 2>::THREADS)) k_rows_r
   using L1 = RegLine<T, N1, NT, col_maxg<T>(), true>;
   using L2 = RegLine<T, N2, NT, col_maxg<T>(), true>;
   extern __shared__ __align__(16) unsigned char smem_raw[];
+  if constexpr (!PAD) {
+    // the blocks past the row pairs fill the ghost planes below and above
+    const long np = (long)N * a.ny, nb = ((long)a.nplanes * (a.ny / 2) + S::LB - 1) / S::LB;
+    if ((long)blockIdx.x >= nb) {
+      TO* __restrict__ lo = a.dst[blockIdx.y] + (a.k0 - 1) * np;
+      TO* __restrict__ hi = a.dst[blockIdx.y] + (a.k0 + a.nplanes) * np;
+      for (long q = (blockIdx.x - nb) * S::THREADS + threadIdx.x; q < np; q += (gridDim.x - nb) * S::THREADS) {
+        lo[q] = (TO)a.ghost;
+        hi[q] = (TO)a.ghost;
+      }
+      return;
+    }
+  }
   const RowAt<S> at((long)a.nplanes * (a.ny / 2));
   Cplx<T>* line = reinterpret_cast<Cplx<T>*>(smem_raw) + at.line() * S::LS;
   const int f = blockIdx.y;
