@@ -927,6 +927,8 @@ static bool setup_fft_attrs(const Les& L) {
          rows_trunc_reg<T>(true, L.nx, RowResArgs<T, T, double>(), 0, nullptr, nullptr, 0);
 }
 static int setup_kernel_attrs(const Les& L) {
+  if (tri_in_lds(L.lhx, L.ny, L.nz))
+    hipFuncSetAttribute((const void*)k_tridiag_lds, hipFuncAttributeMaxDynamicSharedMemorySize, (int)tri_lds(L.nz));
   const bool ok = setup_fft_attrs<double>(L) && setup_fft_attrs<float>(L) &&
                   rows_r2c_reg<float, float>(true, L.nx, RowR2CArgs<float, float>(), 0, nullptr, 0) &&
                   rows_c2r_reg<float, float>(true, L.nx, RowC2RArgs<float, float>(), 0, nullptr, 0) &&

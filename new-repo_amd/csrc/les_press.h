@@ -37,18 +37,20 @@ struct TriArgs {
 // once.
 __host__ __device__ inline long tri_nwork(int lhx, int ny) { return (long)(lhx - 1) * (ny - 1); }
 __host__ __device__ inline long tri_zero_blocks(int lhx, int ny) { return ((long)lhx * ny - tri_nwork(lhx, ny) + 63) / 64; }
+// p^ = 0 of Nyquist mode m: the row j = ny/2 (every i), then the column
+// i = lhx-1 of the other rows
+__device__ __forceinline__ void tri_zero(const TriArgs& a, long m) {
+  if (m >= (long)a.lhx + a.ny - 1) return;
+  const int jn = (int)(m - a.lhx);
+  const long q = m < a.lhx ? (long)(a.ny / 2) * a.lhx + m : (long)(jn < a.ny / 2 ? jn : jn + 1) * a.lhx + a.lhx - 1;
+  for (int k = 0; k <= a.nz + 1; ++k) a.phat[(long)k * a.ns + q] = Cplx<double>{0.0, 0.0};
+}
 __global__ void __launch_bounds__(64) k_tridiag(TriArgs a) {
   const int nz = a.nz;
   const long ns = a.ns;
   const long nzb = tri_zero_blocks(a.lhx, a.ny);
   if (blockIdx.x < nzb) {
-    // Nyquist modes, one lane each: the row j = ny/2 (every i), then the
-    // column i = lhx-1 of the other rows
-    const long m = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (m >= (long)a.lhx + a.ny - 1) return;
-    const int jn = (int)(m - a.lhx);
-    const long q = m < a.lhx ? (long)(a.ny / 2) * a.lhx + m : (long)(jn < a.ny / 2 ? jn : jn + 1) * a.lhx + a.lhx - 1;
-    for (int k = 0; k <= nz + 1; ++k) a.phat[(long)k * ns + q] = Cplx<double>{0.0, 0.0};
+    tri_zero(a, (long)blockIdx.x * blockDim.x + threadIdx.x);
     return;
   }
   const long t = (long)(blockIdx.x - nzb) * blockDim.x + threadIdx.x;
@@ -180,6 +182,161 @@ __global__ void __launch_bounds__(64) k_tridiag(TriArgs a) {
   ph[2 * ((long)(nz + 1) * ns + q)] = 0.0;
 }
 
+// The same sweeps with the columns in LDS: a block of four wavefronts takes
+// LES_TRI_M modes and each wavefront one part of the work, a chunk of
+// LES_TRI_U rows apart:
+//   0  the factors g_k and bet_k (they depend on the mode only),
+//   1  x_k = (r_k - am x_{k-1}) / bet_k, then the back substitution (two lanes
+//      per mode, one per component),
+//   2, 3  the right-hand side r_k of the rows ahead, loaded, divided by dz and
+//      put where x_k will stand.
+// Bound by the chain of a division and two operations per row: 0.17 us a row
+// for both sweeps, where k_tridiag, with all three divisions of a row and the
+// recomputed factors in one wavefront, takes 0.33.  Operations and their order
+// are the same.  64^3: 27.2 -> 16.2 us, 128^3: 52.3 -> 27.9, 192x144x65: 35.1
+// -> 23.1, 512x512x64: 162 -> 130 (the column is not written and read between
+// the sweeps).
+#define LES_TRI_M 32
+__host__ __device__ inline size_t tri_lds(int nz) {
+  return sizeof(double) * ((size_t)(nz + 1) * 2 * LES_TRI_M + (size_t)nz * LES_TRI_M + 2 * LES_TRI_U * LES_TRI_M);
+}
+inline long tri_lds_blocks(int lhx, int ny) { return (tri_nwork(lhx, ny) + LES_TRI_M - 1) / LES_TRI_M; }
+// Taken where two blocks fit a CU (columns up to 95 levels: never slower,
+// 256x256x64 44.0 -> 39.4 us), or where the grid is one round of one block a CU
+// (up to 201 levels).  With more rounds of one block the few modes in flight
+// cost more than the column's traffic: 256x256x128 75 us against 103,
+// 384x384x128 212 against 232.
+inline bool tri_in_lds(int lhx, int ny, int nz) {
+  const size_t cu = 160 * 1024;
+  return 2 * tri_lds(nz) <= cu || (tri_lds(nz) <= cu && tri_lds_blocks(lhx, ny) <= 256);
+}
+__global__ void __launch_bounds__(256) k_tridiag_lds(TriArgs a) {
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  constexpr int U = LES_TRI_U, M = LES_TRI_M;
+  const int nz = a.nz;
+  const long ns = a.ns;
+  const long nzb = ((long)a.lhx + a.ny - 1 + 255) / 256;
+  if (blockIdx.x < nzb) {
+    tri_zero(a, (long)blockIdx.x * 256 + threadIdx.x);
+    return;
+  }
+  double* __restrict__ X = reinterpret_cast<double*>(smem_raw);  // row k at (k-1) 2M: r_k, then x_k
+  double* __restrict__ G = X + (size_t)(nz + 1) * 2 * M;         // row k at (k-2) M: g_k
+  double* __restrict__ B = G + (size_t)nz * M;                   // bet_k of two chunks
+  const int lane = threadIdx.x & 63, role = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const long nwork = tri_nwork(a.lhx, a.ny);
+  const int ml = role == 0 ? lane & (M - 1) : lane >> 1, c = lane & 1;
+  const long w0 = (long)(blockIdx.x - nzb) * M + ml;
+  const bool valid = w0 < nwork;
+  const long w = valid ? w0 : nwork - 1;
+  const int i = (int)(w % (a.lhx - 1)), jw = (int)(w / (a.lhx - 1));
+  const int j = jw < a.ny / 2 ? jw : jw + 1;
+  const long q = (long)j * a.lhx + i;
+  const double dz = a.dz, idz2 = a.idz2;
+  const bool mean = (i == 0 && j == 0);
+  const int nchunk = (nz + U - 1) / U;
+  if (role == 0) {
+    const double kx = a.kkx[q], ky = a.kky[q];
+    const double bmid = -((kx * kx + ky * ky) + 2.0 / (dz * dz));
+    double bet = mean ? 1.0 : -1.0, cprev = mean ? 0.0 : 1.0;
+    for (int ch = 0; ch < nchunk; ++ch) {
+      double* __restrict__ Bc = B + (ch & 1) * U * M + ml;
+      double* __restrict__ Gc = G + (size_t)ch * U * M + ml;
+      const int n = nz - ch * U < U ? nz - ch * U : U;
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        if (u < n) {
+          const double g = cprev / bet;
+          bet = bmid - idz2 * g;
+          cprev = idz2;
+          Gc[u * M] = g;
+          Bc[u * M] = bet;
+        }
+      }
+      block_sync_lds();
+    }
+    return;
+  }
+  if (role >= 2) {
+    // half a chunk each, the next half chunk's loads in flight
+    constexpr int H = U / 2;
+    const double* __restrict__ hd = reinterpret_cast<const double*>(a.Hd) + 2 * q + c;
+    const double* __restrict__ hz = reinterpret_cast<const double*>(a.Hz) + 2 * q + c;
+    double d[H], z[H + 1];
+    auto load = [&](int ch) LES_INLINE {
+      const int k0 = 1 + ch * U + (role - 2) * H;  // plane of the first row
+#pragma unroll
+      for (int u = 0; u < H; ++u) d[u] = k0 + u <= nz ? hd[2 * (k0 + u) * ns] : 0.0;
+#pragma unroll
+      for (int u = 0; u <= H; ++u) z[u] = k0 + u <= nz ? hz[2 * (k0 + u) * ns] : 0.0;
+    };
+    load(0);
+    for (int ch = 0; ch < nchunk; ++ch) {
+      double r[H];
+#pragma unroll
+      for (int u = 0; u < H; ++u) r[u] = d[u] + (z[u + 1] - z[u]) / dz;
+      if (ch + 1 < nchunk) load(ch + 1);
+      const int k0 = 1 + ch * U + (role - 2) * H;
+#pragma unroll
+      for (int u = 0; u < H; ++u)
+        if (k0 + u <= nz) X[(size_t)(k0 + u) * 2 * M + lane] = r[u];
+      block_sync_lds();
+    }
+    return;
+  }
+  double x, bet = mean ? 1.0 : -1.0;
+  {
+    const double r1 = mean ? 0.0 : reinterpret_cast<const double*>(a.bot)[2 * q + c] * dz;
+    x = r1 / bet;
+    X[lane] = x;
+  }
+  const double rtop = reinterpret_cast<const double*>(a.top)[2 * q + c] * dz;
+  for (int ch = 0; ch < nchunk; ++ch) {
+    block_sync_lds();
+    const double* __restrict__ Bc = B + (ch & 1) * U * M + ml;
+    double* __restrict__ Xc = X + (size_t)(1 + ch * U) * 2 * M + lane;
+    const int n = nz - ch * U < U ? nz - ch * U : U;
+    double r[U], b[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      r[u] = u < n ? Xc[u * 2 * M] : 0.0;
+      b[u] = u < n ? Bc[u * M] : 1.0;
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      if (u < n) {
+        x = (r[u] - idz2 * x) / b[u];
+        Xc[u * 2 * M] = x;
+        bet = b[u];
+      }
+    }
+  }
+  // row nz+2 (its value is not kept), then rows nz+1 .. 1
+  const double gtop = idz2 / bet;
+  double xn = (rtop + x) / (1.0 + gtop);
+  double* __restrict__ ph = reinterpret_cast<double*>(a.phat) + 2 * q + c;
+  xn = x - gtop * xn;
+  if (valid) {
+    ph[2 * (long)(nz + 1) * ns] = 0.0;
+    ph[2 * (long)nz * ns] = xn;
+  }
+  for (int k0 = nz - 1; k0 >= 0; k0 -= U) {
+    double v[U], g[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      v[u] = k0 - u >= 0 ? X[(size_t)(k0 - u) * 2 * M + lane] : 0.0;
+      g[u] = k0 - u >= 0 ? G[(size_t)(k0 - u) * M + ml] : 0.0;
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      if (k0 - u >= 0) {
+        xn = v[u] - g[u] * xn;
+        if (valid) ph[2 * (long)(k0 - u) * ns] = xn;
+      }
+    }
+  }
+}
+
 // With ab2 set the right-hand side is formed from u + dt (tadv1 rhs + tadv2
 // rhs_f) on load (u, v, w themselves are left as they are; the projection
 // forms the same predictor again).
@@ -222,8 +379,13 @@ static void press_stag_array(Les& L, double tadv1, bool ab2 = false, double tadv
   t.lhx = L.lhx; t.ny = L.ny; t.nz = nz; t.ns = L.ns;
   t.dz = L.dz; t.idz2 = 1.0 / (L.dz * L.dz);
   kt_begin(L, KT_TRIDIAG);
-  const long tri_blocks = tri_zero_blocks(L.lhx, L.ny) + (2 * tri_nwork(L.lhx, L.ny) + 63) / 64;
-  hipLaunchKernelGGL(k_tridiag, dim3((unsigned)tri_blocks), dim3(64), 0, L.stream, t);
+  if (tri_in_lds(L.lhx, L.ny, nz)) {
+    const long blocks = (L.lhx + L.ny - 1 + 255) / 256 + tri_lds_blocks(L.lhx, L.ny);
+    hipLaunchKernelGGL(k_tridiag_lds, dim3((unsigned)blocks), dim3(256), tri_lds(nz), L.stream, t);
+  } else {
+    const long blocks = tri_zero_blocks(L.lhx, L.ny) + (2 * tri_nwork(L.lhx, L.ny) + 63) / 64;
+    hipLaunchKernelGGL(k_tridiag, dim3((unsigned)blocks), dim3(64), 0, L.stream, t);
+  }
   kt_end(L, KT_TRIDIAG, 16.0 * L.ns * (2.0 * nz + 2.0 + (nz + 2.0)), "k_tridiag");
   // gradient: i kx p, i ky p and p back to physical space (src/compute_pressure.f90:320-357)
   cols<double>(L, COP_PGRAD, ph, nullptr, Hx, Hy, Hz, 3, 0, 1, 0, nz + 2);
