@@ -43,8 +43,9 @@ struct RowR2CArgs {
   T ab_dt, ab_t1, ab_t2;
   int pc_nz;          // LOAD_PCLEAN: nz (planes 0 and nz+1 are ghosts)
   // k_rows_r2c_nyq: the FP64 Nyquist sums of the raw input (row sums A,
-  // column partials P of each band of 8 rows)
+  // column partials P of each band of 8 rows), and the strides between fields
   double *nyq_a, *nyq_p;
+  long nyq_as, nyq_ps;
 };
 
 // LDS layout of the row transforms: the register-twiddle 256-point
@@ -83,7 +84,7 @@ __device__ __forceinline__ void rows_r2c_nyq_body(const RowR2CArgs<TI, T>& a, Cp
     s1 += __shfl_xor(s1, o, LES_WAVE);
   }
   if (lane == 0) {
-    double* A = a.nyq_a + (long)k * a.ny + 2 * jp;
+    double* A = a.nyq_a + f * a.nyq_as + (long)k * a.ny + 2 * jp;
     A[0] = s0 / (double)nx;
     A[1] = s1 / (double)nx;
   }
@@ -130,7 +131,7 @@ k_rows_r2c_nyq(RowR2CArgs<double, T> a, FftPlan pl, const Cplx<T>* __restrict__ 
   }
   __syncthreads();
   const int nx = a.nx;
-  double* __restrict__ P = a.nyq_p + (long)blockIdx.x * nx;
+  double* __restrict__ P = a.nyq_p + blockIdx.y * a.nyq_ps + (long)blockIdx.x * nx;
   for (int i = threadIdx.x; i < nx; i += LES_BLOCK)
     P[i] = ((part[i] + part[nx + i]) + part[2 * nx + i]) + part[3 * nx + i];
 }

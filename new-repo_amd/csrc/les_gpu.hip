@@ -171,26 +171,28 @@ static void rows_r2c(Les& L, const TI* const* src, Cplx<T>* const* dst, int nf, 
          mode == LOAD_AB2_SCALE_DIV ? "AB2 predictor" : mode == LOAD_PCLEAN ? "cleaned pressure" : nullptr);
 }
 
-// The grad_velocity_filt forward transform of one velocity component in the
-// mixed mode, with the FP64 Nyquist sums of field slot fld (0 u, 1 v, 2 w)
+// The grad_velocity_filt forward transforms of nf velocity components in the
+// mixed mode, with the FP64 Nyquist sums of field slots fld.. (0 u, 1 v, 2 w)
 // formed on the way (k_rows_r2c_nyq).  Needs ny % 8 == 0.
-static void rows_r2c_nyq(Les& L, const double* src, Cplx<float>* dst, int npl, float scale, int fld) {
+static void rows_r2c_nyq(Les& L, const double* const* src, Cplx<float>* const* dst, int nf, int npl, float scale, int fld) {
   RowR2CArgs<double, float> a;
-  a.src[0] = src; a.dst[0] = dst;
+  for (int f = 0; f < nf; ++f) { a.src[f] = src[f]; a.dst[f] = dst[f]; }
   a.nx = L.nx; a.ny = L.ny; a.lhx = L.lhx; a.k0 = 0; a.nplanes = npl;
   a.mode = LOAD_SCALE; a.scale = scale; a.div = 1.0f;
   a.ls = row_line<float>(L.nx);
-  a.nyq_a = L.nyq_rows + (long)fld * L.ny * L.nzg;
-  a.nyq_p = L.nyq_part + (long)fld * (L.ny / 4) * L.nx * L.nzg;
+  a.nyq_as = (long)L.ny * L.nzg;
+  a.nyq_ps = (long)(L.ny / 4) * L.nx * L.nzg;
+  a.nyq_a = L.nyq_rows + fld * a.nyq_as;
+  a.nyq_p = L.nyq_part + fld * a.nyq_ps;
   const long jobs = (long)npl * (L.ny / 2);
   assert(L.ny % 8 == 0 && jobs % kWavesPerBlock == 0);
   const size_t sh = (size_t)kWavesPerBlock * a.ls * sizeof(Cplx<float>) + (size_t)kWavesPerBlock * L.nx * sizeof(double);
   kt_begin(L, KT_ROWS_R2C);
-  hipLaunchKernelGGL(k_rows_r2c_nyq<float>, dim3((unsigned)(jobs / kWavesPerBlock), 1), dim3(LES_BLOCK), sh, L.stream, a, L.px,
+  hipLaunchKernelGGL(k_rows_r2c_nyq<float>, dim3((unsigned)(jobs / kWavesPerBlock), nf), dim3(LES_BLOCK), sh, L.stream, a, L.px,
                      twpool<float>(L));
   // the field read, its half spectrum written; A (1/nx) and P (1/(8 nx))
   // of a field not counted, as in k_nyq_reduce
-  kt_end(L, KT_ROWS_R2C, (double)npl * L.ny * (L.nx * 8.0 + (double)L.lhx * sizeof(Cplx<float>)), "k_rows_r2c_nyq", 4);
+  kt_end(L, KT_ROWS_R2C, nf * (double)npl * L.ny * (L.nx * 8.0 + (double)L.lhx * sizeof(Cplx<float>)), "k_rows_r2c_nyq", 4);
 }
 
 template <typename T, typename TO>
@@ -268,7 +270,7 @@ static void grad_filt(Les& L, int fid, int dx_id, int dy_id) {
   Cplx<T>* dst[1] = {s0};
   T c = (T)(1.0 / (double)(L.nx * L.ny));
   if constexpr (std::is_same<T, float>::value) {
-    if (nyq_sums_fused(L)) rows_r2c_nyq(L, src[0], s0, L.nzg, c, fid - LES_U);
+    if (nyq_sums_fused(L)) rows_r2c_nyq(L, src, dst, 1, L.nzg, c, fid - LES_U);
     else rows_r2c<double, T>(L, src, dst, 1, 0, L.nzg, c);
   } else {
     rows_r2c<double, T>(L, src, dst, 1, 0, L.nzg, c);
@@ -285,16 +287,17 @@ static void grad_filt(Les& L, int fid, int dx_id, int dy_id) {
 }
 
 // grad_velocity_filt for u, v and w together, with the arithmetic of
-// grad_filt per field: the forward transforms (one launch of three fields,
-// or one per field where the mixed mode forms the Nyquist sums), one column
-// launch of three jobs and one inverse launch of the six derivatives and, in
+// grad_filt per field: the forward transforms of three fields in one launch
+// (in the mixed mode with their Nyquist sums), one column launch of three jobs and one inverse launch of the six derivatives and, in
 // FP64, the three filtered fields.  The FP64 filtered spectra
 // overwrite the inputs: k_cols_reg reads its whole tile before its first
 // store and every block owns its tile.
-// Measured at 256^3 (MI355X): FP64 0.055 ms per step faster than three
-// grad_filt chains; in FP32 0.025 ms slower, its six-field inverse launch
-// reading spectra that the per-field chain still finds in the 256 MB
-// last-level cache.  So the mixed modes keep the per-field chains.
+// Measured at 256^3: FP64 0.055 ms per step faster than three grad_filt
+// chains; in FP32 0.025 ms slower, its six-field inverse launch reading
+// spectra that the per-field chain still finds in the 256 MB last-level
+// cache.  So the mixed modes keep the per-field chains where the nine spectra
+// do not fit that cache, and take three launches instead of nine where they
+// do (128^3: forward rows and columns 93 -> 58 us a step, 96x48x37 42 -> 17).
 template <typename T>
 static void grad_filt3(Les& L) {
   const int fid[3] = {LES_U, LES_V, LES_W};
@@ -317,7 +320,7 @@ static void grad_filt3(Les& L) {
   T c = (T)(1.0 / (double)(L.nx * L.ny));
   if constexpr (std::is_same<T, float>::value) {
     if (nyq_sums_fused(L)) {
-      for (int f = 0; f < 3; ++f) rows_r2c_nyq(L, src[f], in[f], L.nzg, c, f);
+      rows_r2c_nyq(L, src, in, 3, L.nzg, c, 0);
     } else {
       rows_r2c<double, T>(L, src, in, 3, 0, L.nzg, c);
     }
@@ -351,7 +354,7 @@ static void vel_grad_bc_ddz(Les& L);
 // the horizontal gradients of u, v, w (first part of compute_vel_grad)
 template <typename T>
 static void vel_grads(Les& L) {
-  if (L.mixed) {
+  if (L.mixed && 9.0 * sizeof(Cplx<T>) * L.nsp > 256.0 * (1 << 20)) {
     grad_filt<T>(L, LES_U, LES_DUDX, LES_DUDY);
     grad_filt<T>(L, LES_V, LES_DVDX, LES_DVDY);
     grad_filt<T>(L, LES_W, LES_DWDX, LES_DWDY);
@@ -621,8 +624,16 @@ __global__ void __launch_bounds__(LES_BLOCK) k_nyq_bc(NyqArgs a, int nb) {
   const double* __restrict__ A = a.A + (long)fld * ny * a.nzg + k * ny;
   double* __restrict__ B = a.B + (long)fld * nx * a.nzg + k * nx;
   for (int i = threadIdx.x; i < nx; i += blockDim.x) {
+    // 8 loads in flight, added in order
     double s = 0.0;
-    for (int b = 0; b < nb; ++b) s += P[(k * nb + b) * nx + i];
+    for (int b = 0; b < nb; b += 8) {
+      double v[8];
+#pragma unroll
+      for (int t = 0; t < 8; ++t) v[t] = b + t < nb ? P[(k * nb + b + t) * nx + i] : 0.0;
+#pragma unroll
+      for (int t = 0; t < 8; ++t)
+        if (b + t < nb) s += v[t];
+    }
     B[i] = s / (double)ny;
   }
   double c = 0.0;
