@@ -37,6 +37,8 @@ static bool colres_reg(bool attr, int n, bool pad, const ColResArgs<T>& a, int n
 // resampling n <-> 3 n / 2 (twn, twb).  attr and the result as above.
 template <typename TI, typename T, int PART>
 bool rows_r2c_part(bool attr, int n, const RowR2CArgs<TI, T>& a, int nf, const Cplx<T>* tw, hipStream_t s);
+template <typename T, int PART>
+bool rows_nyq_part(bool attr, int n, const RowR2CArgs<double, T>& a, int nf, const Cplx<T>* tw, hipStream_t s);
 template <typename T, typename TO, int PART>
 bool rows_c2r_part(bool attr, int n, const RowC2RArgs<T, TO>& a, int nf, const Cplx<T>* tw, hipStream_t s);
 template <typename T, int PART>
@@ -55,6 +57,12 @@ static_assert(LES_LENGTH_PARTS == 4, "LES_EACH_PART lists the parts");
 template <typename TI, typename T>
 static bool rows_r2c_reg(bool attr, int n, const RowR2CArgs<TI, T>& a, int nf, const Cplx<T>* tw, hipStream_t s) {
 #define C(P) (rows_r2c_part<TI, T, P>(attr, n, a, nf, tw, s))
+  return LES_EACH_PART(C);
+#undef C
+}
+template <typename T>
+static bool rows_nyq_reg(bool attr, int n, const RowR2CArgs<double, T>& a, int nf, const Cplx<T>* tw, hipStream_t s) {
+#define C(P) (rows_nyq_part<T, P>(attr, n, a, nf, tw, s))
   return LES_EACH_PART(C);
 #undef C
 }

@@ -10,7 +10,7 @@
 // one launch of kernel K over the row pairs of nplanes planes and EXTRA blocks
 // past them, or (attr) only its LDS limit
 #define LES_ROW_LAUNCH(SHAPE, K, ...) LES_ROW_LAUNCH_X(SHAPE, 0, K, __VA_ARGS__)
-#define LES_ROW_LAUNCH_X(SHAPE, EXTRA, K, ...)                                                                             \
+#define LES_ROW_LAUNCH_X(SHAPE, EXTRA, K, ...)                                                                    \
   do {                                                                                                            \
     using S_ = SHAPE;                                                                                             \
     if (attr) {                                                                                                   \
@@ -18,7 +18,7 @@
     } else {                                                                                                      \
       const long jobs_ = (long)a.nplanes * (a.ny / 2);                                                            \
       hipLaunchKernelGGL((K), dim3((unsigned)((jobs_ + S_::LB - 1) / S_::LB + (EXTRA)), (unsigned)nf),            \
-                         dim3(S_::THREADS), S_::LDS, s, a, __VA_ARGS__);                                                             \
+                         dim3(S_::THREADS), S_::LDS, s, a, __VA_ARGS__);                                          \
     }                                                                                                             \
   } while (0)
 
@@ -91,6 +91,13 @@ bool rows_trunc_part<LES_T, LES_PART>(bool attr, int n, const RowResArgs<LES_T, 
 }
 
 #if LES_FP32
+template <>
+bool rows_nyq_part<float, LES_PART>(bool attr, int n, const RowR2CArgs<double, float>& a, int nf, const Cplx<float>* tw,
+                                    hipStream_t s) {
+#define X(N) case N: { using SH = NyqShape<float, N>; LES_ROW_LAUNCH(SH, (k_rows_r2c_nyq<float, N>), tw); return true; }
+  LES_ROW_SWITCH(n, X);
+#undef X
+}
 template <>
 bool rows_r2c_part<float, float, LES_PART>(bool attr, int n, const RowR2CArgs<float, float>& a, int nf, const Cplx<float>* tw,
                                            hipStream_t s) {

@@ -45,14 +45,14 @@ static const double KVONK = 0.4;
 // ------------------------------------------------------------------ plans
 struct HostPlan {
   FftPlan p;
-  std::vector<double> re_f, im_f, re_i, im_i;
+  std::vector<double> re_f, im_f;
 };
 
 static bool build_plan(int n, HostPlan& hp, int pool_off, int* used) {
   int a = 0, b = 0, m = n;
   while (m % 2 == 0) { m /= 2; ++a; }
   while (m % 3 == 0) { m /= 3; ++b; }
-  if (m != 1 || n < 2 || n > LES_MAX_N) return false;  // wave-level transforms hold n <= LES_MAX_N points
+  if (m != 1 || n < 2 || n > LES_MAX_N) return false;
   FftPlan& p = hp.p;
   p.n = n;
   p.nst = 0;
@@ -68,19 +68,16 @@ static bool build_plan(int n, HostPlan& hp, int pool_off, int* used) {
     span *= p.R[s];
   }
   int sz = o > 0 ? o : 1;
-  hp.re_f.assign(sz, 0.0); hp.im_f.assign(sz, 0.0); hp.re_i.assign(sz, 0.0); hp.im_i.assign(sz, 0.0);
+  hp.re_f.assign(sz, 0.0); hp.im_f.assign(sz, 0.0);
   for (int s = 0; s < p.nst; ++s)
     for (int r = 1; r < p.R[s]; ++r)
       for (int k = 0; k < p.P[s]; ++k) {
         double ang = TWO_PI * (double)(r * k) / (double)(p.P[s] * p.R[s]);
-        double c = std::cos(ang), sn = std::sin(ang);
         int q = p.off[s] + (r - 1) * p.P[s] + k;
-        hp.re_f[q] = c; hp.im_f[q] = -sn;
-        hp.re_i[q] = c; hp.im_i[q] = sn;
+        hp.re_f[q] = std::cos(ang); hp.im_f[q] = -std::sin(ang);
       }
   p.twf = pool_off;
-  p.twi = pool_off + sz;
-  *used = 2 * sz;
+  *used = sz;
   return true;
 }
 
@@ -146,7 +143,6 @@ static void kt_end(Les& L, int fam, double bytes, const char* base, int ta = 0, 
 
 // ------------------------------------------------------------------ launch helpers
 // Row kernels: one wavefront per row pair, LES_BLOCK / 64 of them per block.
-static const int kWavesPerBlock = LES_BLOCK / LES_WAVE;
 
 template <typename TI, typename T>
 static void rows_r2c(Les& L, const TI* const* src, Cplx<T>* const* dst, int nf, int k0, int npl, T scale, int mode = LOAD_SCALE,
@@ -179,17 +175,13 @@ static void rows_r2c_nyq(Les& L, const double* const* src, Cplx<float>* const* d
   for (int f = 0; f < nf; ++f) { a.src[f] = src[f]; a.dst[f] = dst[f]; }
   a.nx = L.nx; a.ny = L.ny; a.lhx = L.lhx; a.k0 = 0; a.nplanes = npl;
   a.mode = LOAD_SCALE; a.scale = scale; a.div = 1.0f;
-  a.ls = row_line<float>(L.nx);
   a.nyq_as = (long)L.ny * L.nzg;
   a.nyq_ps = (long)(L.ny / 4) * L.nx * L.nzg;
   a.nyq_a = L.nyq_rows + fld * a.nyq_as;
   a.nyq_p = L.nyq_part + fld * a.nyq_ps;
-  const long jobs = (long)npl * (L.ny / 2);
-  assert(L.ny % 8 == 0 && jobs % kWavesPerBlock == 0);
-  const size_t sh = (size_t)kWavesPerBlock * a.ls * sizeof(Cplx<float>) + (size_t)kWavesPerBlock * L.nx * sizeof(double);
+  assert(L.ny % 8 == 0);
   kt_begin(L, KT_ROWS_R2C);
-  hipLaunchKernelGGL(k_rows_r2c_nyq<float>, dim3((unsigned)(jobs / kWavesPerBlock), nf), dim3(LES_BLOCK), sh, L.stream, a, L.px,
-                     twpool<float>(L));
+  rows_nyq_reg<float>(false, L.nx, a, nf, twpool<float>(L) + L.px.twf, L.stream);
   // the field read, its half spectrum written; A (1/nx) and P (1/(8 nx))
   // of a field not counted, as in k_nyq_reduce
   kt_end(L, KT_ROWS_R2C, nf * (double)npl * L.ny * (L.nx * 8.0 + (double)L.lhx * sizeof(Cplx<float>)), "k_rows_r2c_nyq", 4);
@@ -942,6 +934,7 @@ static int setup_kernel_attrs(const Les& L) {
     hipFuncSetAttribute((const void*)k_tridiag_lds, hipFuncAttributeMaxDynamicSharedMemorySize, (int)tri_lds(L.nz));
   const bool ok = setup_fft_attrs<double>(L) && setup_fft_attrs<float>(L) &&
                   rows_r2c_reg<float, float>(true, L.nx, RowR2CArgs<float, float>(), 0, nullptr, 0) &&
+                  rows_nyq_reg<float>(true, L.nx, RowR2CArgs<double, float>(), 0, nullptr, 0) &&
                   rows_c2r_reg<float, float>(true, L.nx, RowC2RArgs<float, float>(), 0, nullptr, 0) &&
                   rows_proj_reg<double>(true, L.nx, RowC2RArgs<double, double>(), ProjEpi3(), 0, nullptr, 0);
   return ok ? 0 : 10;
@@ -1060,10 +1053,7 @@ int les_init(const les_params* p) {
   std::vector<Cplx<float>> t32(off);
   for (int i = 0; i < 4; ++i) {
     int sz = (int)hp[i].re_f.size();
-    for (int q = 0; q < sz; ++q) {
-      t64[hp[i].p.twf + q] = {hp[i].re_f[q], hp[i].im_f[q]};
-      t64[hp[i].p.twi + q] = {hp[i].re_i[q], hp[i].im_i[q]};
-    }
+    for (int q = 0; q < sz; ++q) t64[hp[i].p.twf + q] = {hp[i].re_f[q], hp[i].im_f[q]};
   }
   for (int q = 0; q < off; ++q) t32[q] = {(float)t64[q].x, (float)t64[q].y};
   L->px = hp[0].p; L->py = hp[1].p; L->px2 = hp[2].p; L->py2 = hp[3].p;

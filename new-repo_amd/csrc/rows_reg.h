@@ -105,6 +105,25 @@ struct RowStream {
   }
 };
 
+// The transformed line of a row pair in natural order -> the half spectra of
+// both rows; dst: the block's first row.
+template <typename S, typename T, int N, typename AT>
+__device__ __forceinline__ void row_unpack(const Cplx<T>* line, Cplx<T>* __restrict__ dst, const AT& at) {
+  constexpr int LHX = N / 2 + 1, NT = S::NT;
+  const unsigned doff = (unsigned)(2 * at.dj * LHX + at.a) * (unsigned)sizeof(Cplx<T>);
+#pragma unroll
+  for (int q = 0; q < LHX; q += NT) {
+    const int kk = q + at.a;
+    if (q + NT <= LHX || kk < LHX) {
+      const Cplx<T> zk = lds_ld(line + kk), zm = lds_ld(line + (q == 0 && at.a == 0 ? 0 : N - kk));
+      const Cplx<T> A = {(T)0.5 * (zk.x + zm.x), (T)0.5 * (zk.y - zm.y)};
+      const Cplx<T> B = {(T)0.5 * (zk.y + zm.y), (T)0.5 * (zm.x - zk.x)};
+      put_bytes(dst + q, doff, A);
+      put_bytes(dst + q + LHX, doff, B);
+    }
+  }
+}
+
 // ------------------------------------------------------------------ r2c
 // STREAM: the input is read in RowStream order into LDS (the AB2 predictor and
 // the cleaned pressure, which read three and four FP64 fields per value: 192
@@ -114,7 +133,7 @@ template <typename TI, typename T, int N, int MODE, bool STREAM>
 __global__ void __launch_bounds__((RowShape<T, N>::THREADS)) k_rows_r2c_reg(RowR2CArgs<TI, T> a, const Cplx<T>* __restrict__ tw) {
   using S = RowShape<T, N>;
   using L = typename S::L1;
-  constexpr int LHX = N / 2 + 1, NT = S::NT;
+  constexpr int LHX = N / 2 + 1;
   extern __shared__ __align__(16) unsigned char smem_raw[];
   const RowAt<S> at((long)a.nplanes * (a.ny / 2));
   Cplx<T>* line = reinterpret_cast<Cplx<T>*>(smem_raw) + at.line() * S::LS;
@@ -176,21 +195,98 @@ __global__ void __launch_bounds__((RowShape<T, N>::THREADS)) k_rows_r2c_reg(RowR
   L::template fft<false>(X, line, tw, at.a, sync);
   L::template put<L::LAST>(X, line, at.a);
   sync();
-  if (at.valid) {
-    Cplx<T>* __restrict__ dst = a.dst[f] + row0 * LHX;
-    const unsigned doff = (unsigned)(2 * at.dj * LHX + at.a) * (unsigned)sizeof(Cplx<T>);
+  if (at.valid) row_unpack<S, T, N>(line, a.dst[f] + row0 * LHX, at);
+}
+
+// k_rows_r2c_reg of FP64 fields with the first pass of the mixed mode's FP64
+// Nyquist removal folded into the load (the sums k_nyq_reduce forms, from the
+// values this kernel reads anyway): A_j = sum_i (-1)^i f_ij / nx of both rows
+// (the same lane-strided sums and butterfly as k_nyq_reduce), and per band of
+// 4 row pairs the column partial sum_j (-1)^j f_ij.  A wavefront reads a whole
+// band, 64 consecutive values at a time, and keeps the column partials in
+// registers, the 4 pairs added in order; the lines go to LDS and from there
+// into the transform's layout.  Lengths that divide a wavefront read their own
+// lines and need no block barrier.
+// Needs ny % 8 == 0: a band lies in one plane and is whole.
+// Bound by memory: u, v, w at 128^3 34.5 -> 20.1 us against lines transformed
+// in LDS by one wavefront each, 192x192x64 31.0 -> 18.0, 384x384x64 138 -> 101,
+// 512x256x64 139 -> 102, 256x256x128 89 -> 85 (3.6 TB/s).  Where a block has
+// fewer bands than wavefronts some only wait while the others load (576 points:
+// 52 -> 55 us at 256x64, equal at 512x128).
+template <typename T, int N>
+struct NyqShape {
+  using R = RowShape<T, N>;
+  static constexpr int NT = R::NT, LS = R::LS;
+  static constexpr bool WAVE = R::WAVE;
+  static constexpr int LB = WAVE ? R::LB : 256 / NT >= 4 ? 256 / NT / 4 * 4 : 4;  // whole bands
+  static constexpr int THREADS = (LB * NT + 63) / 64 * 64, LINES = (THREADS + NT - 1) / NT;  // whole wavefronts
+  static constexpr size_t LDS = (size_t)LINES * LS * sizeof(Cplx<T>);
+  static constexpr int VX = R::VX;
+  static_assert(LB % 4 == 0 && (!WAVE || 64 / NT % 4 == 0), "wavefronts hold whole bands");
+};
+
+template <typename T, int N>
+__global__ void __launch_bounds__((NyqShape<T, N>::THREADS)) k_rows_r2c_nyq(RowR2CArgs<double, T> a, const Cplx<T>* __restrict__ tw) {
+  using S = NyqShape<T, N>;
+  using L = typename S::R::L1;
+  constexpr int J = (N + 63) / 64, NW = S::THREADS / 64;
+  // bands of a wavefront: its own lines', else every NW-th
+  constexpr int BW = S::WAVE ? 64 / S::NT / 4 : (S::LB / 4 + NW - 1) / NW;
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  const long njobs = (long)a.nplanes * (a.ny / 2);
+  RowAt<S> at(njobs);
+  at.valid = at.valid && at.line() < S::LB;  // the last lanes may have no line to store
+  Cplx<T>* lines = reinterpret_cast<Cplx<T>*>(smem_raw);
+  Cplx<T>* line = lines + at.line() * S::LS;
+  const int f = blockIdx.y, lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  auto sync = []() LES_INLINE { row_sync<S::WAVE>(); };
+  for (int i = 0; i < BW; ++i) {
+    const int b = S::WAVE ? wave * BW + i : wave + i * NW;
+    const long job = at.job0 + 4 * b;
+    if (b >= S::LB / 4 || job >= njobs) break;
+    const long row0 = (long)a.k0 * a.ny + 2 * job;
+    const double* __restrict__ src = a.src[f] + row0 * N;
+    double acc[J], s[8];
 #pragma unroll
-    for (int q = 0; q < LHX; q += NT) {
-      const int kk = q + at.a;
-      if (q + NT <= LHX || kk < LHX) {
-        const Cplx<T> zk = lds_ld(line + kk), zm = lds_ld(line + (q == 0 && at.a == 0 ? 0 : N - kk));
-        const Cplx<T> A = {(T)0.5 * (zk.x + zm.x), (T)0.5 * (zk.y - zm.y)};
-        const Cplx<T> B = {(T)0.5 * (zk.y + zm.y), (T)0.5 * (zm.x - zk.x)};
-        put_bytes(dst + q, doff, A);
-        put_bytes(dst + q + LHX, doff, B);
+    for (int t = 0; t < 4; ++t) {
+      double s0 = 0.0, s1 = 0.0;
+      Cplx<T>* z = lines + (4 * b + t) * S::LS;
+#pragma unroll
+      for (int j = 0; j < J; ++j) {
+        const int n = lane + 64 * j;
+        if (N % 64 == 0 || n < N) {
+          const double r0 = src[2 * t * N + n], r1 = src[(2 * t + 1) * N + n];
+          s0 += (lane & 1) ? -r0 : r0;
+          s1 += (lane & 1) ? -r1 : r1;
+          acc[j] = t == 0 ? r0 - r1 : acc[j] + (r0 - r1);
+          lds_st(z + n, Cplx<T>{a.scale * (T)r0, a.scale * (T)r1});
+        }
       }
+      s[2 * t] = s0;
+      s[2 * t + 1] = s1;
     }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1)
+#pragma unroll
+      for (int r = 0; r < 8; ++r) s[r] += __shfl_xor(s[r], o, 64);
+    double* __restrict__ A = a.nyq_a + f * a.nyq_as + row0;
+    if (lane == 0) {
+#pragma unroll
+      for (int r = 0; r < 8; ++r) A[r] = s[r] / (double)N;
+    }
+    double* __restrict__ P = a.nyq_p + f * a.nyq_ps + job / 4 * N;
+#pragma unroll
+    for (int j = 0; j < J; ++j)
+      if (N % 64 == 0 || lane + 64 * j < N) P[lane + 64 * j] = acc[j];
   }
+  sync();
+  Cplx<T> X[S::VX];
+  L::template get<0>(X, line, at.a);
+  sync();
+  L::template fft<false>(X, line, tw, at.a, sync);
+  L::template put<L::LAST>(X, line, at.a);
+  sync();
+  if (at.valid) row_unpack<S, T, N>(line, a.dst[f] + ((long)a.k0 * a.ny + 2 * at.job0) * (N / 2 + 1), at);
 }
 
 // ------------------------------------------------------------------ c2r
