@@ -1,5 +1,5 @@
 // Column (y) transforms of the spectral planes, register resident, one
-// instance per length (cols_f32.hip, cols_f64.hip).
+// instance per length (fft_cols.hip).
 //
 // A block owns a tile of CB adjacent columns, counted through the planes (the
 // columns of plane k + 1 follow those of plane k, so only the last tile of
@@ -11,6 +11,11 @@
 //
 // LDS: CB lines of an odd number of values, so that the lanes that share a
 // row (one 128-byte LDS cycle) fall into different banks whatever row it is.
+//
+// Bound by memory from about 128 columns and levels on, below that by the
+// latency of a block's load, exchanges and store.  Against lines that are
+// exchanged in LDS at every stage the column kernels of five steps took 3.01
+// -> 1.08 ms at 192x144x65 in FP64, of five mixed steps at 128^3 1.75 -> 1.46.
 #pragma once
 #include "fft_kernels.h"
 #include "fft_reg.h"

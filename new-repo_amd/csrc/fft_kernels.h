@@ -1,4 +1,5 @@
-// Batched horizontal transform kernels (device code + launch helpers).
+// Arguments and point-wise parts of the batched horizontal transform kernels
+// (rows_reg.h, cols_reg.h, colres_reg.h).
 //
 // Replaces the reference's FFTW/2DECOMP path (src/decomp_2d_fft_2d.f90:397-577
 // r2c_1d_x / c2c_1d_y / c2r_1d_x, src/compute_convective_padd.f90:274-388
@@ -8,12 +9,12 @@
 // Layout: a real field is (nx, ny, planes) with x fastest; a spectral field is
 // (lhx, ny, planes) complex, lhx = nx/2 + 1.  Row kernels take row pairs
 // (j, j+1) of a plane as one complex line z = a + i b; column kernels take a
-// block of CB adjacent kx columns of a plane and transform along y in LDS.
+// block of adjacent kx columns, counted through the planes.
 #pragma once
 #include "les_common.h"
 
 #define LES_BLOCK 256
-// fields a launch takes: the dynamic models filter up to 21 at once, two results each
+// fields a launch takes (the dynamic models filter up to 21 at once, two results each)
 #define LES_MAX_FIELDS 6
 #define LES_R2C_FIELDS 21
 #define LES_C2R_FIELDS 42

@@ -115,7 +115,7 @@ def rocprof_key(name: str) -> str:
 
 
 # kernel-name patterns of the benchmark's kernel families
-FAMILY_KERNELS = {"rows_r2c": r"\bk_rows_r2c_reg<", "rows_c2r": r"\bk_rows_c2r(_div|_proj)?_reg<",
+FAMILY_KERNELS = {"rows_r2c": r"\bk_rows_r2c_(reg|nyq)<", "rows_c2r": r"\bk_rows_c2r(_div|_proj)?_reg<",
                   "cols": r"\bk_cols_reg<", "rows_resample": r"\bk_rows_resample_reg<",
                   "cols_resample": r"\bk_colres_reg<", "tridiag": r"\bk_tridiag",
                   "lagrangian": r"\bk_lagr<"}
