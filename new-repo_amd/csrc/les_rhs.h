@@ -231,7 +231,7 @@ static void convection(Les& L, double* cx, double* cy, double* cz) {
     kt_begin(L, KT_ROWS_RES);
     rows_trunc_reg<T>(false, nx, a, 3, twpool<T>(L) + L.px.twf, twpool<T>(L) + L.px2.twf, L.stream);
     kt_end(L, KT_ROWS_RES, 3.0 * nz * ny * ((double)nx2 * sizeof(T) + (double)nx * 8), "k_rows_resample_reg", sizeof(T),
-           sizeof(T), "truncate");
+           8, "truncate");
   }
 }
 
