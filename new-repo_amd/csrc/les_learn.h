@@ -23,8 +23,8 @@ struct MlpState {
   int ready;
   // training buffers
   long cap;
-  short *h1, *h2, *h3, *dy, *dz[2];
-  float *z1, *z2, *z3, *c, *dzf, *dyf, *part, *lossp;
+  short *h1, *h2, *h3, *dy, *dz[3];
+  float *z1, *z2, *z3, *c, *dyf, *part, *lossp;
   float* csum;     // column sums: 256 per column, of the output layer and the three hidden ones
 };
 
@@ -60,10 +60,10 @@ static int mlp_train_alloc(Les& L, long n) {
   if (n <= M->cap) return 0;
   const long c = n;
   M->h1 = (short*)dalloc(L, 2 * 64 * c); M->h2 = (short*)dalloc(L, 2 * 64 * c); M->h3 = (short*)dalloc(L, 2 * 64 * c);
-  M->dy = (short*)dalloc(L, 2 * 16 * c); M->dz[0] = (short*)dalloc(L, 2 * 64 * c); M->dz[1] = (short*)dalloc(L, 2 * 64 * c);
+  M->dy = (short*)dalloc(L, 2 * 16 * c);
+  for (short*& d : M->dz) d = (short*)dalloc(L, 2 * 64 * c);
   M->z1 = (float*)dalloc(L, 4 * 64 * c); M->z2 = (float*)dalloc(L, 4 * 64 * c); M->z3 = (float*)dalloc(L, 4 * 64 * c);
-  M->c = (float*)dalloc(L, 4 * 16 * c); M->dzf = (float*)dalloc(L, 4 * 64 * c);
-  M->dyf = (float*)dalloc(L, 4 * 16 * c);
+  M->c = (float*)dalloc(L, 4 * 16 * c); M->dyf = (float*)dalloc(L, 4 * 16 * c);
   M->part = (float*)dalloc(L, 4 * (size_t)(c / MLP_KCHUNK + 2) * MLP_NMAT);
   M->csum = (float*)dalloc(L, 4 * (size_t)MLP_SUMS * (16 + 3 * 64));
   M->lossp = (float*)dalloc(L, 4 * (size_t)(16 * c / 256 + 2));
@@ -89,25 +89,21 @@ static void gemm(Les& L, const short* A, long sam, long sak, const short* B, lon
   else hipLaunchKernelGGL((k_gemm_strip<1, STRIP_C>), grid, dim3(256), 0, L.stream, g, h);
 }
 
-// The weight gradients C[M x N] = A[M x K] B[K x N], K the batch, M and N 16
-// or 64: beyond 1024 rows per-wavefront K chunks into slabs of the training
-// workspace (offset off matrix values in each slab set), added to the sums sp
-// that one launch of k_sum_splits forms after the last matrix.
-static void gemm_wgrad(Les& L, const short* A, long sam, const short* B, long sbk, float* C, int M, int N, int K, SumSplits& sp,
-                       int& nm, long& off) {
+// A weight gradient C[M x N] = A[M x K] B[K x N], K the batch, M and N 16 or
+// 64: beyond 1024 rows added to the set gs whose K chunks one launch of
+// k_gemm_kchunk puts into slabs of the training workspace (offset off matrix
+// values in each slab set) and one of k_sum_splits (sp) adds.
+static void gemm_wgrad(Les& L, const short* A, long sam, const short* B, long sbk, float* C, int M, int N, int K, GemmSet& gs,
+                       SumSplits& sp, int& nm, long& off) {
   if (K <= 1024) {
     gemm(L, A, 1, sam, B, sbk, 1, C, M, N, K);
     return;
   }
-  GemmArgs g;
+  GemmArgs& g = gs.g[nm];
   g.A = A; g.sam = 1; g.sak = sam; g.B = B; g.sbk = sbk; g.sbn = 1;
   g.M = M; g.N = N; g.K = K; g.kchunk = MLP_KCHUNK;
   const int nsplit = (K + MLP_KCHUNK - 1) / MLP_KCHUNK;
   g.C = L.mlp->part + off * nsplit;
-  const dim3 grid((unsigned)((nsplit + 3) / 4));
-  if (M == 64 && N == 64) hipLaunchKernelGGL((k_gemm_kchunk<4, 4>), grid, dim3(256), 0, L.stream, g);
-  else if (M == 64) hipLaunchKernelGGL((k_gemm_kchunk<4, 1>), grid, dim3(256), 0, L.stream, g);
-  else hipLaunchKernelGGL((k_gemm_kchunk<1, 4>), grid, dim3(256), 0, L.stream, g);
   sp.part[nm] = g.C; sp.out[nm] = C; sp.n[nm] = M * N; sp.nsplit = nsplit;
   ++nm;
   off += (long)M * N;
@@ -131,35 +127,34 @@ static int mlp_forward_backward(Les& L, const short* X, const float* Y, long n, 
   hipLaunchKernelGGL(k_out_grad, dim3(nb16), dim3(LES_BLOCK), 0, L.stream, M->c, b + MB4, Y, M->dy, M->dyf, M->lossp, n);
   // backward
   float* g = M->g;
+  const short* hin[4] = {X, M->h1, M->h2, M->h3};
+  float* zs[3] = {M->z1, M->z2, M->z3};  // Z, then its gradient
+  const int mw[4] = {MW1, MW2, MW3, MW4};
+  const int mb[4] = {MB1, MB2, MB3, MB4};
+  const int kin[4] = {16, 64, 64, 64};
+  gemm(L, M->dy, 16, 1, M->wb + MW4, 64, 1, nullptr, N, 64, 16, STRIP_BACK, {M->z3, M->z3, M->dz[2]});
+  for (int l = 2; l > 0; --l)
+    gemm(L, M->dz[l], 64, 1, M->wb + mw[l], 64, 1, nullptr, N, 64, 64, STRIP_BACK, {zs[l - 1], zs[l - 1], M->dz[l - 1]});
+  // the gradients of all layers' weights and biases
+  GemmSet gs = {};
   SumSplits sp = {};
-  ColTree ct = {};
+  ColSums cs = {};
   int nm = 0;
   long off = 0;
-  gemm_wgrad(L, M->dy, 16, M->h3, 64, g + MW4, 16, 64, N, sp, nm, off);
-  float* cs = M->csum;
-  hipLaunchKernelGGL(k_colsum_part<16>, dim3(MLP_SUMS * 16 / 64), dim3(64), 0, L.stream, (const float*)M->dyf, cs, n);
-  ct.part[0] = cs; ct.out[0] = g + MLP_NMAT + MB4; ct.w[0] = 16;
-  cs += MLP_SUMS * 16;
-  short* dz = M->dz[0];
-  short* dn = M->dz[1];
-  gemm(L, M->dy, 16, 1, M->wb + MW4, 64, 1, nullptr, N, 64, 16, STRIP_BACK, {M->z3, M->dzf, dz});
-  const short* hin[3] = {X, M->h1, M->h2};
-  const float* zs[2] = {M->z1, M->z2};
-  const int mw[3] = {MW1, MW2, MW3};
-  const int mb[3] = {MB1, MB2, MB3};
-  const int kin[3] = {16, 64, 64};
-  for (int layer = 2; layer >= 0; --layer) {
-    hipLaunchKernelGGL(k_colsum_part<64>, dim3(MLP_SUMS), dim3(64), 0, L.stream, (const float*)M->dzf, cs, n);
-    ct.part[3 - layer] = cs; ct.out[3 - layer] = g + MLP_NMAT + mb[layer]; ct.w[3 - layer] = 64;
-    cs += MLP_SUMS * 64;
-    gemm_wgrad(L, dz, 64, hin[layer], kin[layer], g + mw[layer], 64, kin[layer], N, sp, nm, off);
-    if (layer > 0) {
-      gemm(L, dz, 64, 1, M->wb + mw[layer], kin[layer], 1, nullptr, N, kin[layer], 64, STRIP_BACK, {zs[layer - 1], M->dzf, dn});
-      std::swap(dz, dn);
-    }
+  float* part = M->csum;
+  for (int l = 3; l >= 0; --l) {
+    const int i = 3 - l, w = l == 3 ? 16 : 64;
+    gemm_wgrad(L, l == 3 ? M->dy : M->dz[l], w, hin[l], kin[l], g + mw[l], w, kin[l], N, gs, sp, nm, off);
+    cs.x[i] = l == 3 ? M->dyf : zs[l];
+    cs.part[i] = part; cs.out[i] = g + MLP_NMAT + mb[l]; cs.w[i] = w;
+    part += MLP_SUMS * w;
   }
-  if (nm > 0) hipLaunchKernelGGL(k_sum_splits, dim3(MLP_NMAT / 16), dim3(256), 0, L.stream, sp);
-  hipLaunchKernelGGL(k_colsum_tree, dim3(16 + 3 * 64), dim3(256), 0, L.stream, ct);
+  if (nm > 0) {
+    hipLaunchKernelGGL(k_gemm_kchunk, dim3((unsigned)((sp.nsplit + 3) / 4), (unsigned)nm), dim3(256), 0, L.stream, gs);
+    hipLaunchKernelGGL(k_sum_splits, dim3(MLP_NMAT / 16), dim3(256), 0, L.stream, sp);
+  }
+  hipLaunchKernelGGL(k_colsum_part, dim3(MLP_SUMS * (16 + 3 * 64) / 64), dim3(64), 0, L.stream, cs, n);
+  hipLaunchKernelGGL(k_colsum_tree, dim3(16 + 3 * 64), dim3(256), 0, L.stream, cs);
   if (loss) {
     std::vector<float> lp(nb16);
     LES_CHECK(hipMemcpyAsync(lp.data(), M->lossp, 4 * nb16, hipMemcpyDeviceToHost, L.stream));

@@ -111,7 +111,9 @@ __device__ __forceinline__ s4v load4(const short* p, long stride) {
 // column tiles, reusing its A fragment across them; four wavefronts per
 // block.  What is stored instead of C (C is then not written and read again):
 // STRIP_HIDDEN a hidden layer, Z = C + bias in fp32 and H = gelu(Z) in bf16;
-// STRIP_BACK its gradient, Zf = C gelu'(Z) in fp32 and H the same in bf16.
+// STRIP_BACK its gradient, Zf = C gelu'(Z) in fp32 (in place of Z: a lane
+// writes the values it read) and H the same in bf16.  Z and the bias are loaded
+// before the products, all in flight, as nothing may pass the stores.
 enum { STRIP_C = 0, STRIP_HIDDEN = 1, STRIP_BACK = 2 };
 struct StripOut {
   const float* in;  // bias (hidden), Z (back)
@@ -127,6 +129,13 @@ __global__ void __launch_bounds__(256) k_gemm_strip(GemmArgs g, StripOut h) {
   f4v acc[NT];
 #pragma unroll
   for (int t = 0; t < NT; ++t) acc[t] = f4v{0.f, 0.f, 0.f, 0.f};
+  float in[NT][4];
+  if constexpr (MODE != STRIP_C) {
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) in[t][j] = h.in[(MODE == STRIP_BACK ? (m0 + q + j) * g.N : 0) + 16 * t + r];
+  }
   for (int k = 0; k < g.K; k += 16) {
     const s4v a = load4(g.A + (m0 + r) * g.sam + (long)(k + q) * g.sak, g.sak);
 #pragma unroll
@@ -139,11 +148,11 @@ __global__ void __launch_bounds__(256) k_gemm_strip(GemmArgs g, StripOut h) {
     for (int j = 0; j < 4; ++j) {
       const long o = (m0 + q + j) * g.N + 16 * t + r;
       if constexpr (MODE == STRIP_HIDDEN) {
-        const float z = acc[t][j] + h.in[16 * t + r];
+        const float z = acc[t][j] + in[t][j];
         h.Zf[o] = z;
         h.H[o] = f2bf(gelu(z));
       } else if constexpr (MODE == STRIP_BACK) {
-        const float d = acc[t][j] * gelu_d(h.in[o]);
+        const float d = acc[t][j] * gelu_d(in[t][j]);
         h.Zf[o] = d;
         h.H[o] = f2bf(d);
       } else {
@@ -156,7 +165,7 @@ __global__ void __launch_bounds__(256) k_gemm_strip(GemmArgs g, StripOut h) {
 // the K chunk [w kchunk, (w + 1) kchunk) for every one of the MT x NT
 // output tiles into slab w of C (summed by k_sum_splits).
 template <int MT, int NT>
-__global__ void __launch_bounds__(256) k_gemm_kchunk(GemmArgs g) {
+__device__ __forceinline__ void gemm_kchunk(const GemmArgs& g) {
   const int l = threadIdx.x & 63;
   const long w = (long)blockIdx.x * 4 + (threadIdx.x >> 6);
   const long k0 = w * g.kchunk;
@@ -186,6 +195,19 @@ __global__ void __launch_bounds__(256) k_gemm_kchunk(GemmArgs g) {
     for (int t = 0; t < NT; ++t)
 #pragma unroll
       for (int j = 0; j < 4; ++j) C[(long)(16 * i + q + j) * g.N + 16 * t + r] = acc[i][t][j];
+}
+// The four matrices in one launch (blockIdx.y; M x N 64 x 64, 64 x 16 or
+// 16 x 64): a 65536-row batch is 512 wavefronts a matrix, half of one per SIMD,
+// each a chain of short loads; together they are two per SIMD (this, the column
+// sums in one launch and Z loaded ahead: a training step 267 -> 203 us).
+struct GemmSet {
+  GemmArgs g[4];
+};
+__global__ void __launch_bounds__(256) k_gemm_kchunk(GemmSet s) {
+  const GemmArgs& g = s.g[blockIdx.y];
+  if (g.M == 16) gemm_kchunk<1, 4>(g);
+  else if (g.N == 16) gemm_kchunk<4, 1>(g);
+  else gemm_kchunk<4, 4>(g);
 }
 
 // Sums of the slabs of up to four matrices, out = part[0] + part[1] + ... in
@@ -259,14 +281,19 @@ __global__ void k_out_grad(const float* C, const float* b4, const float* T, shor
 // column, sum t over the rows t, t + 256, ... in order (this kernel, part[t][c]),
 // then the 256 of a column as a tree (k_colsum_tree).  A wavefront takes whole
 // rows (a block per column read one value of every row: 89 us at 65536 x 64,
-// now 9),
-// 16 rows' loads in flight, one wavefront per block so that the 256 (W = 64)
-// spread over the CUs.
+// now 9), 16 rows' loads in flight, one wavefront per block so that the 256
+// (W = 64) spread over the CUs; the four matrices of a step in one launch.
 #define MLP_SUMS 256
+struct ColSums {
+  const float* x[4];  // [n x w]
+  float* part[4];     // [MLP_SUMS x w]
+  float* out[4];
+  int w[4];           // 16 or 64
+};
 template <int W>
-__global__ void __launch_bounds__(64) k_colsum_part(const float* __restrict__ X, float* part, long n) {
+__device__ __forceinline__ void colsum_part(const float* __restrict__ X, float* __restrict__ part, int block, long n) {
   constexpr int U = 16;
-  const int t = (blockIdx.x * 64 + threadIdx.x) / W, c = threadIdx.x % W;
+  const int t = (block * 64 + threadIdx.x) / W, c = threadIdx.x % W;
   const long step = (long)MLP_SUMS * W, full = n / (U * MLP_SUMS) * (U * MLP_SUMS);
   const float* p = X + (long)t * W + c;
   float s = 0.f, x[U];
@@ -291,13 +318,15 @@ __global__ void __launch_bounds__(64) k_colsum_part(const float* __restrict__ X,
   part[t * W + c] = s;
 }
 
-// the tree over each column's 256 sums, one block per column of up to four matrices
-struct ColTree {
-  const float* part[4];
-  float* out[4];
-  int w[4];
-};
-__global__ void __launch_bounds__(256) k_colsum_tree(ColTree a) {
+__global__ void __launch_bounds__(64) k_colsum_part(ColSums a, long n) {
+  int m = 0, b = blockIdx.x;
+  while (b >= MLP_SUMS * a.w[m] / 64) b -= MLP_SUMS * a.w[m++] / 64;
+  if (a.w[m] == 16) colsum_part<16>(a.x[m], a.part[m], b, n);
+  else colsum_part<64>(a.x[m], a.part[m], b, n);
+}
+
+// the tree over each column's 256 sums, one block per column of the four matrices
+__global__ void __launch_bounds__(256) k_colsum_tree(ColSums a) {
   __shared__ float red[MLP_SUMS];
   int m = 0, c = blockIdx.x;
   while (c >= a.w[m]) c -= a.w[m++];
