@@ -90,9 +90,9 @@ static void gemm(Les& L, const short* A, long sam, long sak, const short* B, lon
 }
 
 // A weight gradient C[M x N] = A[M x K] B[K x N], K the batch, M and N 16 or
-// 64: beyond 1024 rows added to the set gs whose K chunks one launch of
-// k_gemm_kchunk puts into slabs of the training workspace (offset off matrix
-// values in each slab set) and one of k_sum_splits (sp) adds.
+// 64: beyond 1024 rows added to the set gs whose K chunks k_wgrad_parts puts
+// into slabs of the training workspace (offset off matrix values in each slab
+// set) and k_wgrad_sums adds (sp).
 static void gemm_wgrad(Les& L, const short* A, long sam, const short* B, long sbk, float* C, int M, int N, int K, GemmSet& gs,
                        SumSplits& sp, int& nm, long& off) {
   if (K <= 1024) {
@@ -149,12 +149,10 @@ static int mlp_forward_backward(Les& L, const short* X, const float* Y, long n, 
     cs.part[i] = part; cs.out[i] = g + MLP_NMAT + mb[l]; cs.w[i] = w;
     part += MLP_SUMS * w;
   }
-  if (nm > 0) {
-    hipLaunchKernelGGL(k_gemm_kchunk, dim3((unsigned)((sp.nsplit + 3) / 4), (unsigned)nm), dim3(256), 0, L.stream, gs);
-    hipLaunchKernelGGL(k_sum_splits, dim3(MLP_NMAT / 16), dim3(256), 0, L.stream, sp);
-  }
-  hipLaunchKernelGGL(k_colsum_part, dim3(MLP_SUMS * (16 + 3 * 64) / 64), dim3(64), 0, L.stream, cs, n);
-  hipLaunchKernelGGL(k_colsum_tree, dim3(16 + 3 * 64), dim3(256), 0, L.stream, cs);
+  const int gb = (sp.nsplit + 3) / 4, sb = nm > 0 ? MLP_NMAT / 16 : 0;
+  hipLaunchKernelGGL(k_wgrad_parts, dim3((unsigned)(nm * gb + MLP_SUMS * (16 + 3 * 64) / 256)), dim3(256), 0, L.stream, gs, nm,
+                     gb, cs, n);
+  hipLaunchKernelGGL(k_wgrad_sums, dim3((unsigned)(sb + 16 + 3 * 64)), dim3(256), 0, L.stream, sp, sb, cs);
   if (loss) {
     std::vector<float> lp(nb16);
     LES_CHECK(hipMemcpyAsync(lp.data(), M->lossp, 4 * nb16, hipMemcpyDeviceToHost, L.stream));

@@ -163,11 +163,11 @@ __global__ void __launch_bounds__(256) k_gemm_strip(GemmArgs g, StripOut h) {
 
 // The weight-gradient GEMMs (M, N <= 64, K = the batch): wavefront w sums
 // the K chunk [w kchunk, (w + 1) kchunk) for every one of the MT x NT
-// output tiles into slab w of C (summed by k_sum_splits).
+// output tiles into slab w of C (added by sum_splits).
 template <int MT, int NT>
-__device__ __forceinline__ void gemm_kchunk(const GemmArgs& g) {
+__device__ __forceinline__ void gemm_kchunk(const GemmArgs& g, int block) {
   const int l = threadIdx.x & 63;
-  const long w = (long)blockIdx.x * 4 + (threadIdx.x >> 6);
+  const long w = (long)block * 4 + (threadIdx.x >> 6);
   const long k0 = w * g.kchunk;
   if (k0 >= g.K) return;
   const long k1 = k0 + g.kchunk < g.K ? k0 + g.kchunk : g.K;
@@ -196,20 +196,6 @@ __device__ __forceinline__ void gemm_kchunk(const GemmArgs& g) {
 #pragma unroll
       for (int j = 0; j < 4; ++j) C[(long)(16 * i + q + j) * g.N + 16 * t + r] = acc[i][t][j];
 }
-// The four matrices in one launch (blockIdx.y; M x N 64 x 64, 64 x 16 or
-// 16 x 64): a 65536-row batch is 512 wavefronts a matrix, half of one per SIMD,
-// each a chain of short loads; together they are two per SIMD (this, the column
-// sums in one launch and Z loaded ahead: a training step 267 -> 203 us).
-struct GemmSet {
-  GemmArgs g[4];
-};
-__global__ void __launch_bounds__(256) k_gemm_kchunk(GemmSet s) {
-  const GemmArgs& g = s.g[blockIdx.y];
-  if (g.M == 16) gemm_kchunk<1, 4>(g);
-  else if (g.N == 16) gemm_kchunk<4, 1>(g);
-  else gemm_kchunk<4, 4>(g);
-}
-
 // Sums of the slabs of up to four matrices, out = part[0] + part[1] + ... in
 // order, each output one running fp32 sum.  A block sums 16 outputs: its 256
 // threads stage 256 slabs of them in LDS at a time, 16 of them then add from
@@ -222,8 +208,7 @@ struct SumSplits {
   int n[4];  // outputs of each matrix, multiples of 16
   int nsplit;
 };
-__global__ void __launch_bounds__(256) k_sum_splits(SumSplits a) {
-  __shared__ float buf[256 * 16];
+__device__ __forceinline__ void sum_splits(const SumSplits& a, float* buf) {
   int m = 0, o0 = blockIdx.x * 16;
   while (o0 >= a.n[m]) o0 -= a.n[m++];
   const float* __restrict__ p = a.part[m] + o0;
@@ -278,11 +263,10 @@ __global__ void k_out_grad(const float* C, const float* b4, const float* T, shor
 }
 
 // Column sums (bias gradients) of a [n x W] fp32 matrix: 256 running sums per
-// column, sum t over the rows t, t + 256, ... in order (this kernel, part[t][c]),
-// then the 256 of a column as a tree (k_colsum_tree).  A wavefront takes whole
+// column, sum t over the rows t, t + 256, ... in order (here, part[t][c]),
+// then the 256 of a column as a tree (colsum_tree).  A wavefront takes whole
 // rows (a block per column read one value of every row: 89 us at 65536 x 64,
-// now 9), 16 rows' loads in flight, one wavefront per block so that the 256
-// (W = 64) spread over the CUs; the four matrices of a step in one launch.
+// now 9), 16 rows' loads in flight.
 #define MLP_SUMS 256
 struct ColSums {
   const float* x[4];  // [n x w]
@@ -291,9 +275,9 @@ struct ColSums {
   int w[4];           // 16 or 64
 };
 template <int W>
-__device__ __forceinline__ void colsum_part(const float* __restrict__ X, float* __restrict__ part, int block, long n) {
+__device__ __forceinline__ void colsum_part(const float* __restrict__ X, float* __restrict__ part, int wave, long n) {
   constexpr int U = 16;
-  const int t = (block * 64 + threadIdx.x) / W, c = threadIdx.x % W;
+  const int t = (wave * 64 + (threadIdx.x & 63)) / W, c = threadIdx.x % W;
   const long step = (long)MLP_SUMS * W, full = n / (U * MLP_SUMS) * (U * MLP_SUMS);
   const float* p = X + (long)t * W + c;
   float s = 0.f, x[U];
@@ -318,17 +302,9 @@ __device__ __forceinline__ void colsum_part(const float* __restrict__ X, float* 
   part[t * W + c] = s;
 }
 
-__global__ void __launch_bounds__(64) k_colsum_part(ColSums a, long n) {
-  int m = 0, b = blockIdx.x;
-  while (b >= MLP_SUMS * a.w[m] / 64) b -= MLP_SUMS * a.w[m++] / 64;
-  if (a.w[m] == 16) colsum_part<16>(a.x[m], a.part[m], b, n);
-  else colsum_part<64>(a.x[m], a.part[m], b, n);
-}
-
 // the tree over each column's 256 sums, one block per column of the four matrices
-__global__ void __launch_bounds__(256) k_colsum_tree(ColSums a) {
-  __shared__ float red[MLP_SUMS];
-  int m = 0, c = blockIdx.x;
+__device__ __forceinline__ void colsum_tree(const ColSums& a, int block, float* red) {
+  int m = 0, c = block;
   while (c >= a.w[m]) c -= a.w[m++];
   red[threadIdx.x] = a.part[m][threadIdx.x * a.w[m] + c];
   __syncthreads();
@@ -337,6 +313,37 @@ __global__ void __launch_bounds__(256) k_colsum_tree(ColSums a) {
     __syncthreads();
   }
   if (threadIdx.x == 0) a.out[m][c] = red[0];
+}
+
+// The gradients of all weights and biases from the layers' gradients, in two
+// launches: first the K chunks of the weight matrices (gb blocks each; M x N
+// 64 x 64, 64 x 16 or 16 x 64) and, in the blocks after them, the bias sums;
+// then the slabs' sums (sb blocks) and the trees.  A 65536-row batch is 512
+// wavefronts a weight matrix and 832 for the biases, each a chain of short
+// loads: a launch of its own for each is half of one wavefront per SIMD or
+// less.  Training step at that size: 267 us with a launch for each, 203 with the
+// weights in one and the biases in another, 193 with both side by side.
+struct GemmSet {
+  GemmArgs g[4];
+};
+__global__ void __launch_bounds__(256) k_wgrad_parts(GemmSet s, int nm, int gb, ColSums a, long n) {
+  if ((int)blockIdx.x < nm * gb) {
+    const int m = blockIdx.x / gb, block = blockIdx.x - m * gb;
+    const GemmArgs& g = s.g[m];
+    if (g.M == 16) gemm_kchunk<1, 4>(g, block);
+    else if (g.N == 16) gemm_kchunk<4, 1>(g, block);
+    else gemm_kchunk<4, 4>(g, block);
+    return;
+  }
+  int m = 0, b = __builtin_amdgcn_readfirstlane((blockIdx.x - nm * gb) * 4 + (threadIdx.x >> 6));
+  while (b >= MLP_SUMS * a.w[m] / 64) b -= MLP_SUMS * a.w[m++] / 64;
+  if (a.w[m] == 16) colsum_part<16>(a.x[m], a.part[m], b, n);
+  else colsum_part<64>(a.x[m], a.part[m], b, n);
+}
+__global__ void __launch_bounds__(256) k_wgrad_sums(SumSplits sp, int sb, ColSums a) {
+  __shared__ float buf[256 * 16];
+  if ((int)blockIdx.x < sb) sum_splits(sp, buf);
+  else colsum_tree(a, blockIdx.x - sb, buf);
 }
 
 // Adam on the fp32 master parameters; refreshes the bf16 matrix mirror
