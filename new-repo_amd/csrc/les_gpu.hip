@@ -9,6 +9,7 @@
 // replaced by strided column passes and by index arithmetic inside kernels.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cassert>
 #include <cmath>
 #include <cstdarg>
@@ -82,16 +83,49 @@ static bool build_plan(int n, HostPlan& hp, int pool_off, int* used) {
 }
 
 // ------------------------------------------------------------------ memory
-static void* dalloc(Les& L, size_t bytes) {
+static void* dalloc_try(Les& L, size_t bytes) {
   void* p = nullptr;
   if (bytes == 0) bytes = 8;
   if (hipMalloc(&p, bytes) != hipSuccess) {
-    L.alloc_failed = 1;
+    (void)hipGetLastError();  // reported by the caller, not by a later call's check
     return nullptr;
   }
   hipMemset(p, 0, bytes);
   L.allocs.push_back(p);
   return p;
+}
+static void* dalloc(Les& L, size_t bytes) {
+  void* p = dalloc_try(L, bytes);
+  if (!p) L.alloc_failed = 1;
+  return p;
+}
+
+// Buffers that are obtained after les_init, together: all of them or none.
+// What a failed call had obtained is given back and its pointers are null, so
+// that a caller may try again (with less) and nothing runs on half of a set.
+struct DevBuf {
+  void** p;
+  size_t bytes;
+};
+template <typename T>
+static DevBuf dbuf(T*& p, size_t n) { return DevBuf{(void**)&p, sizeof(T) * n}; }
+static void dfree_all(Les& L, const std::vector<DevBuf>& set) {
+  for (const DevBuf& b : set) {
+    if (!*b.p) continue;
+    L.allocs.erase(std::find(L.allocs.begin(), L.allocs.end(), *b.p));
+    hipFree(*b.p);  // waits for the kernels that may still use it
+    *b.p = nullptr;
+  }
+}
+static bool dalloc_all(Les& L, const std::vector<DevBuf>& set) {
+  for (const DevBuf& b : set) {
+    *b.p = dalloc_try(L, b.bytes);
+    if (!*b.p) {
+      dfree_all(L, set);
+      return false;
+    }
+  }
+  return true;
 }
 
 static bool field_is_fp64(int id) {

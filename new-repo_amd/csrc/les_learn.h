@@ -28,47 +28,43 @@ struct MlpState {
   float* csum;     // column sums: 256 per column, of the output layer and the three hidden ones
 };
 
-static void* dalloc(Les& L, size_t bytes);
-
 static int mlp_alloc(Les& L) {
   if (L.mlp) return 0;
   MlpState* M = new MlpState();
   std::memset((void*)M, 0, sizeof(MlpState));
-  M->w = (float*)dalloc(L, 4 * MLP_NPAR);
-  M->wb = (short*)dalloc(L, 2 * MLP_NMAT);
-  M->m = (float*)dalloc(L, 4 * MLP_NPAR);
-  M->v = (float*)dalloc(L, 4 * MLP_NPAR);
-  M->g = (float*)dalloc(L, 4 * MLP_NPAR);
-  M->norm = (float*)dalloc(L, 4 * 32);
   const long npt = L.np * (L.nz + 1);
-  M->X = (short*)dalloc(L, 2 * 16 * (size_t)npt);
-  for (int i = 0; i < 21; ++i) M->fr[i] = (float*)dalloc(L, 4 * (size_t)L.nf);
   M->nb = L.filt_batch >= 7 ? 9 : 3;  // small grids: the nine filtered fields in one launch
-  for (int i = 0; i < 3 * M->nb; ++i) M->fs[i] = dalloc(L, 2 * 4 * (size_t)L.nsp);
   M->redn = 2 * (long)nblk(npt) + 64;
-  M->red = (double*)dalloc(L, 8 * (size_t)M->redn);
+  std::vector<DevBuf> set = {dbuf(M->w, MLP_NPAR), dbuf(M->wb, MLP_NMAT), dbuf(M->m, MLP_NPAR), dbuf(M->v, MLP_NPAR),
+                             dbuf(M->g, MLP_NPAR), dbuf(M->norm, 32), dbuf(M->X, 16 * (size_t)npt), dbuf(M->red, M->redn)};
+  for (float*& f : M->fr) set.push_back(dbuf(f, L.nf));
+  for (int i = 0; i < 3 * M->nb; ++i) set.push_back(DevBuf{&M->fs[i], 2 * 4 * (size_t)L.nsp});
+  if (!dalloc_all(L, set)) {
+    delete M;
+    les_set_error("out of memory (MLP)");
+    return 3;
+  }
   L.mlp = M;
-  if (L.alloc_failed) { les_set_error("out of memory (MLP)"); return 3; }
   return 0;
 }
 
 // K chunk of one wavefront in the weight-gradient GEMMs
 #define MLP_KCHUNK 128
 
+// Training buffers for n points: a larger batch takes the place of the smaller
+// one's buffers; cap is the batch that all of them are there for.
 static int mlp_train_alloc(Les& L, long n) {
   MlpState* M = L.mlp;
   if (n <= M->cap) return 0;
-  const long c = n;
-  M->h1 = (short*)dalloc(L, 2 * 64 * c); M->h2 = (short*)dalloc(L, 2 * 64 * c); M->h3 = (short*)dalloc(L, 2 * 64 * c);
-  M->dy = (short*)dalloc(L, 2 * 16 * c);
-  for (short*& d : M->dz) d = (short*)dalloc(L, 2 * 64 * c);
-  M->z1 = (float*)dalloc(L, 4 * 64 * c); M->z2 = (float*)dalloc(L, 4 * 64 * c); M->z3 = (float*)dalloc(L, 4 * 64 * c);
-  M->c = (float*)dalloc(L, 4 * 16 * c); M->dyf = (float*)dalloc(L, 4 * 16 * c);
-  M->part = (float*)dalloc(L, 4 * (size_t)(c / MLP_KCHUNK + 2) * MLP_NMAT);
-  M->csum = (float*)dalloc(L, 4 * (size_t)MLP_SUMS * (16 + 3 * 64));
-  M->lossp = (float*)dalloc(L, 4 * (size_t)(16 * c / 256 + 2));
-  M->cap = c;
-  if (L.alloc_failed) { les_set_error("out of memory (MLP training)"); return 3; }
+  std::vector<DevBuf> set = {dbuf(M->h1, 64 * n), dbuf(M->h2, 64 * n), dbuf(M->h3, 64 * n), dbuf(M->dy, 16 * n),
+                             dbuf(M->z1, 64 * n), dbuf(M->z2, 64 * n), dbuf(M->z3, 64 * n), dbuf(M->c, 16 * n),
+                             dbuf(M->dyf, 16 * n), dbuf(M->part, (n / MLP_KCHUNK + 2) * MLP_NMAT),
+                             dbuf(M->csum, MLP_SUMS * (16 + 3 * 64)), dbuf(M->lossp, 16 * n / 256 + 2)};
+  for (short*& d : M->dz) set.push_back(dbuf(d, 64 * n));
+  M->cap = 0;
+  dfree_all(L, set);
+  if (!dalloc_all(L, set)) { les_set_error("out of memory (MLP training)"); return 3; }
+  M->cap = n;
   return 0;
 }
 
