@@ -1697,15 +1697,11 @@ extern "C" {
 int les_stat_init(void) {
   Les* L = g_les;
   if (!L) return 1;
-  if (!L->st_sum) {
-    L->st_sum = (double*)dalloc(*L, sizeof(double) * LES_NSTAT * (size_t)L->np * L->nz);
-    L->st_ustar = (double*)dalloc(*L, sizeof(double) * L->np);
-    L->st_part = (double*)dalloc(*L, sizeof(double) * (size_t)L->nz * LES_PROF_SLICES * PS_N);
-    L->st_prof = (double*)dalloc(*L, sizeof(double) * (size_t)LES_NPROF * L->nz);
-    if (!L->st_sum || !L->st_ustar || !L->st_part || !L->st_prof) {
-      les_set_error("Out of memory when initialising io module variables");
-      return 3;
-    }
+  if (!L->st_sum && !dalloc_all(*L, {dbuf(L->st_sum, LES_NSTAT * (size_t)L->np * L->nz), dbuf(L->st_ustar, L->np),
+                                     dbuf(L->st_part, (size_t)L->nz * LES_PROF_SLICES * PS_N),
+                                     dbuf(L->st_prof, (size_t)LES_NPROF * L->nz)})) {
+    les_set_error("Out of memory when initialising io module variables");
+    return 3;
   }
   stat_zero(*L);
   LES_CHECK(hipGetLastError());
@@ -1723,18 +1719,12 @@ int les_set_geostrophic(double ug, double vg) {
 int les_tke_init(void) {
   Les* L = g_les;
   if (!L) return 1;
-  if (!L->tk_sum) {
-    L->tk_sum = (double*)dalloc(*L, sizeof(double) * LES_NTKE * (size_t)L->nz);
-    L->tk_part = (double*)dalloc(*L, sizeof(double) * (size_t)L->nz * LES_TKE_SLICES * LES_NTKE);
-    L->tk_pf = (double*)dalloc(*L, sizeof(double) * L->nf);
-    L->tk_px = (double*)dalloc(*L, sizeof(double) * L->nf);
-    L->tk_py = (double*)dalloc(*L, sizeof(double) * L->nf);
-    for (int i = 0; i < 3; ++i) L->tk_spec[i] = (double*)dalloc(*L, 2 * sizeof(double) * L->nsp);
-    if (!L->tk_sum || !L->tk_part || !L->tk_pf || !L->tk_px || !L->tk_py || !L->tk_spec[0] || !L->tk_spec[1] ||
-        !L->tk_spec[2]) {
-      les_set_error("Out of memory when initialising the tke budget");
-      return 3;
-    }
+  if (!L->tk_sum &&
+      !dalloc_all(*L, {dbuf(L->tk_sum, LES_NTKE * (size_t)L->nz), dbuf(L->tk_part, (size_t)L->nz * LES_TKE_SLICES * LES_NTKE),
+                       dbuf(L->tk_pf, L->nf), dbuf(L->tk_px, L->nf), dbuf(L->tk_py, L->nf), dbuf(L->tk_spec[0], 2 * L->nsp),
+                       dbuf(L->tk_spec[1], 2 * L->nsp), dbuf(L->tk_spec[2], 2 * L->nsp)})) {
+    les_set_error("Out of memory when initialising the tke budget");
+    return 3;
   }
   return les_tke_reset();
 }

@@ -84,3 +84,31 @@ print(json.dumps(dict(buffers=buffers, res=res, live=rt.live, bad=rt.bad)))
     assert out["buffers"] > 20 and out["live"] == 0 and out["bad"] == 0
     for r in out["res"]:
         assert r == [3, 0, 1, 0, out["buffers"]]
+
+
+def test_statistics_and_tke_budget_after_a_failed_allocation():
+    out = host_run("""
+prm = P.LesParams(nx=16, ny=16, nz=8)
+res = []
+for name, use in (("les_stat_init", "les_stat_accumulate"), ("les_tke_init", "les_tke_accumulate")):
+    g = pkg.LesGpu(prm)
+    init, call = getattr(g.lib, name), getattr(g.lib, use)
+    base = rt.live
+    assert init() == 0
+    buffers = rt.live - base
+    assert init() == 0 and rt.live == base + buffers  # a second call only clears
+    g.close()
+    for k in range(1, buffers + 1):
+        g = pkg.LesGpu(prm)
+        base = rt.live
+        rt.fail_at = k
+        rc, left = init(), rt.live - base
+        rt.fail_at = 0
+        early, again, got = call(), init(), rt.live - base - buffers
+        g.close()
+        res.append([rc, left, early, again, got])
+print(json.dumps(dict(res=res, live=rt.live, bad=rt.bad)))
+""")
+    assert len(out["res"]) == 4 + 8 and out["live"] == 0 and out["bad"] == 0
+    for r in out["res"]:
+        assert r == [3, 0, 1, 0, 0]
