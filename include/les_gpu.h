@@ -9,10 +9,11 @@
  *   0 ok, 1 invalid option/model, 3 out of memory, 4 double initialisation,
  *   5 HIP runtime error, 9 NaN found / singular solve, 10 bad shape or id.
  * Calls come from one host thread; every entry point runs its kernels on the
- * default (null) HIP stream (les_step also uses side streams inside a step, joined
- * before it returns, see les_set_overlap); host buffers are synchronised only
- * by download/status calls.  Not reentrant,
- * like the reference's module state.
+ * device of les_init, on a blocking HIP stream of the library's own or on the
+ * default stream (les_set_default_stream; les_step also uses side streams
+ * inside a step, joined by events before its last kernels, see
+ * les_set_overlap); host buffers are synchronised only by download/status
+ * calls.  Not reentrant, like the reference's module state.
  *
  * Sizes: nx, ny multiples of 4 of the form 2^a 3^b with 3 nx / 2, 3 ny / 2 <= 1024
  * (every transform is held by one wavefront); nz >= 3.
@@ -127,6 +128,14 @@ int les_kernel_stat(int i, int* count, char* name, int name_cap, double* v);
  * step on one stream.  Results are the same either way.  The per-kernel
  * timing mode always uses one stream. */
 int les_set_overlap(int on);
+/* Which stream calls run on (no counterpart in the reference): 0 (after
+ * les_init) a blocking stream of the library's own, 1 the default (null) stream
+ * of the device.  Both are ordered with the caller's default-stream work.  With
+ * 1 the host does not wait where the two meet, which it does at every change
+ * between default-stream work and a blocking stream; with 0 the caller's other
+ * blocking streams run beside the library's kernels, and single launches cost
+ * less.  Waits for the work queued so far. */
+int les_set_default_stream(int on);
 
 /* --- operator-level entry points (the compute_* module procedures) -------- */
 /* obukhov + wallstress (src/compute_wall_law.f90:107-254). */

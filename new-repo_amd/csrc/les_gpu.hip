@@ -2,7 +2,7 @@
 // driver and the C-ABI declared in include/les_gpu.h.
 //
 // One LES time step of the reference (src/LES_engine.f90:189-353) runs as a
-// sequence of kernels on the default HIP stream (les_step puts the SGS stage
+// sequence of kernels on the library's HIP stream (les_step puts the SGS stage
 // on a second stream beside the convection); the whole domain is resident in
 // HBM.
 // The 2DECOMP pencil transposes and MPI halo exchanges of the reference are
@@ -988,6 +988,7 @@ static void free_all(Les* L) {
   hipEventDestroy(L->ev_feat1);
   hipStreamDestroy(L->stream3);
   hipStreamDestroy(L->stream2);
+  hipStreamDestroy(L->own_stream);
 }
 
 extern "C" {
@@ -1041,21 +1042,25 @@ int les_init(const les_params* p) {
   L->overlap = LES_OVERLAP;
   L->F_coeff_init = P.lagran_init != 0;
   L->mixed = P.precision != 0;
-  // The library's stream is the default (null) stream: a program that hands
-  // device pointers to other default-stream work (a restore or a diagnostic in
-  // torch between two calls) stays ordered without the runtime's wait between
-  // the null stream and a blocking stream of our own, which cost the host about
-  // 1 ms at each change of stream (64^3 FP64, five steps after a restore: 2.76
-  // -> 1.92 ms; 256^3 mixed 28.6 -> 27.7).  The side streams are joined to it by
-  // events only, so they need no implicit ordering with it.
-  L->stream = nullptr;
+  // A blocking stream of the library's own: ordered with default-stream work by
+  // the runtime, free to run beside a caller's other streams, and of this device
+  // whatever device is current later.  The side streams are joined to it by
+  // events only, so they need no implicit ordering with anything.
+  if (hipStreamCreate(&L->own_stream) != hipSuccess) {
+    delete L;
+    les_set_error("stream");
+    return 5;
+  }
+  L->stream = L->own_stream;
   if (hipStreamCreateWithFlags(&L->stream2, hipStreamNonBlocking) != hipSuccess) {
+    hipStreamDestroy(L->own_stream);
     delete L;
     les_set_error("stream");
     return 5;
   }
   if (hipStreamCreateWithFlags(&L->stream3, hipStreamNonBlocking) != hipSuccess) {
     hipStreamDestroy(L->stream2);
+    hipStreamDestroy(L->own_stream);
     delete L;
     les_set_error("stream");
     return 5;
@@ -1235,25 +1240,28 @@ int les_init(const les_params* p) {
 }
 
 int les_finalize(void) {
-  if (!g_les) return 0;
-  hipStreamSynchronize(g_les->stream);
-  free_all(g_les);
-  g_les->allocs.~vector();
-  ::operator delete((void*)g_les);
+  LES_ENTER(L);
+  if (!L) return 0;
+  hipStreamSynchronize(L->stream);
+  free_all(L);
+  L->allocs.~vector();
+  ::operator delete((void*)L);
   g_les = nullptr;
   return 0;
 }
 
 int les_sync(void) {
-  if (!g_les) return 1;
-  LES_CHECK(hipStreamSynchronize(g_les->stream));
+  LES_ENTER(L);
+  if (!L) return 1;
+  LES_CHECK(hipStreamSynchronize(L->stream));
   return 0;
 }
 
 int les_jt_total(void) { return g_les ? g_les->jt_total : -1; }
 int les_set_jt_total(int jt) {
-  if (!g_les) return 1;
-  g_les->jt_total = jt;
+  LES_ENTER(L);
+  if (!L) return 1;
+  L->jt_total = jt;
   return 0;
 }
 
@@ -1268,7 +1276,7 @@ __global__ void k_cvt_f2d(const float* a, double* b, long n) {
 }
 
 static int copy_field(int id, double* host, int up) {
-  Les* L = g_les;
+  LES_ENTER(L);
   if (!L) { les_set_error("not initialised"); return 1; }
   if (id < 0 || id >= LES_NFIELDS) { les_set_error("bad field id %d", id); return 10; }
   // the step leaves the pressure gradient to be formed on request
@@ -1297,19 +1305,20 @@ int les_upload_field(int id, const double* host) { return copy_field(id, (double
 int les_download_field(int id, double* host) { return copy_field(id, host, 0); }
 
 int les_field_ptr(int id, void** dptr, int* elem_bytes) {
-  if (!g_les) return 1;
+  LES_ENTER(L);
+  if (!L) return 1;
   if (id < 0 || id >= LES_NFIELDS) return 10;
   if (id == LES_DPDX || id == LES_DPDY || id == LES_DPDZ || id == LES_P) {
-    refresh_gradp(*g_les);
-    LES_CHECK(hipStreamSynchronize(g_les->stream));
+    refresh_gradp(*L);
+    LES_CHECK(hipStreamSynchronize(L->stream));
   }
-  *dptr = g_les->f[id];
-  *elem_bytes = g_les->fbytes[id];
+  *dptr = L->f[id];
+  *elem_bytes = L->fbytes[id];
   return 0;
 }
 
 int les_upload_layer(int id, const double* host) {
-  Les* L = g_les;
+  LES_ENTER(L);
   if (!L) return 1;
   if (id < 0 || id >= LES_NLAYERS) return 10;
   LES_CHECK(hipMemcpy(L->layer[id], host, 8 * L->np, hipMemcpyHostToDevice));
@@ -1323,7 +1332,7 @@ int les_upload_layer(int id, const double* host) {
 }
 
 int les_download_layer(int id, double* host) {
-  Les* L = g_les;
+  LES_ENTER(L);
   if (!L) return 1;
   if (id < 0 || id >= LES_NLAYERS) return 10;
   LES_CHECK(hipStreamSynchronize(L->stream));
@@ -1332,7 +1341,7 @@ int les_download_layer(int id, double* host) {
 }
 
 int les_set_ic(const double* u0, const double* v0, const double* w0) {
-  Les* L = g_les;
+  LES_ENTER(L);
   if (!L) return 1;
   std::vector<double> h(L->nf, 0.0);
   const double* src[3] = {u0, v0, w0};
@@ -1355,7 +1364,7 @@ int les_set_ic(const double* u0, const double* v0, const double* w0) {
 }
 
 int les_step(int nsteps) {
-  Les* L = g_les;
+  LES_ENTER(L);
   if (!L) { les_set_error("not initialised"); return 1; }
   for (int s = 0; s < nsteps; ++s) {
     int rc = L->mixed ? les_step_t<float>(*L) : les_step_t<double>(*L);
@@ -1366,7 +1375,7 @@ int les_step(int nsteps) {
 }
 
 int les_check_nan(int* found) {
-  Les* L = g_les;
+  LES_ENTER(L);
   if (!L) return 1;
   LES_CHECK(hipMemsetAsync(L->nanflag, 0, 4, L->stream));
   NanArgs a;
@@ -1382,7 +1391,7 @@ int les_check_nan(int* found) {
 }
 
 int les_timers(double* t, int reset) {
-  Les* L = g_les;
+  LES_ENTER(L);
   if (!L) return 1;
   if (t) {
     for (int i = 0; i < 5; ++i) t[i] = L->phase_ms[i];
@@ -1401,7 +1410,7 @@ int les_timers(double* t, int reset) {
 }
 
 int les_kernel_stat(int i, int* count, char* name, int name_cap, double* v) {
-  Les* L = g_les;
+  LES_ENTER(L);
   if (!L) return 1;
   if (count) *count = L->nkst;
   if (i < 0 && !name && !v) return 0;
@@ -1424,58 +1433,74 @@ int les_kernel_stat(int i, int* count, char* name, int name_cap, double* v) {
 }
 
 int les_set_timing(int on) {
-  if (!g_les) return 1;
-  g_les->timing = on;
+  LES_ENTER(L);
+  if (!L) return 1;
+  L->timing = on;
+  return 0;
+}
+
+int les_set_default_stream(int on) {
+  LES_ENTER(L);
+  if (!L) return 1;
+  LES_CHECK(hipStreamSynchronize(L->stream));
+  L->stream = on ? nullptr : L->own_stream;
   return 0;
 }
 
 int les_set_overlap(int on) {
-  if (!g_les) return 1;
-  g_les->overlap = on ? 1 : 0;
+  LES_ENTER(L);
+  if (!L) return 1;
+  L->overlap = on ? 1 : 0;
   return 0;
 }
 
 // ---- operator-level entry points
 int les_wall_law(void) {
-  if (!g_les) return 1;
-  if (g_les->mixed) wall_law<float>(*g_les); else wall_law<double>(*g_les);
+  LES_ENTER(L);
+  if (!L) return 1;
+  if (L->mixed) wall_law<float>(*L); else wall_law<double>(*L);
   LES_CHECK(hipGetLastError());
   return 0;
 }
 int les_compute_vel_grad(void) {
-  if (!g_les) return 1;
-  if (g_les->mixed) compute_vel_grad<float>(*g_les); else compute_vel_grad<double>(*g_les);
+  LES_ENTER(L);
+  if (!L) return 1;
+  if (L->mixed) compute_vel_grad<float>(*L); else compute_vel_grad<double>(*L);
   LES_CHECK(hipGetLastError());
   return 0;
 }
 int les_grad_velocity_filt(int f, int dfdx, int dfdy) {
-  if (!g_les) return 1;
+  LES_ENTER(L);
+  if (!L) return 1;
   if (f < LES_U || f > LES_W) { les_set_error("grad_velocity_filt: f must be u, v or w"); return 10; }
-  if (g_les->mixed) grad_filt<float>(*g_les, f, dfdx, dfdy); else grad_filt<double>(*g_les, f, dfdx, dfdy);
+  if (L->mixed) grad_filt<float>(*L, f, dfdx, dfdy); else grad_filt<double>(*L, f, dfdx, dfdy);
   LES_CHECK(hipGetLastError());
   return 0;
 }
 int les_sgs_stress(int jt, int jtt) {
-  if (!g_les) return 1;
-  if (g_les->mixed) sgs_stress<float>(*g_les, jt, jtt); else sgs_stress<double>(*g_les, jt, jtt);
+  LES_ENTER(L);
+  if (!L) return 1;
+  if (L->mixed) sgs_stress<float>(*L, jt, jtt); else sgs_stress<double>(*L, jt, jtt);
   LES_CHECK(hipGetLastError());
   return 0;
 }
 int les_compute_rhs_adv(void) {
-  if (!g_les) return 1;
-  if (g_les->mixed) compute_rhs_adv<float>(*g_les); else compute_rhs_adv<double>(*g_les);
+  LES_ENTER(L);
+  if (!L) return 1;
+  if (L->mixed) compute_rhs_adv<float>(*L); else compute_rhs_adv<double>(*L);
   LES_CHECK(hipGetLastError());
   return 0;
 }
 int les_press_stag_array(double tadv1) {
-  if (!g_les) return 1;
-  if (g_les->mixed) press_stag_array<float>(*g_les, tadv1); else press_stag_array<double>(*g_les, tadv1);
+  LES_ENTER(L);
+  if (!L) return 1;
+  if (L->mixed) press_stag_array<float>(*L, tadv1); else press_stag_array<double>(*L, tadv1);
   LES_CHECK(hipGetLastError());
   return 0;
 }
 
 int les_fft2d_r2c(const void* d_in, void* d_out, int nplanes, double scale) {
-  Les* L = g_les;
+  LES_ENTER(L);
   if (!L) return 1;
   if (L->mixed) {
     const float* s[1] = {(const float*)d_in};
@@ -1494,7 +1519,7 @@ int les_fft2d_r2c(const void* d_in, void* d_out, int nplanes, double scale) {
 }
 
 int les_fft2d_c2r(const void* d_in, void* d_out, int nplanes) {
-  Les* L = g_les;
+  LES_ENTER(L);
   if (!L) return 1;
   // the input is preserved (unlike FFTW's c2r): the y pass goes to a workspace
   size_t need = (size_t)nplanes * L->ns;
@@ -1537,7 +1562,7 @@ __global__ void k_ddz(const TI* f, TO* d, long np, int nz, double cz, int w_node
 }
 
 static int ddz_any(int dfdz, int f, int w_nodes) {
-  Les* L = g_les;
+  LES_ENTER(L);
   if (!L) return 1;
   if (dfdz < 0 || dfdz >= LES_NFIELDS || f < 0 || f >= LES_NFIELDS) return 10;
   const double cz = 1.0 / L->dz;
@@ -1572,7 +1597,7 @@ int les_ddz_uv(int dfdz, int f) { return ddz_any(dfdz, f, 0); }
 int les_ddz_w(int dfdz, int f) { return ddz_any(dfdz, f, 1); }
 
 int les_compute_dealias_convec(int cx, int cy, int cz) {
-  Les* L = g_les;
+  LES_ENTER(L);
   if (!L) return 1;
   for (int id : {cx, cy, cz})
     if (id < 0 || id >= LES_NFIELDS || L->fbytes[id] != 8) { les_set_error("convective output must be an FP64 field"); return 10; }
@@ -1583,7 +1608,7 @@ int les_compute_dealias_convec(int cx, int cy, int cz) {
 }
 
 int les_div_stress(int rhs, int tx, int ty, int tz, int stag, int save_wk) {
-  Les* L = g_les;
+  LES_ENTER(L);
   if (!L) return 1;
   if (L->fbytes[rhs] != 8) { les_set_error("div_stress: rhs must be an FP64 field"); return 10; }
   for (int id : {tx, ty, tz})
@@ -1595,21 +1620,23 @@ int les_div_stress(int rhs, int tx, int ty, int tz, int stag, int save_wk) {
 }
 
 int les_ab2(double tadv1, double tadv2) {
-  if (!g_les) return 1;
-  ab2(*g_les, tadv1, tadv2);
+  LES_ENTER(L);
+  if (!L) return 1;
+  ab2(*L, tadv1, tadv2);
   LES_CHECK(hipGetLastError());
   return 0;
 }
 
 int les_projection(double tadv1) {
-  if (!g_les) return 1;
-  projection(*g_les, tadv1);
+  LES_ENTER(L);
+  if (!L) return 1;
+  projection(*L, tadv1);
   LES_CHECK(hipGetLastError());
   return 0;
 }
 
 int les_test_filter(int f, int alpha) {
-  Les* L = g_les;
+  LES_ENTER(L);
   if (!L) return 1;
   if (f < 0 || f >= LES_NFIELDS || field_is_fp64(f)) { les_set_error("test_filter: flow-precision field expected"); return 10; }
   if (alpha != 2 && alpha != 4) { les_set_error("test_filter: alpha must be 2 or 4"); return 1; }
@@ -1695,7 +1722,7 @@ static void stat_zero(Les& L) {
 extern "C" {
 
 int les_stat_init(void) {
-  Les* L = g_les;
+  LES_ENTER(L);
   if (!L) return 1;
   if (!L->st_sum && !dalloc_all(*L, {dbuf(L->st_sum, LES_NSTAT * (size_t)L->np * L->nz), dbuf(L->st_ustar, L->np),
                                      dbuf(L->st_part, (size_t)L->nz * LES_PROF_SLICES * PS_N),
@@ -1709,7 +1736,7 @@ int les_stat_init(void) {
 }
 
 int les_set_geostrophic(double ug, double vg) {
-  Les* L = g_les;
+  LES_ENTER(L);
   if (!L) return 1;
   L->P.ug = ug;
   L->P.vg = vg;
@@ -1717,7 +1744,7 @@ int les_set_geostrophic(double ug, double vg) {
 }
 
 int les_tke_init(void) {
-  Les* L = g_les;
+  LES_ENTER(L);
   if (!L) return 1;
   if (!L->tk_sum &&
       !dalloc_all(*L, {dbuf(L->tk_sum, LES_NTKE * (size_t)L->nz), dbuf(L->tk_part, (size_t)L->nz * LES_TKE_SLICES * LES_NTKE),
@@ -1730,7 +1757,7 @@ int les_tke_init(void) {
 }
 
 int les_tke_reset(void) {
-  Les* L = g_les;
+  LES_ENTER(L);
   if (!L) return 1;
   if (!L->tk_sum) { les_set_error("tke budget not initialised (les_tke_init)"); return 1; }
   hipLaunchKernelGGL(k_fill_zero, dim3(nblk((long)LES_NTKE * L->nz)), dim3(LES_BLOCK), 0, L->stream, L->tk_sum,
@@ -1740,7 +1767,7 @@ int les_tke_reset(void) {
 }
 
 int les_tke_accumulate(void) {
-  Les* L = g_les;
+  LES_ENTER(L);
   if (!L) return 1;
   if (!L->tk_sum) { les_set_error("tke budget not initialised (les_tke_init)"); return 1; }
   if (L->mixed) tke_accumulate<float>(*L); else tke_accumulate<double>(*L);
@@ -1749,7 +1776,7 @@ int les_tke_accumulate(void) {
 }
 
 int les_tke_download(double* sums) {
-  Les* L = g_les;
+  LES_ENTER(L);
   if (!L) return 1;
   if (!L->tk_sum) { les_set_error("tke budget not initialised (les_tke_init)"); return 1; }
   if (!sums) { les_set_error("les_tke_download: null output"); return 10; }
@@ -1759,7 +1786,7 @@ int les_tke_download(double* sums) {
 }
 
 int les_stat_reset(void) {
-  Les* L = g_les;
+  LES_ENTER(L);
   if (!L) return 1;
   if (!L->st_sum) { les_set_error("statistics not initialised (les_stat_init)"); return 1; }
   stat_zero(*L);
@@ -1768,7 +1795,7 @@ int les_stat_reset(void) {
 }
 
 int les_stat_accumulate(void) {
-  Les* L = g_les;
+  LES_ENTER(L);
   if (!L) return 1;
   if (!L->st_sum) { les_set_error("statistics not initialised (les_stat_init)"); return 1; }
   if (L->mixed) stat_accumulate<float>(*L); else stat_accumulate<double>(*L);
@@ -1778,7 +1805,7 @@ int les_stat_accumulate(void) {
 }
 
 int les_stat_download(double* sums3d, double* ustar2d, int* iterations) {
-  Les* L = g_les;
+  LES_ENTER(L);
   if (!L) return 1;
   if (!L->st_sum) { les_set_error("statistics not initialised (les_stat_init)"); return 1; }
   LES_CHECK(hipStreamSynchronize(L->stream));
@@ -1790,7 +1817,7 @@ int les_stat_download(double* sums3d, double* ustar2d, int* iterations) {
 }
 
 int les_stat_profiles(double* prof) {
-  Les* L = g_les;
+  LES_ENTER(L);
   if (!L) return 1;
   if (!L->st_sum) { les_set_error("statistics not initialised (les_stat_init)"); return 1; }
   if (L->st_iters < 1) { les_set_error("no accumulated statistics"); return 1; }
@@ -1815,7 +1842,7 @@ int les_stat_profiles(double* prof) {
 // needs no clearing: k_stat_planes writes every partial k_stat_profiles
 // reads, and k_stat_profiles every profile value copied out.
 int les_stat_profiles_noalloc(double* prof) {
-  Les* L = g_les;
+  LES_ENTER(L);
   if (!L) return 1;
   if (L->nz > LES_NOALLOC_MAX_NZ) {
     les_set_error("les_stat_profiles_noalloc: nz = %d exceeds the scratch limit of %d levels", L->nz,
@@ -1842,7 +1869,7 @@ int les_stat_profiles_noalloc(double* prof) {
 }
 
 int les_running_diagnostics(double* out) {
-  Les* L = g_les;
+  LES_ENTER(L);
   if (!L) return 1;
   if (L->mixed) diagnostics<float>(*L); else diagnostics<double>(*L);
   LES_CHECK(hipGetLastError());

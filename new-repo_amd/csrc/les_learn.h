@@ -420,7 +420,7 @@ int les_mlp_layout(long* nweights) {
 }
 
 int les_mlp_set_weights(const float* w, long nweights) {
-  Les* L = g_les;
+  LES_ENTER(L);
   if (!L) return 1;
   if (nweights != MLP_NPUB) { les_set_error("les_mlp_set_weights: expected %d values", MLP_NPUB); return 10; }
   int rc = mlp_alloc(*L);
@@ -440,7 +440,7 @@ int les_mlp_set_weights(const float* w, long nweights) {
 }
 
 int les_mlp_get_weights(float* w) {
-  Les* L = g_les;
+  LES_ENTER(L);
   if (!L || !L->mlp) return 1;
   std::vector<float> dev(MLP_NPAR);
   LES_CHECK(hipStreamSynchronize(L->stream));
@@ -452,7 +452,7 @@ int les_mlp_get_weights(float* w) {
 // raw samples (device: [n][12] features, [n][2] targets) -> normalised
 // training buffers (device: bf16 [n][16], float [n][16])
 int les_mlp_prepare(const void* d_raw, const void* d_tgt, long n, void* d_x, void* d_y) {
-  Les* L = g_les;
+  LES_ENTER(L);
   if (!L || !L->mlp) { les_set_error("les_mlp_prepare: set weights/normalisers first"); return 1; }
   MlpState* M = L->mlp;
   hipLaunchKernelGGL(k_prepare, dim3(nblk(n)), dim3(LES_BLOCK), 0, L->stream, (const float*)d_raw, (const float*)d_tgt,
@@ -464,7 +464,7 @@ int les_mlp_prepare(const void* d_raw, const void* d_tgt, long n, void* d_x, voi
 
 // gradient (compact layout, weights and biases only) and loss of a batch
 int les_mlp_grad(const void* d_x, const void* d_y, long n, float* grad, double* loss) {
-  Les* L = g_les;
+  LES_ENTER(L);
   if (!L || !L->mlp) return 1;
   int rc = mlp_forward_backward(*L, (const short*)d_x, (const float*)d_y, n, loss);
   if (rc) return rc;
@@ -479,7 +479,7 @@ int les_mlp_grad(const void* d_x, const void* d_y, long n, float* grad, double* 
 
 // one Adam step on a batch
 int les_mlp_train_step(const void* d_x, const void* d_y, long n, double lr, double* loss) {
-  Les* L = g_les;
+  LES_ENTER(L);
   if (!L || !L->mlp) return 1;
   MlpState* M = L->mlp;
   int rc = mlp_forward_backward(*L, (const short*)d_x, (const float*)d_y, n, loss);
@@ -495,7 +495,7 @@ int les_mlp_train_step(const void* d_x, const void* d_y, long n, double lr, doub
 // fused inference on a feature batch (device bf16 [n][16]) -> normalised
 // outputs (device float [n][2])
 int les_mlp_forward(const void* d_x, long n, void* d_out) {
-  Les* L = g_les;
+  LES_ENTER(L);
   if (!L || !L->mlp) return 1;
   MlpState* M = L->mlp;
   InferArgs ia;
@@ -514,7 +514,7 @@ int les_mlp_forward(const void* d_x, long n, void* d_out) {
 // training samples at the current state (call right after a step with a
 // plain dynamic-procedure update; mixed-precision modes only)
 int les_sgs_samples(void* d_x, void* d_y, long max_samples, long* n_written, int stride) {
-  Les* L = g_les;
+  LES_ENTER(L);
   if (!L) return 1;
   if (!L->mixed) { les_set_error("les_sgs_samples: run in a mixed-precision mode"); return 1; }
   if (stride < 1) stride = 1;
@@ -561,7 +561,7 @@ int les_sgs_samples(void* d_x, void* d_y, long max_samples, long* n_written, int
 }
 
 int les_mlp_judge_stats(double* out) {
-  Les* L = g_les;
+  LES_ENTER(L);
   if (!L) return 1;
   for (int i = 0; i < 4; ++i) out[i] = L->judge[i];
   return 0;

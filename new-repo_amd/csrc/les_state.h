@@ -27,7 +27,9 @@ struct Les {
   int jt_total;
   int jt;                // steps since les_init (the reference's local count)
   int F_coeff_init;
-  hipStream_t stream;    // the stream calls run on: the default (null) one, except while a step issues work to a side stream
+  hipStream_t stream;    // the stream calls run on: own_stream or (les_set_default_stream) the default one,
+                         // except while a step issues work to a side stream
+  hipStream_t own_stream;
   hipStream_t stream2;   // second stream of the step: the SGS stage beside the convection
   hipEvent_t ev_fork, ev_join;
   hipStream_t stream3;   // learned mode: the surrogate's chain beside the band's plain update
@@ -119,6 +121,25 @@ struct Les {
 };
 
 extern Les* g_les;
+
+// Makes the device of les_init current for the length of a call: allocations,
+// and launches on the default stream, go to the current device, which a
+// caller with several may have changed since.
+struct OnDevice {
+  int prev = -1;
+  explicit OnDevice(const Les* L) {
+    int d;
+    if (L && hipGetDevice(&d) == hipSuccess && d != L->dev && hipSetDevice(L->dev) == hipSuccess) prev = d;
+  }
+  ~OnDevice() {
+    if (prev >= 0) hipSetDevice(prev);
+  }
+  OnDevice(const OnDevice&) = delete;
+};
+// first line of every entry point
+#define LES_ENTER(L) \
+  Les* L = g_les;    \
+  const OnDevice on_device_(L)
 
 // helpers implemented in les_gpu.hip
 template <typename T>

@@ -38,6 +38,9 @@ static void* bufs[MAXBUF];
 int hipMalloc(void** p, size_t n) {
   *p = NULL;
   if (host_fail_at > 0 && --host_fail_at == 0) return last_error = NOMEM;
+  char t[80];
+  snprintf(t, sizeof t, "malloc %zu device %d", n, host_device);
+  log_line(t);
   *p = calloc(1, n);
   ++host_mallocs;
   ++host_live;
