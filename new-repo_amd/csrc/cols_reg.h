@@ -138,14 +138,6 @@ k_cols_reg(ColArgs<T> a, const Cplx<T>* __restrict__ tw) {
   }
 }
 
-// The instances a step uses: FP32 has no pressure operations, FP64 no
-// two-output gradient.
-#define LES_COL_INSTANCES(X)                                                                                     \
-  X(COP_DIV, 1, true, true) X(COP_FILT1, 1, true, true) X(COP_FILT2, 2, true, true) X(COP_COPY, 1, true, false)   \
-  X(COP_COPY, 1, false, true)
-#define LES_COL_INSTANCES_F32(X) X(COP_GRAD, 2, true, true)
-#define LES_COL_INSTANCES_F64(X) X(COP_GRAD, 3, true, true) X(COP_DIV, 1, true, false) X(COP_PGRAD, 3, false, true)
-
 // Launches the instance of op (nout outputs, fwd, inv) of length N; with attr
 // set only raises every instance's LDS limit.
 template <typename T, int N>

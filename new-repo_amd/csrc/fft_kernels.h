@@ -29,6 +29,9 @@
 // p - (u u + v v + W W) / 2, W = (w(k) + w(k+1)) / 2, from p (src) and u, v, w
 // (ab_r), 0 on the planes 0 and nz+1.
 enum { LOAD_SCALE = 0, LOAD_SCALE_DIV = 1, LOAD_AB2_SCALE_DIV = 2, LOAD_PCLEAN = 3 };
+// the load modes compiled for transforms of precision T
+template <typename T>
+constexpr bool r2c_has(int mode) { return sizeof(T) == 8 ? mode >= LOAD_SCALE && mode <= LOAD_PCLEAN : mode == LOAD_SCALE; }
 
 template <typename TI, typename T>
 struct RowR2CArgs {
@@ -36,7 +39,6 @@ struct RowR2CArgs {
   Cplx<T>* dst[LES_R2C_FIELDS];
   int nx, ny, lhx;
   int k0, nplanes;  // planes [k0, k0+nplanes)
-  int mode;
   T scale, div;
   const TI* ab_r[3];  // LOAD_AB2_SCALE_DIV: rhs and rhs_f of field f
   const TI* ab_f[3];
@@ -60,6 +62,21 @@ struct RowC2RArgs {
 // ------------------------------------------------------------------ columns
 // Spectral-space operations applied between the forward and inverse y passes.
 enum { COP_GRAD = 0, COP_DIV = 1, COP_FILT2 = 2, COP_FILT1 = 3, COP_COPY = 4, COP_PGRAD = 5 };
+
+// The instances (op, outputs, forward and inverse transform) a step uses: FP32
+// has no pressure operations, FP64 no two-output gradient.
+#define LES_COL_INSTANCES(X)                                                                                     \
+  X(COP_DIV, 1, true, true) X(COP_FILT1, 1, true, true) X(COP_FILT2, 2, true, true) X(COP_COPY, 1, true, false)   \
+  X(COP_COPY, 1, false, true)
+#define LES_COL_INSTANCES_F32(X) X(COP_GRAD, 2, true, true)
+#define LES_COL_INSTANCES_F64(X) X(COP_GRAD, 3, true, true) X(COP_DIV, 1, true, false) X(COP_PGRAD, 3, false, true)
+template <typename T>
+constexpr bool cols_has(int op, int nout, bool fwd, bool inv) {
+#define X(OP, NOUT, FWD, INV) || (op == OP && nout == NOUT && fwd == FWD && inv == INV)
+  return (false LES_COL_INSTANCES(X)) || (sizeof(T) == 4 && (false LES_COL_INSTANCES_F32(X))) ||
+         (sizeof(T) == 8 && (false LES_COL_INSTANCES_F64(X)));
+#undef X
+}
 
 template <typename T>
 struct ColArgs {  // k_cols_reg, cols_reg.h

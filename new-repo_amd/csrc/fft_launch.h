@@ -17,26 +17,10 @@ bool cols_reg_part(bool attr, int ny, int op, int nout, bool fwd, bool inv, cons
 template <typename T, int PART>
 bool colres_reg_part(bool attr, int n, bool pad, const ColResArgs<T>& a, int nf, const Cplx<T>* twn, const Cplx<T>* twb,
                      hipStream_t s);
-
-template <typename T, int PART = 0>
-static bool cols_reg(bool attr, int ny, int op, int nout, bool fwd, bool inv, const ColArgs<T>& a, int njobs,
-                     const Cplx<T>* tw, hipStream_t s) {
-  if (cols_reg_part<T, PART>(attr, ny, op, nout, fwd, inv, a, njobs, tw, s)) return true;
-  if constexpr (PART + 1 < LES_LENGTH_PARTS) return cols_reg<T, PART + 1>(attr, ny, op, nout, fwd, inv, a, njobs, tw, s);
-  return false;
-}
-template <typename T, int PART = 0>
-static bool colres_reg(bool attr, int n, bool pad, const ColResArgs<T>& a, int nf, const Cplx<T>* twn, const Cplx<T>* twb,
-                       hipStream_t s) {
-  if (colres_reg_part<T, PART>(attr, n, pad, a, nf, twn, twb, s)) return true;
-  if constexpr (PART + 1 < LES_LENGTH_PARTS) return colres_reg<T, PART + 1>(attr, n, pad, a, nf, twn, twb, s);
-  return false;
-}
-
 // Row transforms of length n (nf fields; tw: the forward table of n), the
 // resampling n <-> 3 n / 2 (twn, twb).  attr and the result as above.
 template <typename TI, typename T, int PART>
-bool rows_r2c_part(bool attr, int n, const RowR2CArgs<TI, T>& a, int nf, const Cplx<T>* tw, hipStream_t s);
+bool rows_r2c_part(bool attr, int n, int mode, const RowR2CArgs<TI, T>& a, int nf, const Cplx<T>* tw, hipStream_t s);
 template <typename T, int PART>
 bool rows_nyq_part(bool attr, int n, const RowR2CArgs<double, T>& a, int nf, const Cplx<T>* tw, hipStream_t s);
 template <typename T, typename TO, int PART>
@@ -51,12 +35,30 @@ template <typename T, int PART>
 bool rows_trunc_part(bool attr, int n, const RowResArgs<T, T, double>& a, int nf, const Cplx<T>* twn, const Cplx<T>* twb,
                      hipStream_t s);
 
-// the part that has length n, over all parts
+// The part that has length n, over all parts.  Operation and load mode are
+// template arguments: a kernel that is not compiled is an error of the build
+// and not a call that launches nothing.  That the lengths have kernels is
+// checked once, by les_init (attr).
 #define LES_EACH_PART(CALL) CALL(0) || CALL(1) || CALL(2) || CALL(3)
 static_assert(LES_LENGTH_PARTS == 4, "LES_EACH_PART lists the parts");
-template <typename TI, typename T>
+template <typename T, int OP, int NOUT, bool FWD, bool INV>
+static bool cols_reg(bool attr, int ny, const ColArgs<T>& a, int njobs, const Cplx<T>* tw, hipStream_t s) {
+  static_assert(cols_has<T>(OP, NOUT, FWD, INV), "no column kernel of this operation and precision (LES_COL_INSTANCES)");
+#define C(P) (cols_reg_part<T, P>(attr, ny, OP, NOUT, FWD, INV, a, njobs, tw, s))
+  return LES_EACH_PART(C);
+#undef C
+}
+template <typename T>
+static bool colres_reg(bool attr, int n, bool pad, const ColResArgs<T>& a, int nf, const Cplx<T>* twn, const Cplx<T>* twb,
+                       hipStream_t s) {
+#define C(P) (colres_reg_part<T, P>(attr, n, pad, a, nf, twn, twb, s))
+  return LES_EACH_PART(C);
+#undef C
+}
+template <typename TI, typename T, int MODE>
 static bool rows_r2c_reg(bool attr, int n, const RowR2CArgs<TI, T>& a, int nf, const Cplx<T>* tw, hipStream_t s) {
-#define C(P) (rows_r2c_part<TI, T, P>(attr, n, a, nf, tw, s))
+  static_assert(r2c_has<T>(MODE), "no forward row kernel of this load mode and precision");
+#define C(P) (rows_r2c_part<TI, T, P>(attr, n, MODE, a, nf, tw, s))
   return LES_EACH_PART(C);
 #undef C
 }

@@ -23,14 +23,14 @@
   } while (0)
 
 template <typename TI, typename T, int N>
-static void r2c_n(bool attr, const RowR2CArgs<TI, T>& a, int nf, const Cplx<T>* tw, hipStream_t s) {
+static void r2c_n(bool attr, int mode, const RowR2CArgs<TI, T>& a, int nf, const Cplx<T>* tw, hipStream_t s) {
   using SH = RowShape<T, N>;
   if constexpr (sizeof(T) == 8) {
-    if (attr || a.mode == LOAD_SCALE_DIV) LES_ROW_LAUNCH(SH, (k_rows_r2c_reg<TI, T, N, LOAD_SCALE_DIV, false>), tw);
-    if (attr || a.mode == LOAD_AB2_SCALE_DIV) LES_ROW_LAUNCH(SH, (k_rows_r2c_reg<TI, T, N, LOAD_AB2_SCALE_DIV, true>), tw);
-    if (attr || a.mode == LOAD_PCLEAN) LES_ROW_LAUNCH(SH, (k_rows_r2c_reg<TI, T, N, LOAD_PCLEAN, true>), tw);
+    if (attr || mode == LOAD_SCALE_DIV) LES_ROW_LAUNCH(SH, (k_rows_r2c_reg<TI, T, N, LOAD_SCALE_DIV, false>), tw);
+    if (attr || mode == LOAD_AB2_SCALE_DIV) LES_ROW_LAUNCH(SH, (k_rows_r2c_reg<TI, T, N, LOAD_AB2_SCALE_DIV, true>), tw);
+    if (attr || mode == LOAD_PCLEAN) LES_ROW_LAUNCH(SH, (k_rows_r2c_reg<TI, T, N, LOAD_PCLEAN, true>), tw);
   }
-  if (attr || a.mode == LOAD_SCALE) LES_ROW_LAUNCH(SH, (k_rows_r2c_reg<TI, T, N, LOAD_SCALE, false>), tw);
+  if (attr || mode == LOAD_SCALE) LES_ROW_LAUNCH(SH, (k_rows_r2c_reg<TI, T, N, LOAD_SCALE, false>), tw);
 }
 
 #define LES_ROW_SWITCH(n, CALL)   \
@@ -40,9 +40,9 @@ static void r2c_n(bool attr, const RowR2CArgs<TI, T>& a, int nf, const Cplx<T>* 
   return false
 
 template <>
-bool rows_r2c_part<double, LES_T, LES_PART>(bool attr, int n, const RowR2CArgs<double, LES_T>& a, int nf,
+bool rows_r2c_part<double, LES_T, LES_PART>(bool attr, int n, int mode, const RowR2CArgs<double, LES_T>& a, int nf,
                                             const Cplx<LES_T>* tw, hipStream_t s) {
-#define X(N) case N: r2c_n<double, LES_T, N>(attr, a, nf, tw, s); return true;
+#define X(N) case N: r2c_n<double, LES_T, N>(attr, mode, a, nf, tw, s); return true;
   LES_ROW_SWITCH(n, X);
 #undef X
 }
@@ -99,9 +99,9 @@ bool rows_nyq_part<float, LES_PART>(bool attr, int n, const RowR2CArgs<double, f
 #undef X
 }
 template <>
-bool rows_r2c_part<float, float, LES_PART>(bool attr, int n, const RowR2CArgs<float, float>& a, int nf, const Cplx<float>* tw,
+bool rows_r2c_part<float, float, LES_PART>(bool attr, int n, int mode, const RowR2CArgs<float, float>& a, int nf, const Cplx<float>* tw,
                                            hipStream_t s) {
-#define X(N) case N: r2c_n<float, float, N>(attr, a, nf, tw, s); return true;
+#define X(N) case N: r2c_n<float, float, N>(attr, mode, a, nf, tw, s); return true;
   LES_ROW_SWITCH(n, X);
 #undef X
 }

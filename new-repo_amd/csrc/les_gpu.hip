@@ -176,29 +176,27 @@ static void kt_end(Les& L, int fam, double bytes, const char* base, int ta = 0, 
 }
 
 // ------------------------------------------------------------------ launch helpers
-// Row kernels: one wavefront per row pair, LES_BLOCK / 64 of them per block.
-
-template <typename TI, typename T>
-static void rows_r2c(Les& L, const TI* const* src, Cplx<T>* const* dst, int nf, int k0, int npl, T scale, int mode = LOAD_SCALE,
-                     T div = (T)1, int ny_override = 0, const TI* const* ab = nullptr, const T* abc = nullptr) {
+template <typename TI, typename T, int MODE = LOAD_SCALE>
+static void rows_r2c(Les& L, const TI* const* src, Cplx<T>* const* dst, int nf, int k0, int npl, T scale, T div = (T)1,
+                     const TI* const* ab = nullptr, const T* abc = nullptr) {
   RowR2CArgs<TI, T> a;
   for (int f = 0; f < nf; ++f) { a.src[f] = src[f]; a.dst[f] = dst[f]; }
-  a.nx = L.nx; a.ny = ny_override ? ny_override : L.ny; a.lhx = L.lhx; a.k0 = k0; a.nplanes = npl;
-  a.mode = mode; a.scale = scale; a.div = div;
-  if (mode == LOAD_AB2_SCALE_DIV) {
+  a.nx = L.nx; a.ny = L.ny; a.lhx = L.lhx; a.k0 = k0; a.nplanes = npl;
+  a.scale = scale; a.div = div;
+  if (MODE == LOAD_AB2_SCALE_DIV) {
     for (int f = 0; f < nf && f < 3; ++f) { a.ab_r[f] = ab[f]; a.ab_f[f] = ab[3 + f]; }
     a.ab_dt = abc[0]; a.ab_t1 = abc[1]; a.ab_t2 = abc[2];
   }
-  if (mode == LOAD_PCLEAN) {  // one field; ab = u, v, w
+  if (MODE == LOAD_PCLEAN) {  // one field; ab = u, v, w
     for (int f = 0; f < 3; ++f) a.ab_r[f] = ab[f];
     a.pc_nz = L.nz;
   }
   kt_begin(L, KT_ROWS_R2C);
-  rows_r2c_reg<TI, T>(false, L.nx, a, nf, twpool<T>(L) + L.px.twf, L.stream);
-  const double in_fields = mode == LOAD_AB2_SCALE_DIV ? 3.0 : mode == LOAD_PCLEAN ? 4.0 : 1.0;
+  rows_r2c_reg<TI, T, MODE>(false, L.nx, a, nf, twpool<T>(L) + L.px.twf, L.stream);
+  const double in_fields = MODE == LOAD_AB2_SCALE_DIV ? 3.0 : MODE == LOAD_PCLEAN ? 4.0 : 1.0;
   kt_end(L, KT_ROWS_R2C, (double)nf * npl * a.ny * (in_fields * L.nx * sizeof(TI) + (double)L.lhx * sizeof(Cplx<T>)),
          "k_rows_r2c_reg", sizeof(TI), sizeof(T),
-         mode == LOAD_AB2_SCALE_DIV ? "AB2 predictor" : mode == LOAD_PCLEAN ? "cleaned pressure" : nullptr);
+         MODE == LOAD_AB2_SCALE_DIV ? "AB2 predictor" : MODE == LOAD_PCLEAN ? "cleaned pressure" : nullptr);
 }
 
 // The grad_velocity_filt forward transforms of nf velocity components in the
@@ -208,7 +206,7 @@ static void rows_r2c_nyq(Les& L, const double* const* src, Cplx<float>* const* d
   RowR2CArgs<double, float> a;
   for (int f = 0; f < nf; ++f) { a.src[f] = src[f]; a.dst[f] = dst[f]; }
   a.nx = L.nx; a.ny = L.ny; a.lhx = L.lhx; a.k0 = 0; a.nplanes = npl;
-  a.mode = LOAD_SCALE; a.scale = scale; a.div = 1.0f;
+  a.scale = scale; a.div = 1.0f;
   a.nyq_as = (long)L.ny * L.nzg;
   a.nyq_ps = (long)(L.ny / 4) * L.nx * L.nzg;
   a.nyq_a = L.nyq_rows + fld * a.nyq_as;
@@ -235,10 +233,9 @@ static void rows_c2r(Les& L, const Cplx<T>* const* src, TO* const* dst, int nf, 
 // The same column op on njobs (at most LES_COL_JOBS) independent sets of
 // inputs and outputs in one launch: the sets' tiles share the grid, so the
 // partly filled last round of blocks is paid once instead of once per set.
-template <typename T>
-static void cols_jobs(Les& L, int op, int njobs, const Cplx<T>* const* in0, const Cplx<T>* const* in1,
-                      Cplx<T>* const* o0, Cplx<T>* const* o1, Cplx<T>* const* o2, int nout, int fwd, int inv, int k0,
-                      int npl, const T* g0 = nullptr, const T* g1 = nullptr) {
+template <typename T, int OP, int NOUT, bool FWD, bool INV>
+static void cols_jobs(Les& L, int njobs, const Cplx<T>* const* in0, const Cplx<T>* const* in1, Cplx<T>* const* o0,
+                      Cplx<T>* const* o1, Cplx<T>* const* o2, int k0, int npl, const T* g0 = nullptr, const T* g1 = nullptr) {
   assert(njobs >= 1 && njobs <= LES_COL_JOBS);
   ColArgs<T> a;
   for (int j = 0; j < LES_COL_JOBS; ++j) {
@@ -251,20 +248,20 @@ static void cols_jobs(Les& L, int op, int njobs, const Cplx<T>* const* in0, cons
   a.g0 = g0; a.g1 = g1;
   a.lhx = L.lhx; a.k0 = k0; a.nplanes = npl;
   kt_begin(L, KT_COLS);
-  cols_reg<T>(false, L.ny, op, nout, fwd, inv, a, njobs, twpool<T>(L) + L.py.twf, L.stream);
+  cols_reg<T, OP, NOUT, FWD, INV>(false, L.ny, a, njobs, twpool<T>(L) + L.py.twf, L.stream);
   static const char* const opn[] = {"GRAD", "DIV", "FILT2", "FILT1", "COPY", "PGRAD"};
-  kt_end(L, KT_COLS, (double)njobs * npl * L.ns * sizeof(Cplx<T>) * ((in1 ? 2 : 1) + nout), "k_cols_reg", sizeof(T), 0, opn[op]);
+  kt_end(L, KT_COLS, (double)njobs * npl * L.ns * sizeof(Cplx<T>) * ((in1 ? 2 : 1) + NOUT), "k_cols_reg", sizeof(T), 0, opn[OP]);
 }
 
-template <typename T>
-static void cols(Les& L, int op, const Cplx<T>* in0, const Cplx<T>* in1, Cplx<T>* o0, Cplx<T>* o1, Cplx<T>* o2,
-                 int nout, int fwd, int inv, int k0, int npl, const T* g0 = nullptr, const T* g1 = nullptr) {
+template <typename T, int OP, int NOUT, bool FWD, bool INV>
+static void cols(Les& L, const Cplx<T>* in0, const Cplx<T>* in1, Cplx<T>* o0, Cplx<T>* o1, Cplx<T>* o2, int k0, int npl,
+                 const T* g0 = nullptr, const T* g1 = nullptr) {
   const Cplx<T>* i0[1] = {in0};
   const Cplx<T>* i1[1] = {in1};
   Cplx<T>* p0[1] = {o0};
   Cplx<T>* p1[1] = {o1};
   Cplx<T>* p2[1] = {o2};
-  cols_jobs<T>(L, op, 1, i0, in1 ? i1 : nullptr, p0, p1, p2, nout, fwd, inv, k0, npl, g0, g1);
+  cols_jobs<T, OP, NOUT, FWD, INV>(L, 1, i0, in1 ? i1 : nullptr, p0, p1, p2, k0, npl, g0, g1);
 }
 
 // ------------------------------------------------------------------ field access
@@ -301,7 +298,7 @@ static void grad_filt(Les& L, int fid, int dx_id, int dy_id) {
   } else {
     rows_r2c<double, T>(L, src, dst, 1, 0, L.nzg, c);
   }
-  cols<T>(L, COP_GRAD, s0, nullptr, s1, s2, s3, L.mixed ? 2 : 3, 1, 1, 0, L.nzg);
+  cols<T, COP_GRAD, sizeof(T) == 4 ? 2 : 3, true, true>(L, s0, nullptr, s1, s2, s3, 0, L.nzg);
   const Cplx<T>* cs[2] = {s1, s2};
   T* outs[2] = {F<T>(L, dx_id), F<T>(L, dy_id)};
   rows_c2r<T, T>(L, cs, outs, 2, 0, L.nzg);
@@ -353,7 +350,7 @@ static void grad_filt3(Les& L) {
   } else {
     rows_r2c<double, T>(L, src, in, 3, 0, L.nzg, c);
   }
-  cols_jobs<T>(L, COP_GRAD, 3, in, nullptr, ox, oy, L.mixed ? nullptr : in, L.mixed ? 2 : 3, 1, 1, 0, L.nzg);
+  cols_jobs<T, COP_GRAD, sizeof(T) == 4 ? 2 : 3, true, true>(L, 3, in, nullptr, ox, oy, sizeof(T) == 4 ? nullptr : in, 0, L.nzg);
   if constexpr (std::is_same<T, double>::value) {
     // the filtered fields with the derivatives in one launch
     for (int f = 0; f < 3; ++f) { cs[6 + f] = in[f]; outs[6 + f] = D(L, fid[f]); }
@@ -432,7 +429,7 @@ static void wall_law(Les& L) {
     rows_r2c<double, T>(L, src, dst, 2, 0, 1, (T)1);
     const T* g2 = sizeof(T) == 8 ? (const T*)L.g2_64 : (const T*)L.g2_32;
     Cplx<T>* fl[2] = {sc, sd};
-    cols_jobs<T>(L, COP_FILT1, 2, dst, nullptr, fl, nullptr, nullptr, 1, 1, 1, 0, 1, g2);
+    cols_jobs<T, COP_FILT1, 1, true, true>(L, 2, dst, nullptr, fl, nullptr, nullptr, 0, 1, g2);
     const Cplx<T>* cs[2] = {sc, sd};
     T* outs[2] = {u1, v1};
     rows_c2r<T, T>(L, cs, outs, 2, 0, 1);
@@ -955,9 +952,9 @@ static int les_step_t(Les& L) {
 // LDS limits of the kernels of this domain's lengths; nonzero: a length has no kernels
 template <typename T>
 static bool setup_fft_attrs(const Les& L) {
-  return cols_reg<T>(true, L.ny, 0, 0, 0, 0, ColArgs<T>(), 0, nullptr, 0) &&
+  return cols_reg<T, COP_COPY, 1, true, false>(true, L.ny, ColArgs<T>(), 0, nullptr, 0) &&
          colres_reg<T>(true, L.ny, true, ColResArgs<T>(), 0, nullptr, nullptr, 0) &&
-         rows_r2c_reg<double, T>(true, L.nx, RowR2CArgs<double, T>(), 0, nullptr, 0) &&
+         rows_r2c_reg<double, T, LOAD_SCALE>(true, L.nx, RowR2CArgs<double, T>(), 0, nullptr, 0) &&
          rows_c2r_reg<T, double>(true, L.nx, RowC2RArgs<T, double>(), 0, nullptr, 0) &&
          rows_div_reg<T>(true, L.nx, RowC2RArgs<T, T>(), DivEpi3<T>(), 0, nullptr, 0) &&
          rows_pad_reg<T>(true, L.nx, RowResArgs<T, T, T>(), 0, nullptr, nullptr, 0) &&
@@ -967,7 +964,7 @@ static int setup_kernel_attrs(const Les& L) {
   if (tri_in_lds(L.lhx, L.ny, L.nz))
     hipFuncSetAttribute((const void*)k_tridiag_lds, hipFuncAttributeMaxDynamicSharedMemorySize, (int)tri_lds(L.nz));
   const bool ok = setup_fft_attrs<double>(L) && setup_fft_attrs<float>(L) &&
-                  rows_r2c_reg<float, float>(true, L.nx, RowR2CArgs<float, float>(), 0, nullptr, 0) &&
+                  rows_r2c_reg<float, float, LOAD_SCALE>(true, L.nx, RowR2CArgs<float, float>(), 0, nullptr, 0) &&
                   rows_nyq_reg<float>(true, L.nx, RowR2CArgs<double, float>(), 0, nullptr, 0) &&
                   rows_c2r_reg<float, float>(true, L.nx, RowC2RArgs<float, float>(), 0, nullptr, 0) &&
                   rows_proj_reg<double>(true, L.nx, RowC2RArgs<double, double>(), ProjEpi3(), 0, nullptr, 0);
@@ -1506,12 +1503,12 @@ int les_fft2d_r2c(const void* d_in, void* d_out, int nplanes, double scale) {
     const float* s[1] = {(const float*)d_in};
     Cplx<float>* d[1] = {(Cplx<float>*)d_out};
     rows_r2c<float, float>(*L, s, d, 1, 0, nplanes, (float)scale);
-    cols<float>(*L, COP_COPY, d[0], nullptr, d[0], nullptr, nullptr, 1, 1, 0, 0, nplanes);
+    cols<float, COP_COPY, 1, true, false>(*L, d[0], nullptr, d[0], nullptr, nullptr, 0, nplanes);
   } else {
     const double* s[1] = {(const double*)d_in};
     Cplx<double>* d[1] = {(Cplx<double>*)d_out};
     rows_r2c<double, double>(*L, s, d, 1, 0, nplanes, scale);
-    cols<double>(*L, COP_COPY, d[0], nullptr, d[0], nullptr, nullptr, 1, 1, 0, 0, nplanes);
+    cols<double, COP_COPY, 1, true, false>(*L, d[0], nullptr, d[0], nullptr, nullptr, 0, nplanes);
   }
   LES_CHECK(hipGetLastError());
   LES_CHECK(hipStreamSynchronize(L->stream));
@@ -1526,13 +1523,13 @@ int les_fft2d_c2r(const void* d_in, void* d_out, int nplanes) {
   if (need > (size_t)L->nsp) { les_set_error("les_fft2d_c2r: at most nz+2 planes"); return 10; }
   if (L->mixed) {
     Cplx<float>* w = (Cplx<float>*)L->wk_spec[7];
-    cols<float>(*L, COP_COPY, (const Cplx<float>*)d_in, nullptr, w, nullptr, nullptr, 1, 0, 1, 0, nplanes);
+    cols<float, COP_COPY, 1, false, true>(*L, (const Cplx<float>*)d_in, nullptr, w, nullptr, nullptr, 0, nplanes);
     const Cplx<float>* s[1] = {w};
     float* d[1] = {(float*)d_out};
     rows_c2r<float, float>(*L, s, d, 1, 0, nplanes);
   } else {
     Cplx<double>* w = (Cplx<double>*)L->wk_spec[7];
-    cols<double>(*L, COP_COPY, (const Cplx<double>*)d_in, nullptr, w, nullptr, nullptr, 1, 0, 1, 0, nplanes);
+    cols<double, COP_COPY, 1, false, true>(*L, (const Cplx<double>*)d_in, nullptr, w, nullptr, nullptr, 0, nplanes);
     const Cplx<double>* s[1] = {w};
     double* d[1] = {(double*)d_out};
     rows_c2r<double, double>(*L, s, d, 1, 0, nplanes);
@@ -1585,7 +1582,7 @@ static int test_filter_t(Les& L, int fid, int alpha) {
   rows_r2c<T, T>(L, src, dst, 1, 1, L.nz + 1, (T)1);
   const T* g = alpha == 2 ? (sizeof(T) == 8 ? (const T*)L.g2_64 : (const T*)L.g2_32)
                           : (sizeof(T) == 8 ? (const T*)L.g4_64 : (const T*)L.g4_32);
-  cols<T>(L, COP_FILT1, s0, nullptr, s1, nullptr, nullptr, 1, 1, 1, 1, L.nz + 1, g);
+  cols<T, COP_FILT1, 1, true, true>(L, s0, nullptr, s1, nullptr, nullptr, 1, L.nz + 1, g);
   const Cplx<T>* cs[1] = {s1};
   T* outs[1] = {F<T>(L, fid)};
   rows_c2r<T, T>(L, cs, outs, 1, 1, L.nz + 1);
@@ -1689,8 +1686,8 @@ static void tke_accumulate(Les& L) {
   const double* src[1] = {D(L, LES_P)};
   const double* uvw[3] = {D(L, LES_U), D(L, LES_V), D(L, LES_W)};
   Cplx<double>* dst[1] = {s0};
-  rows_r2c<double, double>(L, src, dst, 1, 0, L.nzg, 1.0 / (double)(L.nx * L.ny), LOAD_PCLEAN, 1.0, 0, uvw);
-  cols<double>(L, COP_GRAD, s0, nullptr, s1, s2, s0, 3, 1, 1, 0, L.nzg);
+  rows_r2c<double, double, LOAD_PCLEAN>(L, src, dst, 1, 0, L.nzg, 1.0 / (double)(L.nx * L.ny), 1.0, uvw);
+  cols<double, COP_GRAD, 3, true, true>(L, s0, nullptr, s1, s2, s0, 0, L.nzg);
   const Cplx<double>* cs[3] = {s1, s2, s0};
   double* outs[3] = {L.tk_px, L.tk_py, L.tk_pf};
   rows_c2r<double, double>(L, cs, outs, 3, 0, L.nzg);

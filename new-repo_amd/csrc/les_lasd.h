@@ -187,7 +187,7 @@ static void lasd_update(Les& L, int jtt, int nlev) {
       outs[2 * t + 1] = fl4[f0 + t];
     }
     rows_r2c<T, T>(L, src, sp, nb, 1, nlev, (T)1);
-    cols_jobs<T>(L, COP_FILT2, nb, sp, nullptr, o2, o4, nullptr, 2, 1, 1, 1, nlev, g2, g4);
+    cols_jobs<T, COP_FILT2, 2, true, true>(L, nb, sp, nullptr, o2, o4, nullptr, 1, nlev, g2, g4);
     rows_c2r<T, T>(L, cs, outs, 2 * nb, 1, nlev);
   }
   T* LM = (T*)L.wk_real[57];
@@ -369,7 +369,7 @@ static void dynsmag_update(Les& L) {
       outs[t] = fl[f0 + t];
     }
     rows_r2c<T, T>(L, src, sp, nb, 1, nlev, (T)1);
-    cols_jobs<T>(L, COP_FILT1, nb, sp, nullptr, fo, nullptr, nullptr, 1, 1, 1, 1, nlev, g2);
+    cols_jobs<T, COP_FILT1, 1, true, true>(L, nb, sp, nullptr, fo, nullptr, nullptr, 1, nlev, g2);
     rows_c2r<T, T>(L, cs, outs, nb, 1, nlev);
   }
   GermanoArgs<T> ga;

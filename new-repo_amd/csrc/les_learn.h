@@ -220,7 +220,7 @@ static void learned_coeffs(Les& L, void* cs, void* beta, int eb, int k0) {
       outs[2 * t + 1] = f4[f0 + t];
     }
     rows_r2c<T, T>(L, src, sp, nb, k0, nlev, (T)1);
-    cols_jobs<T>(L, COP_FILT2, nb, sp, nullptr, o2, o4, nullptr, 2, 1, 1, k0, nlev, g2, g4);
+    cols_jobs<T, COP_FILT2, 2, true, true>(L, nb, sp, nullptr, o2, o4, nullptr, k0, nlev, g2, g4);
     rows_c2r<T, T>(L, cs18, outs, 2 * nb, k0, nlev);
   }
   FeatArgs fa;

@@ -355,21 +355,21 @@ static void press_stag_array(Les& L, double tadv1, bool ab2 = false, double tadv
     const double* ab[6] = {D(L, LES_RHSX), D(L, LES_RHSY), D(L, LES_RHSZ),
                            D(L, LES_RHSX_F), D(L, LES_RHSY_F), D(L, LES_RHSZ_F)};
     const double abc[3] = {L.P.dt, tadv1, tadv2};
-    rows_r2c<double, double>(L, src, dst, 3, 1, nz, c / tadv1, LOAD_AB2_SCALE_DIV, L.P.dt, 0, ab, abc);
+    rows_r2c<double, double, LOAD_AB2_SCALE_DIV>(L, src, dst, 3, 1, nz, c / tadv1, L.P.dt, ab, abc);
   } else {
-    rows_r2c<double, double>(L, src, dst, 3, 1, nz, c / tadv1, LOAD_SCALE_DIV, L.P.dt);
+    rows_r2c<double, double, LOAD_SCALE_DIV>(L, src, dst, 3, 1, nz, c / tadv1, L.P.dt);
   }
   // forward y transforms; the horizontal divergence i kx Hx + i ky Hy is
   // formed by the column pass (into Hx), so the solve reads two spectra
-  cols<double>(L, COP_DIV, Hx, Hy, Hx, nullptr, nullptr, 1, 1, 0, 1, nz);
-  cols<double>(L, COP_COPY, Hz, nullptr, Hz, nullptr, nullptr, 1, 1, 0, 1, nz);
+  cols<double, COP_DIV, 1, true, false>(L, Hx, Hy, Hx, nullptr, nullptr, 1, nz);
+  cols<double, COP_COPY, 1, true, false>(L, Hz, nullptr, Hz, nullptr, nullptr, 1, nz);
   // bottom and top layers (src/compute_pressure.f90:152-165, 196-203)
   Cplx<double>* lb = (Cplx<double>*)L.playr[0];
   Cplx<double>* lt = (Cplx<double>*)L.playr[1];
   const double* lsrc[2] = {L.layer[LES_BOTTOM_WK], L.layer[LES_TOP_WK]};
   Cplx<double>* ldst[2] = {lb, lt};
   rows_r2c<double, double>(L, lsrc, ldst, 2, 0, 1, c);
-  cols_jobs<double>(L, COP_COPY, 2, ldst, nullptr, ldst, nullptr, nullptr, 1, 1, 0, 0, 1);
+  cols_jobs<double, COP_COPY, 1, true, false>(L, 2, ldst, nullptr, ldst, nullptr, nullptr, 0, 1);
   // tridiagonal solve per mode
   TriArgs t;
   t.Hd = Hx; t.Hz = Hz; t.bot = lb; t.top = lt;
@@ -388,7 +388,7 @@ static void press_stag_array(Les& L, double tadv1, bool ab2 = false, double tadv
   }
   kt_end(L, KT_TRIDIAG, 16.0 * L.ns * (2.0 * nz + 2.0 + (nz + 2.0)), "k_tridiag");
   // gradient: i kx p, i ky p and p back to physical space (src/compute_pressure.f90:320-357)
-  cols<double>(L, COP_PGRAD, ph, nullptr, Hx, Hy, Hz, 3, 0, 1, 0, nz + 2);
+  cols<double, COP_PGRAD, 3, false, true>(L, ph, nullptr, Hx, Hy, Hz, 0, nz + 2);
   if (fused) return;  // les_step: the projection is the inverse x transform's store (press_project)
   const Cplx<double>* cs[3] = {Hx, Hy, Hz};
   double* outs[3] = {D(L, LES_DPDX), D(L, LES_DPDY), D(L, LES_P)};
@@ -536,7 +536,7 @@ static void refresh_gradp(Les& L) {
   Cplx<double>* Hx = (Cplx<double>*)L.pspec[0];
   Cplx<double>* Hy = (Cplx<double>*)L.pspec[1];
   Cplx<double>* Hz = (Cplx<double>*)L.pspec[2];
-  cols<double>(L, COP_PGRAD, (Cplx<double>*)L.pspec[3], nullptr, Hx, Hy, Hz, 3, 0, 1, 0, nz + 2);
+  cols<double, COP_PGRAD, 3, false, true>(L, (Cplx<double>*)L.pspec[3], nullptr, Hx, Hy, Hz, 0, nz + 2);
   const Cplx<double>* cs[2] = {Hx, Hy};
   double* outs[2] = {D(L, LES_DPDX), D(L, LES_DPDY)};
   rows_c2r<double, double>(L, cs, outs, 2, 0, nz + 2);

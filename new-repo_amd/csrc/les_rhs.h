@@ -100,7 +100,7 @@ static void spectral_multiply(Les& L, T* const* src, TO* const* dst, int nf, int
     rows_r2c<T, T>(L, s, sp, m, 1, nlev, (T)1);
     Cplx<T>* fo[3];
     for (int t = 0; t < m; ++t) fo[t] = (Cplx<T>*)L.wk_spec[3 + t];
-    cols_jobs<T>(L, COP_FILT1, m, sp, nullptr, fo, nullptr, nullptr, 1, 1, 1, 1, nlev, g);
+    cols_jobs<T, COP_FILT1, 1, true, true>(L, m, sp, nullptr, fo, nullptr, nullptr, 1, nlev, g);
     rows_c2r<T, TO>(L, cs, o, m, 1, nlev);
   }
 }
@@ -276,7 +276,7 @@ static void div_stress(Les& L, int rhs_id, int tx, int ty, int tz, int stag, int
   Cplx<T>* dst[2] = {s0, s1};
   const T c = (T)(1.0 / (double)(L.nx * L.ny));
   rows_r2c<T, T>(L, src, dst, 2, 1, L.nz + 1, c);
-  cols<T>(L, COP_DIV, s0, s1, s2, nullptr, nullptr, 1, 1, 1, 1, L.nz + 1);
+  cols<T, COP_DIV, 1, true, true>(L, s0, s1, s2, nullptr, nullptr, 1, L.nz + 1);
   DivEpi3<T> ep;
   ep.c[0] = div_epi_args<T>(L, rhs_id, tz, stag, save_wk, forcing);
   const Cplx<T>* cs[1] = {s2};
@@ -300,7 +300,7 @@ static void div_stress_spectra(Les& L) {
   const Cplx<T>* a0[3] = {sp[0], sp[1], sp[3]};
   const Cplx<T>* a1[3] = {sp[1], sp[2], sp[4]};
   Cplx<T>* d[3] = {sp[5], sp[6], sp[7]};
-  cols_jobs<T>(L, COP_DIV, 3, a0, a1, d, nullptr, nullptr, 1, 1, 1, 1, L.nz + 1);
+  cols_jobs<T, COP_DIV, 1, true, true>(L, 3, a0, a1, d, nullptr, nullptr, 1, L.nz + 1);
 }
 
 // Second half: inverse transforms with the rhs update as their store.
