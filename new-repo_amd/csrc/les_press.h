@@ -378,15 +378,16 @@ static void press_stag_array(Les& L, double tadv1, bool ab2 = false, double tadv
   t.gam = L.tri_gam;
   t.lhx = L.lhx; t.ny = L.ny; t.nz = nz; t.ns = L.ns;
   t.dz = L.dz; t.idz2 = 1.0 / (L.dz * L.dz);
+  const bool lds = tri_in_lds(L.lhx, L.ny, nz);
   kt_begin(L, KT_TRIDIAG);
-  if (tri_in_lds(L.lhx, L.ny, nz)) {
+  if (lds) {
     const long blocks = (L.lhx + L.ny - 1 + 255) / 256 + tri_lds_blocks(L.lhx, L.ny);
     hipLaunchKernelGGL(k_tridiag_lds, dim3((unsigned)blocks), dim3(256), tri_lds(nz), L.stream, t);
   } else {
     const long blocks = tri_zero_blocks(L.lhx, L.ny) + (2 * tri_nwork(L.lhx, L.ny) + 63) / 64;
     hipLaunchKernelGGL(k_tridiag, dim3((unsigned)blocks), dim3(64), 0, L.stream, t);
   }
-  kt_end(L, KT_TRIDIAG, 16.0 * L.ns * (2.0 * nz + 2.0 + (nz + 2.0)), "k_tridiag");
+  kt_end(L, KT_TRIDIAG, 16.0 * L.ns * (2.0 * nz + 2.0 + (nz + 2.0)), lds ? "k_tridiag_lds" : "k_tridiag");
   // gradient: i kx p, i ky p and p back to physical space (src/compute_pressure.f90:320-357)
   cols<double, COP_PGRAD, 3, false, true>(L, ph, nullptr, Hx, Hy, Hz, 0, nz + 2);
   if (fused) return;  // les_step: the projection is the inverse x transform's store (press_project)
