@@ -961,7 +961,7 @@ static bool setup_fft_attrs(const Les& L) {
          rows_trunc_reg<T>(true, L.nx, RowResArgs<T, T, double>(), 0, nullptr, nullptr, 0);
 }
 static int setup_kernel_attrs(const Les& L) {
-  if (tri_in_lds(L.lhx, L.ny, L.nz))
+  if (tri_in_lds(L.lhx, L.ny, L.nz, L.ncu))
     hipFuncSetAttribute((const void*)k_tridiag_lds, hipFuncAttributeMaxDynamicSharedMemorySize, (int)tri_lds(L.nz));
   const bool ok = setup_fft_attrs<double>(L) && setup_fft_attrs<float>(L) &&
                   rows_r2c_reg<float, float, LOAD_SCALE>(true, L.nx, RowR2CArgs<float, float>(), 0, nullptr, 0) &&
@@ -1066,13 +1066,7 @@ int les_init(const les_params* p) {
   hipEventCreateWithFlags(&L->ev_join, hipEventDisableTiming);
   hipEventCreateWithFlags(&L->ev_feat0, hipEventDisableTiming);
   hipEventCreateWithFlags(&L->ev_feat1, hipEventDisableTiming);
-  {
-    int dev = 0;
-    L->ncu = 0;
-    if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&L->ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-        L->ncu < 1)
-      L->ncu = 256;
-  }
+  if (hipDeviceGetAttribute(&L->ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || L->ncu < 1) L->ncu = 256;
   for (int i = 0; i < KT_COUNT; ++i) { hipEventCreate(&L->ev_a[i]); hipEventCreate(&L->ev_b[i]); }
   for (int i = 0; i < 6; ++i) hipEventCreate(&L->ph_ev[i]);
   g_les = L;

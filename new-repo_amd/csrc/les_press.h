@@ -203,12 +203,12 @@ __host__ __device__ inline size_t tri_lds(int nz) {
 inline long tri_lds_blocks(int lhx, int ny) { return (tri_nwork(lhx, ny) + LES_TRI_M - 1) / LES_TRI_M; }
 // Taken where two blocks fit a CU (columns up to 95 levels: never slower,
 // 256x256x64 44.0 -> 39.4 us), or where the grid is one round of one block a CU
-// (up to 201 levels).  With more rounds of one block the few modes in flight
+// (up to 202 levels, whose columns are the 160 KiB of a CU).  With more rounds of one block the few modes in flight
 // cost more than the column's traffic: 256x256x128 75 us against 103,
 // 384x384x128 212 against 232.
-inline bool tri_in_lds(int lhx, int ny, int nz) {
+inline bool tri_in_lds(int lhx, int ny, int nz, int ncu) {
   const size_t cu = 160 * 1024;
-  return 2 * tri_lds(nz) <= cu || (tri_lds(nz) <= cu && tri_lds_blocks(lhx, ny) <= 256);
+  return 2 * tri_lds(nz) <= cu || (tri_lds(nz) <= cu && tri_lds_blocks(lhx, ny) <= ncu);
 }
 __global__ void __launch_bounds__(256) k_tridiag_lds(TriArgs a) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
@@ -378,7 +378,7 @@ static void press_stag_array(Les& L, double tadv1, bool ab2 = false, double tadv
   t.gam = L.tri_gam;
   t.lhx = L.lhx; t.ny = L.ny; t.nz = nz; t.ns = L.ns;
   t.dz = L.dz; t.idz2 = 1.0 / (L.dz * L.dz);
-  const bool lds = tri_in_lds(L.lhx, L.ny, nz);
+  const bool lds = tri_in_lds(L.lhx, L.ny, nz, L.ncu);
   kt_begin(L, KT_TRIDIAG);
   if (lds) {
     const long blocks = (L.lhx + L.ny - 1 + 255) / 256 + tri_lds_blocks(L.lhx, L.ny);

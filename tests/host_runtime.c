@@ -68,7 +68,8 @@ int hipMemsetAsync(void* d, int v, size_t n, void* st) { (void)d; (void)v; (void
 /* ---- devices, streams, events, errors */
 int hipGetDevice(int* d) { *d = host_device; return OK; }
 int hipSetDevice(int d) { host_device = d; return OK; }
-int hipDeviceGetAttribute(int* v, int a, int d) { (void)a; (void)d; *v = 256; return OK; }
+int host_cus = 256;        /* compute units */
+int hipDeviceGetAttribute(int* v, int a, int d) { (void)a; (void)d; *v = host_cus; return OK; }
 int hipDeviceSynchronize(void) { return OK; }
 static uintptr_t handles = 0x1000;
 int hipStreamCreateWithFlags(void** s, unsigned f) {
