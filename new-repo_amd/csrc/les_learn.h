@@ -33,7 +33,13 @@ static int mlp_alloc(Les& L) {
   MlpState* M = new MlpState();
   std::memset((void*)M, 0, sizeof(MlpState));
   const long npt = L.np * (L.nz + 1);
-  M->nb = L.filt_batch >= 7 ? 9 : 3;  // small grids: the nine filtered fields in one launch
+  // The nine filtered fields in one launch where the grids are small (all 21
+  // fields of the plain procedure in one, spectra of at most 110 MB here), else
+  // three: the chain runs beside the band's plain update and convection, and its
+  // 27 spectra at once push theirs out of the last-level cache.  A step with an
+  // update, 9 against 3: 64^3 350 and 357 us, 96^3 689 and 708, 128x128x96 (168 MB)
+  // 915 and 892, 128^3 1140 and 1107, 144x144x128 (282 MB) 1541 and 1490.
+  M->nb = L.filt_batch == 21 ? 9 : 3;
   M->redn = 2 * (long)nblk(npt) + 64;
   std::vector<DevBuf> set = {dbuf(M->w, MLP_NPAR), dbuf(M->wb, MLP_NMAT), dbuf(M->m, MLP_NPAR), dbuf(M->v, MLP_NPAR),
                              dbuf(M->g, MLP_NPAR), dbuf(M->norm, 32), dbuf(M->X, 16 * (size_t)npt), dbuf(M->red, M->redn)};
