@@ -219,10 +219,14 @@ struct NyqShape {
   static constexpr int NT = R::NT, LS = R::LS;
   static constexpr bool WAVE = R::WAVE;
   // whole bands; short lines in one wavefront (96x48x37: 17 -> 12 us), long ones
-  // in four (288x288x64: 53 -> 50)
+  // in four (288x288x64: 53 -> 50).  A wavefront sums its bands in turn: at most
+  // four of them, also where lines of one or two threads would fill it with 8 or
+  // 16 (grad_velocity_filt at ny 16, 8 levels: 12 points 35.0 -> 16.6 us, 24 23.7 ->
+  // 17.3, 8 20.1 -> 15.2; at ny 64, 512 levels 12 points 40.3 -> 24.3).
   static constexpr int TH = N < 256 ? 64 : 256;
-  static constexpr int LB = WAVE ? R::LB : TH / NT >= 4 ? TH / NT / 4 * 4 : 4;
+  static constexpr int LB = !WAVE ? (TH / NT >= 4 ? TH / NT / 4 * 4 : 4) : R::THREADS == 64 && R::LB > 16 ? 16 : R::LB;
   static constexpr int THREADS = (LB * NT + 63) / 64 * 64, LINES = (THREADS + NT - 1) / NT;  // whole wavefronts
+  static constexpr int NW = THREADS / 64, BW = (LB / 4 + NW - 1) / NW;  // wavefronts, bands of one
   static constexpr size_t LDS = (size_t)LINES * LS * sizeof(Cplx<T>);
   static constexpr int VX = R::VX;
   static_assert(LB % 4 == 0 && (!WAVE || 64 / NT % 4 == 0), "wavefronts hold whole bands");
@@ -232,9 +236,8 @@ template <typename T, int N>
 __global__ void __launch_bounds__((NyqShape<T, N>::THREADS)) k_rows_r2c_nyq(RowR2CArgs<double, T> a, const Cplx<T>* __restrict__ tw) {
   using S = NyqShape<T, N>;
   using L = typename S::R::L1;
-  constexpr int J = (N + 63) / 64, NW = S::THREADS / 64;
   // bands of a wavefront: its own lines', else every NW-th
-  constexpr int BW = S::WAVE ? 64 / S::NT / 4 : (S::LB / 4 + NW - 1) / NW;
+  constexpr int J = (N + 63) / 64, NW = S::NW, BW = S::BW;
   extern __shared__ __align__(16) unsigned char smem_raw[];
   const long njobs = (long)a.nplanes * (a.ny / 2);
   RowAt<S> at(njobs);

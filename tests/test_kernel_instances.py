@@ -75,3 +75,21 @@ print(json.dumps(res))
         assert seen.setdefault((prec, prec and ny % 8 == 0), kernels) == kernels, (nx, ny, prec)
         assert lds <= 160 * 1024 and block <= 1024
     assert len(seen) == 3 and all(len(k) > 50 for k in seen.values())
+
+
+def test_short_lines_spread_their_nyquist_sums():
+    """A wavefront of the forward rows with Nyquist sums adds its bands of 8 rows
+    one after the other: at most 4 of them below 128 points, where one wavefront
+    could hold the lines of 16."""
+    out = host_run(f"""
+res = []
+for n in {[n for n in LENGTHS if n < 128]}:
+    with pkg.LesGpu(P.LesParams(nx=n, ny=64, nz=30, precision=1)) as g:
+        rt.clear()
+        g.grad_velocity_filt("u", "dudx", "dudy")
+        l, = [l for l in rt.launches() if "r2c_nyq" in l["name"]]
+        res.append([n, 32 * 8, l["grid"][0] * l["block"] // 64])
+print(json.dumps(res))
+""")
+    for n, bands, wavefronts in out:
+        assert bands <= 4 * wavefronts, n
