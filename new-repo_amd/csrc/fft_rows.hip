@@ -27,8 +27,8 @@ static void r2c_n(bool attr, int mode, const RowR2CArgs<TI, T>& a, int nf, const
   using SH = RowShape<T, N>;
   if constexpr (sizeof(T) == 8) {
     if (attr || mode == LOAD_SCALE_DIV) LES_ROW_LAUNCH(SH, (k_rows_r2c_reg<TI, T, N, LOAD_SCALE_DIV, false>), tw);
-    if (attr || mode == LOAD_AB2_SCALE_DIV) LES_ROW_LAUNCH(SH, (k_rows_r2c_reg<TI, T, N, LOAD_AB2_SCALE_DIV, true>), tw);
-    if (attr || mode == LOAD_PCLEAN) LES_ROW_LAUNCH(SH, (k_rows_r2c_reg<TI, T, N, LOAD_PCLEAN, true>), tw);
+    if (attr || mode == LOAD_AB2_SCALE_DIV) LES_ROW_LAUNCH(SH, (k_rows_r2c_reg<TI, T, N, LOAD_AB2_SCALE_DIV, r2c_stream(N)>), tw);
+    if (attr || mode == LOAD_PCLEAN) LES_ROW_LAUNCH(SH, (k_rows_r2c_reg<TI, T, N, LOAD_PCLEAN, r2c_stream(N)>), tw);
   }
   if (attr || mode == LOAD_SCALE) LES_ROW_LAUNCH(SH, (k_rows_r2c_reg<TI, T, N, LOAD_SCALE, false>), tw);
 }

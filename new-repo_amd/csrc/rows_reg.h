@@ -125,10 +125,19 @@ __device__ __forceinline__ void row_unpack(const Cplx<T>* line, Cplx<T>* __restr
 }
 
 // ------------------------------------------------------------------ r2c
-// STREAM: the input is read in RowStream order into LDS (the AB2 predictor and
-// the cleaned pressure, which read three and four FP64 fields per value: 192
-// points 56 -> 35 us, 512 1487 -> 1204 us); else by each thread into its
-// registers (one field: 64 points 10 -> 6 us, 192 19 -> 16).
+// STREAM: the input is read in RowStream order into LDS, else by each thread
+// into its registers (one field: 64 points 10 -> 6 us, 192 19 -> 16).  The AB2
+// predictor and the cleaned pressure, which read three and four FP64 fields per
+// value, are streamed from 108 points on.  Registers against streamed, AB2: 48^3
+// 8.2 us against 11.7, 64^3 14.2 and 14.6, 96x48x37 11.9 and 15.7, then 108x108x64
+// 23.6 and 19.5, 128x64x64 23.8 and 16.0, 192x144x65 57.3 and 36.5, 512x512x256
+// 1487 and 1204; cleaned pressure: 48^3 10.2 and 13.1, 64^3 11.7 and 15.1, 96x48x37
+// 14.7 and 17.8, 192x144x65 23.0 and 19.7.
+// At 256 and 512 points lines of one wavefront each, transformed in LDS stage by
+// stage, read both faster (AB2 256^3 272 us against 317, 512x512x32 175 and 195;
+// cleaned pressure 256^3 123 and 136): a block's 70 KB leave two wavefronts per
+// SIMD, each with four rounds of loads waited for one after the other.
+constexpr bool r2c_stream(int n) { return n >= 108; }
 template <typename TI, typename T, int N, int MODE, bool STREAM>
 __global__ void __launch_bounds__((RowShape<T, N>::THREADS)) k_rows_r2c_reg(RowR2CArgs<TI, T> a, const Cplx<T>* __restrict__ tw) {
   using S = RowShape<T, N>;

@@ -62,3 +62,13 @@ def test_fp32_two_result_filter_of_every_length(n, axis):
     for f, ref in out[0].items():
         assert np.isfinite(ref).all() and np.abs(ref).max() > 0, f
         assert rel_l2(out[1][f], ref) <= 1e-3, (f, rel_l2(out[1][f], ref))
+
+
+@pytest.mark.parametrize("n", LENGTHS)
+def test_tke_record_of_every_length(n):
+    """The cleaned pressure's forward rows at every length, in either load order:
+    the sums against the oracle's, to the bar of the step at all lengths
+    (relative to the sums of |value|, as the sums run in another order)."""
+    from test_gpu_tke import _compare, _run
+    dev, orc, ab = _run((n, 16, 6), load_params().PREC_FP64, steps=2, seed=n)
+    _compare(dev, orc, ab, 1e-11)

@@ -93,3 +93,24 @@ print(json.dumps(res))
 """)
     for n, bands, wavefronts in out:
         assert bands <= 4 * wavefronts, n
+
+
+def test_many_field_rows_are_streamed_from_108_points():
+    """AB2 predictor (load mode 2) and cleaned pressure (3): which of the two
+    load orders a length takes."""
+    out = host_run(f"""
+res = []
+for n in {LENGTHS}:
+    with pkg.LesGpu(P.LesParams(nx=n, ny=16, nz=5)) as g:
+        g.tke_init()
+        rt.clear()
+        g.step(1)
+        g.tke_accumulate()
+        res.append([n] + [l["name"] for l in rt.launches() if "r2c_reg" in l["name"]])
+print(json.dumps(res))
+""")
+    for n, *names in out:
+        streamed = "1" if n >= 108 else "0"
+        for mode in "23":
+            assert [s for s in names if f"ELi{mode}ELb{streamed}E" in s] and \
+                not [s for s in names if f"ELi{mode}ELb{'10'[int(streamed)]}E" in s], (n, mode)
