@@ -1206,8 +1206,15 @@ int les_init(const les_params* p) {
   L->filt_batch = 3;
   for (int nb : {7, 21})
     if (3.0 * nb * 2 * tb * L->nsp <= 256.0 * (1 << 20)) L->filt_batch = nb;
-  const int nspec = 3 * L->filt_batch > LES_NSPEC ? 3 * L->filt_batch : LES_NSPEC;
-  for (int i = 0; i < nspec; ++i) L->wk_spec[i] = dalloc(*L, 2 * tb * L->nsp);
+  const bool dynamic = P.sgs_model == 1 || P.sgs_model == 2;
+  for (int i = 0; i < LES_NSPEC; ++i) L->wk_spec[i] = dalloc(*L, 2 * tb * L->nsp);
+  // the batches' further slots as one buffer: giving a buffer back takes about 0.25 ms
+  const int more = dynamic && 3 * L->filt_batch > LES_NSPEC ? 3 * L->filt_batch - LES_NSPEC : 0;
+  if (more > 0) {
+    const size_t slot = (2 * tb * L->nsp + 255) / 256 * 256;
+    char* block = (char*)dalloc(*L, more * slot);
+    for (int i = 0; block && i < more; ++i) L->wk_spec[LES_NSPEC + i] = block + i * slot;
+  }
   for (int i = 0; i < 64; ++i) L->wk_real[i] = dalloc(*L, tb * L->nf);
   for (int i = 0; i < 6; ++i) L->wk_hyb[i] = dalloc(*L, tb * (size_t)L->nx2 * L->ny * L->nzg);
   for (int i = 0; i < 6; ++i) L->wk_big[i] = dalloc(*L, tb * (size_t)L->nbp * L->nzg);

@@ -44,12 +44,16 @@ static int mlp_alloc(Les& L) {
   std::vector<DevBuf> set = {dbuf(M->w, MLP_NPAR), dbuf(M->wb, MLP_NMAT), dbuf(M->m, MLP_NPAR), dbuf(M->v, MLP_NPAR),
                              dbuf(M->g, MLP_NPAR), dbuf(M->norm, 32), dbuf(M->X, 16 * (size_t)npt), dbuf(M->red, M->redn)};
   for (float*& f : M->fr) set.push_back(dbuf(f, L.nf));
-  for (int i = 0; i < 3 * M->nb; ++i) set.push_back(DevBuf{&M->fs[i], 2 * 4 * (size_t)L.nsp});
+  // 9 spectra, on small grids 18 more in one buffer (giving one back takes about 0.25 ms)
+  const size_t slot = (2 * 4 * (size_t)L.nsp + 255) / 256 * 256;
+  for (int i = 0; i < 9; ++i) set.push_back(DevBuf{&M->fs[i], slot});
+  if (M->nb > 3) set.push_back(DevBuf{&M->fs[9], 18 * slot});
   if (!dalloc_all(L, set)) {
     delete M;
     les_set_error("out of memory (MLP)");
     return 3;
   }
+  for (int i = 10; M->nb > 3 && i < 27; ++i) M->fs[i] = (char*)M->fs[i - 1] + slot;
   L.mlp = M;
   return 0;
 }
