@@ -11,8 +11,11 @@
 // Bound by memory (FP64, and FP32 from 256 points: 4-5 TB/s).  Measured
 // (MI355X) per launch: FP64 192x144x65 r2c 27 -> 16 us, c2r 33 -> 21, padding
 // and truncation 91 -> 69 and 29, divergence store 61 -> 41; FP32 256^3 c2r of
-// two fields 95 -> 80, padding 392 -> 309, divergence store 300 -> 224; the
-// FP64 stores with the projection are where they were.
+// two fields 95 -> 80, padding 392 -> 309, divergence store 300 -> 224.  The FP64
+// stores with the projection are faster below 64 points and at 648 (48x64x512 68 ->
+// 45 us, 648x64x48 66 -> 51), within 10% either way from 128 to 512, and slower at
+// 64, 96 and 256 on some grids: 64x64x488 66 -> 84, 96x64x325 63 -> 87, 256^3 402 ->
+// 420, 256x64x122 41 -> 55.
 //
 // Where NT divides a wavefront the threads of a line are in one wavefront and
 // no block barrier is needed.  Consecutive row pairs are consecutive in memory,
