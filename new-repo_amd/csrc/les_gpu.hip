@@ -1471,6 +1471,8 @@ int les_grad_velocity_filt(int f, int dfdx, int dfdy) {
   LES_ENTER(L);
   if (!L) return 1;
   if (f < LES_U || f > LES_W) { les_set_error("grad_velocity_filt: f must be u, v or w"); return 10; }
+  for (int id : {dfdx, dfdy})
+    if (id < 0 || id >= LES_NFIELDS) { les_set_error("bad field id %d", id); return 10; }
   if (L->mixed) grad_filt<float>(*L, f, dfdx, dfdy); else grad_filt<double>(*L, f, dfdx, dfdy);
   LES_CHECK(hipGetLastError());
   return 0;
@@ -1608,7 +1610,7 @@ int les_compute_dealias_convec(int cx, int cy, int cz) {
 int les_div_stress(int rhs, int tx, int ty, int tz, int stag, int save_wk) {
   LES_ENTER(L);
   if (!L) return 1;
-  if (L->fbytes[rhs] != 8) { les_set_error("div_stress: rhs must be an FP64 field"); return 10; }
+  if (rhs < 0 || rhs >= LES_NFIELDS || L->fbytes[rhs] != 8) { les_set_error("div_stress: rhs must be an FP64 field"); return 10; }
   for (int id : {tx, ty, tz})
     if (id < 0 || id >= LES_NFIELDS || field_is_fp64(id)) { les_set_error("div_stress: stress fields expected"); return 10; }
   if (L->mixed) div_stress<float>(*L, rhs, tx, ty, tz, stag, save_wk, 0);
